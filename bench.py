@@ -395,7 +395,7 @@ def neighbours_report(torch, dev, nx, ins, n, reps=5):
     del out, wout
 
     # Rasterisation (trilinear scatter) of 4096 of the insertion workload's slices into a 256^3 volume + weights,
-    # forward rotations (h2h, cutoff 0.5): the tiled kernel (per-wave LDS slabs, one device-atomic flush per work
+    # forward rotations (h2h, cutoff 0.5): the boxed kernel (sums of a box in LDS, one device-atomic flush per work
     # item), and once the one-lane-per-pixel kernel with device-wide float atomics for comparison.
     b_r = min(4096, b)
     rvol = torch.zeros((1, n, n, n // 2 + 1), dtype=torch.complex64, device=dev)
@@ -417,7 +417,7 @@ def neighbours_report(torch, dev, nx, ins, n, reps=5):
     rep["rasterize"] = {
         "workload": f"rasterize_central_slices_3d of {b_r} slices 256^2 into a 256^3 c32 volume + f32 weights (h2h, "
                     "cutoff 0.5)", "avg_ms": t * 1e3, "slices_per_s": b_r / t, "pixels_per_s": px / t,
-        "kernel": "tiled (LDS slabs per wave)", "direct_kernel_ms": t_direct * 1e3}
+        "kernel": "boxed (LDS sums per wave)", "direct_kernel_ms": t_direct * 1e3}
     log(f"rasterize {b_r} slices: {t * 1e3:.3f} ms (direct kernel {t_direct * 1e3:.1f} ms)")
     del rvol, rw, fwd
 

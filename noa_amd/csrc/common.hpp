@@ -102,6 +102,18 @@ __device__ __forceinline__ i32 wave_inclusive_sum(i32 x) {
     return x;
 }
 
+// Inclusive running maximum of non-negative values over the 64 lanes of a wave (the same moves; a lane without a
+// source sees 0).
+__device__ __forceinline__ i32 wave_inclusive_max(i32 x) {
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
+    return x;
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // Index <-> frequency (fft/core/Frequency.hpp:80-87, :115-122).
 // ---------------------------------------------------------------------------------------------------------

@@ -10,15 +10,19 @@
 // the atomics execute. Summation order across pixels is not fixed: the result is deterministic only up to
 // float reassociation, as with noa's CUDA and OpenMP paths.
 //
-// Many slices into one cubic volume (FP32 values and weights, Mat33<f32> rotations, cutoff <= 0.5) take the tiled
-// path instead, rasterize_tile_kernel: the accumulation happens in LDS and reaches the volume once per work item.
+// One cubic size (FP32 values and weights, single-precision rotations, cutoff <= 0.5) takes rasterize_box_kernel
+// instead: the accumulation happens in LDS and reaches the volume once per work item.
 #include "common.hpp"
 #include "kernels.hpp"
-#include "tiles.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <mutex>
+#include <tuple>
+#include <vector>
 
 namespace noa_hip {
 
@@ -134,63 +138,71 @@ __global__ __launch_bounds__(256) void rasterize_kernel(const RasterParams<C, In
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Tiled rasterisation. The floor positions of the (flipped) pixel coordinates are cut into tiles of 16^3 (as for the
-// tiled extraction, tiles.hpp). A work item is (tile, range of slices), one workgroup of four waves; wave w owns the
-// slab of floor positions z in [Z0 + 4w, Z0 + 4w + 4) of the tile:
-//   - LDS holds each wave's own accumulators over its slab and the layer above it (the trilinear taps reach
-//     floor + 1), 5 x 17 x 17 positions of value and weight, zeroed at the start. No other wave touches them.
-//   - The wave visits every slice of the item whose plane crosses its slab and enumerates the slab's candidate
-//     pixels (tile_candidates). A candidate runs noa's expressions of rasterize_kernel and is kept only where its
-//     floor lies in the slab, so every pixel inside the cutoff is rasterised by exactly one wave of one item.
-//   - The eight taps are added with plain LDS read-modify-write, tap by tap in program order (LDS executes one
-//     wave's instructions in order; compiler barriers keep the order). Lanes whose candidates share a floor
-//     position would update the same words in one instruction: each lane writes its id into a tag byte of its
-//     floor position and reads it back, the lane that reads its own id does the read-modify-write and the others
-//     add with the LDS float atomic (ds_add_f32) after it. Two pixels share a floor position only when they are
-//     neighbours in the slice, so these lanes are few; the float atomic costs about two clocks per lane.
-//   - The x = 0 duplicates (conjugate at (-w, -v, 0)) go straight to the volume with device-wide atomics, as in
-//     rasterize_kernel: they land anywhere in the x = 0 plane and are a thin set.
-//   - After the item's slices, each wave adds its 5 x 17 x 17 sums to the volume with device-wide atomics at noa's
-//     indices: frequency2index of the position, dropped outside [0, D) x [0, H) x [0, W/2+1) (the bounds checks
+// Boxed rasterisation. The floor positions of the (flipped) pixel coordinates are cut into boxes of 8 x 8 x 16. A work
+// item is (box, a number of consecutive slices that cross it), one wave, which runs without barriers:
+//   - LDS holds the box's own accumulators, 9 x 9 x 17 positions of value and weight (the trilinear taps reach
+//     floor + 1), zeroed at the start.
+//   - 64 slices at a time, lane l sets up slice c0 + l: its plane's normal (the crossing test), the row equation of
+//     its pixels in the box and the reciprocals of its row direction. A crossing slice's geometry is broadcast from
+//     that lane; nothing is divided or loaded per (box, slice) pair.
+//   - Lanes 0-31 take pixel rows of the direct set and lanes 32-63 rows of the mirrored one (the x < 0 flip), each
+//     the range of its row inside the box (widened by a margin far above the rounding). Every row marks its first
+//     candidate in LDS; a running maximum over the wave then gives each of 64 consecutive candidates its row.
+//   - A candidate runs noa's expressions of rasterize_kernel, up to its cutoff test and its floor position; the ones
+//     inside the box go into a queue in LDS, so that the pixels of several slices share a wave: a slice alone fills
+//     half of its lanes (60 pixels of an average crossing, in one or two groups of 64).
+//   - When the queue holds 64 pixels, their values and weights are loaded, and the 64 pixels loaded before them are
+//     accumulated: eight taps by plain LDS read-modify-write, tap by tap in program order (LDS executes one wave's
+//     instructions in order; compiler barriers keep the order). Lanes with the same floor position would update the
+//     same words in one instruction: each lane writes its id into a tag byte of its position and reads it back; the
+//     lane that reads its own id accumulates, the others (12 % of the pixels of a rotation share their position with
+//     an earlier one) return to the queue. A batch with many of them (a collapsed transform puts a whole slice into
+//     one position) adds them with the LDS float atomic instead, which costs about two clocks per lane and tap.
+//   - After the item's slices, the 9 x 9 x 17 sums are added to the volume with device-wide atomics at noa's indices:
+//     frequency2index of the position, dropped outside [0, D) x [0, H) x [0, W/2+1) (the bounds checks
 //     rasterize_kernel applies per tap, so the wrapped taps of the non-centred layout land where they land there).
-//     Neighbouring slabs and tiles overlap by one layer; both add theirs.
+//     Neighbouring boxes overlap by one layer; both add theirs. The x = 0 duplicates (the conjugate at (-w, -v, 0)
+//     with the same fraction, :347-372) are the conjugates of the sums at x = 0, which only the pixels with a floor
+//     of 0 reach: they are added once per item at the mirrored position.
 // Summation order is not fixed (the device atomics), as with rasterize_kernel.
+// Bound by the issue of its instructions at 8 waves per CU (20 KB of LDS each): 1.06e8 pixels in 2.35 ms at 4,096 slices
+// of 256^2. Four 16 x 16 x 4 slabs of a tile per workgroup, one slice at a time (no queue) and the LDS float atomic for
+// every pixel that shares its position, took 5.5 ms, of which the atomics were more than half.
 // ---------------------------------------------------------------------------------------------------------
-constexpr i32 RS_Z = 4;                             // floor layers per wave
-constexpr i32 RS_L = RS_Z + 1;                      // LDS layers per wave
-constexpr i32 RS_CELLS = RS_L * XTT * XTT;          // accumulator positions per wave
-constexpr i32 RS_TAGS = RS_Z * XT * XT;             // floor positions per wave
-constexpr i32 RS_LIST = 384;                        // candidate pixels per wave and round
-static_assert(RS_Z * XT_WAVES == XT, "the waves' slabs cover the tile");
+constexpr i32 RB_Z = 8, RB_Y = 8, RB_X = 16;                  // floor positions of a box
+constexpr i32 RL_Y = RB_Y + 1, RL_X = RB_X + 1;               // LDS extents
+constexpr i32 RB_CELLS = (RB_Z + 1) * RL_Y * RL_X;            // accumulator positions
+constexpr i32 RB_TAGS = RB_Z * RB_Y * RB_X;
+constexpr i32 RB_QUEUE = 128;                                 // at most 63 waiting + 64 new pixels
+constexpr i32 RB_MAX_N = 766;                                 // rows and columns of a slice fit 10 bits of a queue word
+constexpr i32 RB_MAX_SHARED = 24;                             // more same-position lanes than this: LDS atomics
+static_assert(RB_Z == 8 && RB_Y == 8 && RB_X == 16, "a floor position takes 10 bits of a queue word");
 
 template<class In, class Out>
-struct RasterTileParams {
+struct RasterBoxParams {
     const In* in; i64 is_b; i32 is_y, is_x; bool in_is_value; In in_value;
     const float* win; i64 wis_b; i32 wis_y, wis_x; bool win_present, win_is_value; float win_value;
     Out* vol; i32 vs0, vs1, vs2;
     float* wvol; i32 wvs0, wvs1, wvs2; bool has_wvol;
     XformArg<float> rot, scale;         // scale: Mat22 inverse scaling, or none
-    const int4* items;                  // {tile, first slice, end slice, 0}
-    i32 n, nty, ntx, base, n_slices, pixels;
-    float inv_wr, cutoff_sqd, margin;
+    const i32* boxes;                   // active boxes, the ones nearest to the origin first
+    i32* starts;                        // first slice of each item (RB_DONE: none), or null: each wave scans for it
+    i32 n, nby, nbx, base, n_slices, pixels;
+    i32 n_boxes, per_item, max_items;   // crossing slices per item, items per box
+    float inv_wr, inv_n, cutoff_sqd, margin;
     bool vol_centered, slice_centered, scaled;
 };
 
 __device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
 
-// The plane geometry of the tiled path (crossing test, candidate enumeration) takes the rotation as a matrix; the
-// per-pixel expressions keep the rotation as given (noa's quaternion rotation for quaternions).
-__device__ __forceinline__ Rot<float> as_matrix(const Rot<float>& r) {
+// The plane geometry (crossing test, candidate rows) takes the rotation as a matrix; the per-pixel expressions keep
+// the rotation as given (noa's quaternion rotation for quaternions). With an inverse scaling S (applied to the 2D
+// frequency before the rotation), pixel (y, x) lands at y (s0 a + s2 c) + x (s1 a + s3 c), with a and c the rotation's
+// 2nd and 3rd columns: the same plane, other columns.
+__device__ __forceinline__ Rot<float> plane_matrix(const Rot<float>& r, const Scale<float>& s) {
     Rot<float> g;
     rot_matrix(r, g.m);
     g.quat = false;
-    return g;
-}
-
-// With an inverse scaling S (applied to the 2D frequency before the rotation), pixel (y, x) lands at
-// y (s0 a + s2 c) + x (s1 a + s3 c), with a and c the rotation's 2nd and 3rd columns: the same plane, other columns.
-__device__ __forceinline__ Rot<float> plane_matrix(const Rot<float>& r, const Scale<float>& s) {
-    Rot<float> g = as_matrix(r);
     if (s.identity) return g;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -208,182 +220,399 @@ __device__ __forceinline__ Scale<float> slice_scaling(const XformArg<float>& a, 
     return s;
 }
 
+struct BoxOrigin { i32 z, y, x; };
+
+__device__ __forceinline__ BoxOrigin box_origin(i32 box, i32 nby, i32 nbx, i32 base) {
+    const i32 bx = box % nbx, zy = box / nbx;
+    return {base + (zy / nby) * RB_Z, base + (zy % nby) * RB_Y, bx * RB_X};
+}
+
+// Does the plane of `r` (spanned by its 2nd and 3rd columns; any matrix) cross the box widened by M? The plane is
+// symmetric through the origin, so this also decides the mirrored box.
+__device__ __forceinline__ bool box_crossed(const Rot<float>& r, BoxOrigin o, float M) {
+    const float nz = r.m[4] * r.m[8] - r.m[7] * r.m[5];
+    const float ny = r.m[7] * r.m[2] - r.m[1] * r.m[8];
+    const float nx = r.m[1] * r.m[5] - r.m[4] * r.m[2];
+    const float cz = static_cast<float>(o.z) + 0.5f * RB_Z, cy = static_cast<float>(o.y) + 0.5f * RB_Y;
+    const float cx = static_cast<float>(o.x) + 0.5f * RB_X;
+    const float d = fabsf((nz * cz + ny * cy) + nx * cx);
+    const float az = fabsf(nz), ay = fabsf(ny), ax = fabsf(nx);
+    return d <= ((0.5f * RB_Z) * az + (0.5f * RB_Y) * ay) + (0.5f * RB_X) * ax + M * ((az + ay) + ax) + 1e-6f;
+}
+
+// The first slice of each item, for more than 64 slices (otherwise, and where nothing can be allocated, the items scan
+// for it themselves, from the first slice): one workgroup per box counts the slices that cross it, and the
+// slices whose rank among them is a multiple of per_item start an item. So an item holds per_item crossing slices
+// whatever the orientations are: a model of uniform orientations makes one long item of every box on the axis of a
+// tilt series (1,200 slices of 200^2: 4.3 ms, against 0.8 ms).
+constexpr i32 RB_DONE = -1;
+constexpr i32 RB_SCAN = 256;                                  // slices tested at a time by the items kernel
 template<class In, class Out>
-__global__ __launch_bounds__(256) void rasterize_tile_kernel(const RasterTileParams<In, Out> p) {
+__global__ __launch_bounds__(RB_SCAN) void rasterize_items_kernel(const RasterBoxParams<In, Out> p) {
+    __shared__ i32 passed[2][RB_SCAN / 64];
+    const i32 t = static_cast<i32>(threadIdx.x), wave = t >> 6;
+    const BoxOrigin o = box_origin(p.boxes[blockIdx.x], p.nby, p.nbx, p.base);
+    i32* starts = p.starts + static_cast<i64>(blockIdx.x) * p.max_items;
+    i32 seen = 0, turn = 0;
+    for (i32 c0 = 0; c0 < p.n_slices; c0 += RB_SCAN, turn ^= 1) {
+        bool cross = false;
+        if (c0 + t < p.n_slices)
+            cross = box_crossed(plane_matrix(load_rotation(p.rot, c0 + t), slice_scaling(p.scale, p.scaled, c0 + t)), o,
+                                p.margin);
+        const unsigned long long m = __ballot(cross);
+        if ((t & 63) == 0) passed[turn][wave] = static_cast<i32>(__popcll(m));
+        __syncthreads();                 // one barrier per turn: the next one writes the other half
+        i32 rank = seen + static_cast<i32>(__builtin_amdgcn_mbcnt_hi(
+            static_cast<u32>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<u32>(m), 0u)));
+#pragma unroll
+        for (i32 w = 0; w < RB_SCAN / 64; ++w) {
+            if (w < wave) rank += passed[turn][w];
+            seen += passed[turn][w];
+        }
+        if (cross && rank % p.per_item == 0) starts[rank / p.per_item] = c0 + t;
+    }
+    for (i32 j = (seen + p.per_item - 1) / p.per_item + t; j < p.max_items; j += RB_SCAN) starts[j] = RB_DONE;
+}
+
+// i / n rounded to nearest, for integers |i| <= n < 2^12 with inv_n = 1 / n rounded: one Newton step on the product
+// (the remainder is exact), checked for every such pair on the CPU.
+__device__ __forceinline__ float divide_index(float i, float n, float inv_n) {
+    const float q = i * inv_n;
+    return fmaf(fmaf(-q, n, i), inv_n, q);
+}
+
+// GEN: quaternions or inverse scalings (noa's expressions at run time); otherwise Mat33 rotations.
+template<class In, class Out, bool GEN>
+__global__ __launch_bounds__(64) void rasterize_box_kernel(const RasterBoxParams<In, Out> p) {
     using RIn = typename vt<In>::real;
     constexpr bool CX = vt<Out>::cx;
-    __shared__ Out vacc_all[XT_WAVES][RS_CELLS];
-    __shared__ float wacc_all[XT_WAVES][RS_CELLS];
-    __shared__ unsigned char tags_all[XT_WAVES][RS_TAGS];
-    __shared__ u32 list[XT_WAVES][RS_LIST];
+    __shared__ Out vacc[RB_CELLS];
+    __shared__ float wacc[RB_CELLS];
+    __shared__ unsigned char tags[RB_TAGS];
+    __shared__ u32 starts[64];
+    __shared__ u32 q_word[RB_QUEUE];    // position in the box | slice column << 10 | slice row << 20 | flipped << 31
+    __shared__ i32 q_slice[RB_QUEUE];
+    __shared__ float q_z[RB_QUEUE], q_y[RB_QUEUE], q_x[RB_QUEUE];
 
-    const int4 item = p.items[blockIdx.x];
-    const i32 first = item.y, end = min(item.z, p.n_slices);
-    const i32 tx = item.x % p.ntx, tzy = item.x / p.ntx;
-    const i32 ty = tzy % p.nty, tz = tzy / p.nty;
-    const i32 wave = static_cast<i32>(threadIdx.x) >> 6, lane = static_cast<i32>(threadIdx.x) & 63;
-    const i32 Z0 = p.base + tz * XT + wave * RS_Z, Y0 = p.base + ty * XT, X0 = tx * XT;   // this wave's slab
+    const i32 lane = static_cast<i32>(threadIdx.x);
+    // Part by part over all boxes: workgroup i runs on XCD i % 8, and most boxes have only their first parts, so an order
+    // with a box's parts next to each other would give whole XCDs nothing but parts that do not exist.
+    const i32 slot = static_cast<i32>(blockIdx.x % static_cast<u32>(p.n_boxes));
+    const i32 part = static_cast<i32>(blockIdx.x / static_cast<u32>(p.n_boxes));
+    const i32 box = p.boxes[slot];
+    const BoxOrigin at0 = box_origin(box, p.nby, p.nbx, p.base);
+    const i32 Z0 = at0.z, Y0 = at0.y, X0 = at0.x;
     const i32 n = p.n, width = n / 2 + 1;
-    Out* vacc = vacc_all[wave];
-    float* wacc = wacc_all[wave];
-    unsigned char* tags = tags_all[wave];
-    u32* wl = list[wave];
-
-    for (i32 i = lane; i < RS_CELLS; i += 64) {
+    const i32 lo = -n / 2, hi = (n - 1) / 2, hix = n / 2;
+    const float P0[3] = {static_cast<float>(Z0), static_cast<float>(Y0), static_cast<float>(X0)};
+    constexpr float EXT[3] = {RB_Z, RB_Y, RB_X};
+    const float M = p.margin;
+    // The item's first slice: its slices are the next `left` ones that cross the box.
+    i32 first = 0, left = p.per_item;
+    if (p.starts) {
+        first = p.starts[static_cast<i64>(slot) * p.max_items + part];
+        if (first < 0) return;
+    } else {
+        i32 skip = part * p.per_item;
+        unsigned long long m = 0;
+        for (; first < p.n_slices; first += 64) {
+            bool cross = false;
+            if (first + lane < p.n_slices)
+                cross = box_crossed(plane_matrix(load_rotation(p.rot, first + lane),
+                                                 slice_scaling(p.scale, GEN && p.scaled, first + lane)), at0, M);
+            m = __ballot(cross);
+            const i32 cnt = static_cast<i32>(__popcll(m));
+            if (skip < cnt) break;
+            skip -= cnt;
+        }
+        if (first >= p.n_slices) return;
+        for (; skip > 0; --skip) m &= m - 1;
+        first += __ffsll(static_cast<long long>(m)) - 1;
+    }
+    for (i32 i = lane; i < RB_CELLS; i += 64) {
         vacc[i] = vzero<Out>();
         wacc[i] = 0.f;
     }
     lds_order();
 
-    const float slice_f = static_cast<float>(n), target = static_cast<float>(n);
-    const float M = p.margin;
-    const float cz = static_cast<float>(Z0) + 0.5f * RS_Z, cy = static_cast<float>(Y0) + 0.5f * XT;
-    const float cx = static_cast<float>(X0) + 0.5f * XT;
-    for (i32 c0 = first; c0 < end; c0 += 64) {
-        const bool cross = c0 + lane < end &&
-                           slab_crossed<RS_Z>(plane_matrix(load_rotation(p.rot, c0 + lane),
-                                                           slice_scaling(p.scale, p.scaled, c0 + lane)),
-                                              cz, cy, cx, M);
+    const float nf = static_cast<float>(n);
+    // The box of this lane's set, widened by the margin: direct positions in [P0, P0 + EXT), mirrored ones in
+    // (-P0 - EXT, -P0].
+    const bool mirrored_rows = lane >= 32;
+    float blo[3], bhi[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        blo[i] = (mirrored_rows ? -(P0[i] + EXT[i]) : P0[i]) - M;
+        bhi[i] = (mirrored_rows ? -P0[i] : P0[i] + EXT[i]) + M;
+    }
+
+    // One batch of queued pixels whose loads are in flight.
+    struct Batch {
+        u32 word;
+        i32 slice;
+        float tz, ty, tx, weight;
+        In raw;
+        bool valid;
+    };
+    Batch batch{};
+    bool have = false;
+    i32 queued = 0;
+
+    // Takes the last (at most 64) pixels of the queue and issues their loads.
+    auto issue = [&](Batch& q) {
+        const i32 m = min(queued, 64);
+        queued -= m;
+        q.valid = lane < m;
+        const i32 at = queued + (q.valid ? lane : 0);
+        q.word = q_word[at];
+        q.slice = q_slice[at];
+        q.tz = q_z[at];
+        q.ty = q_y[at];
+        q.tx = q_x[at];
+        const i32 u = static_cast<i32>((q.word >> 10) & 1023u), y = static_cast<i32>((q.word >> 20) & 1023u);
+        q.raw = p.in_value;
+        q.weight = p.win_present ? p.win_value : 1.f;
+        if (q.valid) {
+            if (!p.in_is_value)
+                q.raw = p.in[static_cast<i64>(q.slice) * p.is_b + static_cast<i64>(y) * p.is_y + static_cast<i64>(u) * p.is_x];
+            if (p.has_wvol && p.win_present && !p.win_is_value)
+                q.weight = p.win[static_cast<i64>(q.slice) * p.wis_b + static_cast<i64>(y) * p.wis_y + static_cast<i64>(u) * p.wis_x];
+        }
+    };
+    auto push = [&](bool ok, u32 word, i32 slice, float fz, float fy, float fx) {
+        const unsigned long long m = __ballot(ok);
+        if (ok) {
+            const i32 at = queued + static_cast<i32>(__builtin_amdgcn_mbcnt_hi(
+                static_cast<u32>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<u32>(m), 0u)));
+            q_word[at] = word;
+            q_slice[at] = slice;
+            q_z[at] = fz;
+            q_y[at] = fy;
+            q_x[at] = fx;
+        }
+        queued += static_cast<i32>(__popcll(m));
+    };
+    // Accumulates a batch: the eight taps of the lanes that own their floor position.
+    auto finish = [&](const Batch& q) {
+        const i32 cell = static_cast<i32>(q.word & 1023u);
+        if (q.valid) tags[cell] = static_cast<unsigned char>(lane);
+        lds_order();
+        const bool own = q.valid && tags[cell] == static_cast<unsigned char>(lane);
+        const bool shared = q.valid && !own;
+        lds_order();
+        // get_input_value_ (:270-277): complex -> complex is multiplied by `conjugate`, i.e. negated when flipped.
+        Out value;
+        if constexpr (vt<In>::cx && CX) value = vcast<Out>(vmul(q.raw, (q.word >> 31) ? RIn(-1) : RIn(1)));
+        else value = vcast<Out>(q.raw);
+        const float fr[2][3] = {{1 - q.tz, 1 - q.ty, 1 - q.tx}, {q.tz, q.ty, q.tx}};
+        const i32 o = ((cell >> 7) * RL_Y + ((cell >> 4) & 7)) * RL_X + (cell & 15);
+        const bool many = __popcll(__ballot(shared)) > RB_MAX_SHARED;
+#pragma unroll
+        for (int w = 0; w < 2; ++w)
+#pragma unroll
+            for (int v = 0; v < 2; ++v)
+#pragma unroll
+                for (int uu = 0; uu < 2; ++uu) {
+                    const float kk = fr[w][0] * fr[v][1] * fr[uu][2];
+                    const i32 at = o + (w * RL_Y + v) * RL_X + uu;
+                    if (own) {
+                        const Out v0 = vacc[at];
+                        const float w0 = wacc[at];
+                        vacc[at] = vadd(v0, vmul(value, kk));
+                        wacc[at] = w0 + q.weight * kk;
+                    }
+                    lds_order();
+                }
+        if (many) {
+            if (shared) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const float kk = fr[t >> 2][0] * fr[(t >> 1) & 1][1] * fr[t & 1][2];
+                    const i32 at = o + ((t >> 2) * RL_Y + ((t >> 1) & 1)) * RL_X + (t & 1);
+                    const Out add = vmul(value, kk);
+                    if constexpr (CX) {
+                        atomicAdd(&vacc[at].x, add.x);
+                        atomicAdd(&vacc[at].y, add.y);
+                    } else {
+                        atomicAdd(vacc + at, add);
+                    }
+                    atomicAdd(wacc + at, q.weight * kk);
+                }
+            }
+            lds_order();
+        } else {
+            push(shared, q.word, q.slice, q.tz, q.ty, q.tx);
+        }
+    };
+    // Batches of 64 as long as the queue holds one; each accumulates the batch loaded before it. `all`: to the end.
+    auto drain = [&](bool all) {
+        while (queued >= 64 || (all && (queued > 0 || have))) {
+            lds_order();
+            Batch next{};
+            const bool more = queued > 0;
+            if (more) issue(next);
+            lds_order();
+            if (have) finish(batch);
+            batch = next;
+            have = more;
+        }
+    };
+
+    for (i32 c0 = first; c0 < p.n_slices && left > 0; c0 += 64) {
+        // Lane l: the plane of slice c0 + l. F = Y a + U c; on the plane Y = g . F with g the first row of
+        // (G^T G)^-1 G^T, G = [a c].
+        float a[3] = {}, c[3] = {}, g[3] = {}, ic[3] = {};
+        bool cross = false, flat = false;
+        if (c0 + lane < p.n_slices) {
+            const Rot<float> r = plane_matrix(load_rotation(p.rot, c0 + lane), slice_scaling(p.scale, GEN && p.scaled, c0 + lane));
+            cross = box_crossed(r, at0, M);
+            a[0] = r.m[1]; a[1] = r.m[4]; a[2] = r.m[7];
+            c[0] = r.m[2]; c[1] = r.m[5]; c[2] = r.m[8];
+            const float aa = (a[0] * a[0] + a[1] * a[1]) + a[2] * a[2];
+            const float ac = (a[0] * c[0] + a[1] * c[1]) + a[2] * c[2];
+            const float cc = (c[0] * c[0] + c[1] * c[1]) + c[2] * c[2];
+            const float det = aa * cc - ac * ac;
+            flat = !(det > 1e-6f * aa * cc);
+            const float idet = 1.f / det;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                g[i] = (cc * a[i] - ac * c[i]) * idet;
+                // A row direction with no component along the axis is inside or outside as a whole: the huge
+                // reciprocal turns the distances to the faces into an unbounded or an empty range.
+                ic[i] = fabsf(c[i]) > 1e-12f ? 1.f / c[i] : 1e30f;
+            }
+        }
         unsigned long long mask = __ballot(cross);
-        while (mask) {
+        const unsigned long long flat_mask = __ballot(flat);
+        while (mask && left > 0) {
             const i32 k = __ffsll(static_cast<long long>(mask)) - 1;
             mask &= mask - 1;
+            --left;
             const i32 b = c0 + k;
-            const Rot<float> r = load_rotation(p.rot, b);
-            const Scale<float> sc = slice_scaling(p.scale, p.scaled, b);
-
-            // fetch: noa's expressions up to the fractions and the input value and weight (the loads of two
-            // candidates in flight per lane); store: the eight taps into LDS, and the x = 0 duplicates.
-            struct Cand {
-                Out value;
-                float weight, tz, ty, tx;
-                i32 lz, ly, lx;
-                bool ok;
-            };
-            auto fetch = [&](i32 fy, i32 u, bool mirrored, Cand& c) {
-                c.ok = false;
+            const float A[3] = {bcast(a[0], k), bcast(a[1], k), bcast(a[2], k)};
+            const float Cc[3] = {bcast(c[0], k), bcast(c[1], k), bcast(c[2], k)};
+            Rot<float> rot{};
+            Scale<float> sc;
+            sc.identity = true;
+            if constexpr (GEN) {
+                rot = load_rotation(p.rot, b);
+                sc = slice_scaling(p.scale, p.scaled, b);
+            }
+            // One candidate per lane: noa's expressions (rasterize_kernel) up to the floor position; queued if inside.
+            auto evaluate = [&](bool live, i32 fy, i32 u, bool mirrored) {
                 vec2<float> f2;
-                f2.y = static_cast<float>(fy) / slice_f;
-                f2.x = static_cast<float>(u) / slice_f;
-                // With a scaling: rasterize_kernel's general expression, without Ewald sphere (0 curvature).
-                vec3<float> f = p.scaled ? slice2grid<true>(f2, sc, r, 0.f, 0.f) : slice2grid<false>(f2, sc, r, 0.f, 0.f);
-                if (dot3(f) > p.cutoff_sqd) return;
-                const bool flip = f.x < 0;
-                if (flip != mirrored) return;
-                RIn conjugate = 1;
-                if (flip) {
-                    f.z = -f.z; f.y = -f.y; f.x = -f.x;
-                    if constexpr (vt<In>::cx) conjugate = -1;
+                f2.y = divide_index(static_cast<float>(fy), nf, p.inv_n);
+                f2.x = divide_index(static_cast<float>(u), nf, p.inv_n);
+                vec3<float> f;
+                if constexpr (GEN) {
+                    f = p.scaled ? slice2grid<true>(f2, sc, rot, 0.f, 0.f) : slice2grid<false>(f2, sc, rot, 0.f, 0.f);
+                } else {
+                    f.z = A[0] * f2.y + Cc[0] * f2.x;        // the rotation's first column meets a zero
+                    f.y = A[1] * f2.y + Cc[1] * f2.x;
+                    f.x = A[2] * f2.y + Cc[2] * f2.x;
                 }
-                const float fz = f.z * target, fyv = f.y * target, fx = f.x * target;
+                const bool flip = f.x < 0;
+                bool ok = live && !(dot3(f) > p.cutoff_sqd) && flip == mirrored;
+                if (flip) { f.z = -f.z; f.y = -f.y; f.x = -f.x; }
+                const float fz = f.z * nf, fyv = f.y * nf, fx = f.x * nf;
                 const float flz = floorf(fz), fly = floorf(fyv), flx = floorf(fx);
                 const i32 lz = static_cast<i32>(flz) - Z0, ly = static_cast<i32>(fly) - Y0;
                 const i32 lx = static_cast<i32>(flx) - X0;
-                if (static_cast<u32>(lz) >= static_cast<u32>(RS_Z) || static_cast<u32>(ly) >= static_cast<u32>(XT) ||
-                    static_cast<u32>(lx) >= static_cast<u32>(XT))
-                    return;
+                ok = ok && static_cast<u32>(lz) < static_cast<u32>(RB_Z) && static_cast<u32>(ly) < static_cast<u32>(RB_Y) &&
+                     static_cast<u32>(lx) < static_cast<u32>(RB_X);
                 const i32 y = frequency2index(p.slice_centered, fy, n);
-                const In raw = p.in_is_value ? p.in_value : p.in[static_cast<i64>(b) * p.is_b + y * p.is_y + u * p.is_x];
-                if constexpr (vt<In>::cx && CX) c.value = vcast<Out>(vmul(raw, conjugate));
-                else c.value = vcast<Out>(raw);
-                c.weight = 0.f;
-                if (p.has_wvol) {
-                    if (!p.win_present) c.weight = 1.f;
-                    else c.weight = p.win_is_value ? p.win_value
-                                                   : p.win[static_cast<i64>(b) * p.wis_b + y * p.wis_y + u * p.wis_x];
-                }
-                c.tz = fz - flz;
-                c.ty = fyv - fly;
-                c.tx = fx - flx;
-                c.lz = lz; c.ly = ly; c.lx = lx;
-                c.ok = true;
+                const u32 word = static_cast<u32>((lz << 7) | (ly << 4) | lx) | (static_cast<u32>(u) << 10) |
+                                 (static_cast<u32>(y) << 20) | (flip ? 0x80000000u : 0u);
+                push(ok, word, b, fz - flz, fyv - fly, fx - flx);
+                drain(false);
             };
-            auto store = [&](const Cand& c) {
-                // One lane per floor position does the plain read-modify-write, the others the atomic add.
-                const i32 cell = (c.lz * XT + c.ly) * XT + c.lx;
-                if (c.ok) tags[cell] = static_cast<unsigned char>(lane);
-                lds_order();
-                const bool own = c.ok && tags[cell] == static_cast<unsigned char>(lane);
-                const bool shared = c.ok && !own;
-                lds_order();
-                float fr[2][3];
-                fr[1][0] = c.tz; fr[1][1] = c.ty; fr[1][2] = c.tx;
-                fr[0][0] = 1 - c.tz; fr[0][1] = 1 - c.ty; fr[0][2] = 1 - c.tx;
-                const i32 o = (c.lz * XTT + c.ly) * XTT + c.lx;
-#pragma unroll
-                for (int w = 0; w < 2; ++w)
-#pragma unroll
-                    for (int v = 0; v < 2; ++v)
-#pragma unroll
-                        for (int uu = 0; uu < 2; ++uu) {
-                            const float kk = fr[w][0] * fr[v][1] * fr[uu][2];
-                            const i32 at = o + (w * XTT + v) * XTT + uu;
-                            const Out add = vmul(c.value, kk);
-                            const float wadd = c.weight * kk;
-                            if (own) {
-                                // Value and weight together (the weight is 0 without a weight volume).
-                                const Out v0 = vacc[at];
-                                const float w0 = wacc[at];
-                                vacc[at] = vadd(v0, add);
-                                wacc[at] = w0 + wadd;
-                            }
-                            lds_order();
-                            if (shared) {
-                                if constexpr (CX) {
-                                    atomicAdd(&vacc[at].x, add.x);
-                                    atomicAdd(&vacc[at].y, add.y);
-                                } else {
-                                    atomicAdd(vacc + at, add);
-                                }
-                                if (p.has_wvol) atomicAdd(wacc + at, wadd);
-                            }
-                            lds_order();
-                        }
-                // The x = 0 plane is redundant: the conjugate at (-w, -v, 0) with the same fraction (:347-372).
-                if (c.ok && X0 + c.lx == 0) {
-                    Out value = c.value;
-                    if constexpr (CX) value.y = -value.y;
-                    const i32 b0z = Z0 + c.lz, b0y = Y0 + c.ly;
-#pragma unroll
-                    for (int w = 0; w < 2; ++w) {
-                        const i32 iw = frequency2index(p.vol_centered, -(b0z + w), n);
-                        if (iw < 0 || iw >= n) continue;
-#pragma unroll
-                        for (int v = 0; v < 2; ++v) {
-                            const i32 iv = frequency2index(p.vol_centered, -(b0y + v), n);
-                            if (iv < 0 || iv >= n) continue;
-                            const float kk = fr[w][0] * fr[v][1] * fr[0][2];
-                            atomic_add(p.vol + (iw * p.vs0 + iv * p.vs1), vmul(value, kk));
-                            if (p.has_wvol) atomic_add(p.wvol + (iw * p.wvs0 + iv * p.wvs1), c.weight * kk);
-                        }
-                    }
+            if ((flat_mask >> k) & 1u) {
+                // Degenerate transform (the plane collapses): every pixel of the slice is a candidate.
+                for (i32 pix0 = 0; pix0 < p.pixels; pix0 += 64) {
+                    const i32 pix = min(pix0 + lane, p.pixels - 1);
+                    const i32 yq = static_cast<i32>((static_cast<float>(pix) + 0.5f) * p.inv_wr);
+                    const i32 u = pix - yq * width;
+                    const i32 fy = index2frequency(p.slice_centered, yq, n);
+                    evaluate(pix0 + lane < p.pixels, fy, u, false);
+                    evaluate(pix0 + lane < p.pixels, fy, u, true);
                 }
-            };
-
-            tile_candidates<Cand, RS_Z, RS_LIST>(plane_matrix(r, sc), Z0, Y0, X0, n, M, p.pixels, p.inv_wr, p.slice_centered,
-                                                 lane, wl, fetch, store);
+                continue;
+            }
+            const float G[3] = {bcast(g[0], k), bcast(g[1], k), bcast(g[2], k)};
+            const float IC[3] = {bcast(ic[0], k), bcast(ic[1], k), bcast(ic[2], k)};
+            float ymin = 0.f, ymax = 0.f;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const float t1 = G[i] * blo[i], t2 = G[i] * bhi[i];
+                ymin += fminf(t1, t2);
+                ymax += fmaxf(t1, t2);
+            }
+            // The first row of each set (uniform over its 32 lanes).
+            const i32 yfirst = max(static_cast<i32>(ceilf(fmaxf(ymin, static_cast<float>(lo) - 1.f))), lo);
+            const i32 ylast = min(static_cast<i32>(floorf(fminf(ymax, static_cast<float>(hi) + 1.f))), hi);
+            const i32 y_direct = __builtin_amdgcn_readlane(yfirst, 0), y_mirror = __builtin_amdgcn_readlane(yfirst, 32);
+            for (i32 rb = 0;; rb += 32) {
+                const i32 fy = yfirst + rb + (lane & 31);
+                const bool row = fy <= ylast;
+                if (__ballot(row) == 0) break;
+                // Pixel range of the row: U with Y a + U c inside the box.
+                float ulo = 0.f, uhi = static_cast<float>(hix);
+                const float fyf = static_cast<float>(fy);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const float at = A[i] * fyf;
+                    const float t1 = (blo[i] - at) * IC[i], t2 = (bhi[i] - at) * IC[i];
+                    ulo = fmaxf(ulo, fminf(t1, t2));
+                    uhi = fminf(uhi, fmaxf(t1, t2));
+                }
+                i32 u0 = 0, cnt = 0;
+                if (row && ulo <= uhi) {
+                    u0 = static_cast<i32>(ceilf(ulo));
+                    cnt = max(0, static_cast<i32>(floorf(uhi)) - u0 + 1);
+                }
+                const i32 incl = wave_inclusive_sum(cnt), excl = incl - cnt;
+                const i32 total = __builtin_amdgcn_readlane(incl, 63);
+                const i32 from = u0 - excl;
+                for (i32 base = 0; base < total; base += 64) {
+                    // The row of candidate base + lane: every row with candidates in the window marks its first one.
+                    starts[lane] = 0u;
+                    lds_order();
+                    if (cnt > 0 && incl > base && excl < base + 64)
+                        starts[max(excl - base, 0)] = static_cast<u32>(lane);
+                    lds_order();
+                    const i32 r = wave_inclusive_max(static_cast<i32>(starts[lane]));
+                    lds_order();
+                    const i32 u = __builtin_amdgcn_ds_bpermute(r << 2, from) + base + lane;
+                    const bool live = base + lane < total;
+                    evaluate(live, (r < 32 ? y_direct : y_mirror) + rb + (r & 31), live ? u : 0, r >= 32);
+                }
+            }
         }
     }
+    drain(true);
     lds_order();
 
-    // Flush: positions [Z0, Z0 + 4] x [Y0, Y0 + 16] x [X0, X0 + 16] at noa's indices, inside the stored volume.
-    for (i32 i = lane; i < RS_CELLS; i += 64) {
-        const i32 dz = i / (XTT * XTT), rem = i - dz * (XTT * XTT);
-        const i32 dy = rem / XTT, dx = rem - dy * XTT;
+    // Flush: positions [Z0, Z0 + 8] x [Y0, Y0 + 8] x [X0, X0 + 16] at noa's indices, inside the stored volume.
+    for (i32 i = lane; i < RB_CELLS; i += 64) {
+        const i32 dz = i / (RL_Y * RL_X), rem = i - dz * (RL_Y * RL_X);
+        const i32 dy = rem / RL_X, dx = rem - dy * RL_X;
         const i32 iu = X0 + dx;
-        if (iu >= width) continue;
-        const i32 iw = frequency2index(p.vol_centered, Z0 + dz, n);
-        const i32 iv = frequency2index(p.vol_centered, Y0 + dy, n);
-        if (iw < 0 || iw >= n || iv < 0 || iv >= n) continue;
-        const Out v = vacc[i];
-        if constexpr (CX) {
-            if (v.x != 0.f || v.y != 0.f) atomic_add(p.vol + (iw * p.vs0 + iv * p.vs1 + iu * p.vs2), v);
-        } else {
-            if (v != 0.f) atomic_add(p.vol + (iw * p.vs0 + iv * p.vs1 + iu * p.vs2), v);
-        }
-        if (p.has_wvol) {
-            const float w = wacc[i];
-            if (w != 0.f) atomic_add(p.wvol + (iw * p.wvs0 + iv * p.wvs1 + iu * p.wvs2), w);
+        Out v = vacc[i];
+        const float w = wacc[i];
+        bool any = w != 0.f;
+        if constexpr (CX) any = any || v.x != 0.f || v.y != 0.f;
+        else any = any || v != 0.f;
+        if (iu >= width || !any) continue;
+        auto add = [&](i32 z, i32 y, const Out& value) {
+            const i32 iw = frequency2index(p.vol_centered, z, n), iv = frequency2index(p.vol_centered, y, n);
+            if (iw < 0 || iw >= n || iv < 0 || iv >= n) return;
+            atomic_add(p.vol + (iw * p.vs0 + iv * p.vs1 + iu * p.vs2), value);
+            if (p.has_wvol) atomic_add(p.wvol + (iw * p.wvs0 + iv * p.wvs1 + iu * p.wvs2), w);
+        };
+        add(Z0 + dz, Y0 + dy, v);
+        if (iu == 0) {
+            if constexpr (CX) v.y = -v.y;
+            add(-(Z0 + dz), -(Y0 + dy), v);
         }
     }
 }
@@ -411,36 +640,97 @@ template<class T> T value_of(const Arr& a) {
 
 constexpr int NOT_TILED = -1000;
 
-// The tiled path (rasterize_tile_kernel) where it applies: cubic volume and slices, no target shape, no Ewald
-// sphere, cutoff <= 0.5, Mat33<f32> or Quaternion<f32> rotations, Mat22 inverse scalings or none. NOA_HIP_RASTERIZE_LAYOUT=direct|tiles forces either; by default
-// the tiles take launches of at least 64 slices. NOA_HIP_RASTERIZE_PAIRS: expected crossing slices per work item.
+// The boxes that the cutoff sphere reaches, for one size and cutoff: every pixel inside the cutoff has its floor within
+// [lo - 1, hi + 1] along z and y and [0, n/2] along x. The ones nearest to the origin, which most slices cross, come
+// first. Kept per (device, size, cutoff) for the process lifetime.
+struct BoxPlan {
+    i32* boxes{};
+    i32 n_boxes{}, nby{}, nbx{}, base{};
+};
+std::mutex g_box_mutex;
+std::map<std::tuple<int, i32, double>, BoxPlan> g_box_plans;
+
+int make_box_plan(int device, i32 n, double cutoff, BoxPlan& plan, std::string& err) {
+    std::lock_guard<std::mutex> lock(g_box_mutex);
+    const auto key = std::make_tuple(device, n, cutoff);
+    const auto it = g_box_plans.find(key);
+    if (it != g_box_plans.end()) {
+        plan = it->second;
+        return NOA_HIP_OK;
+    }
+    BoxPlan pl;
+    const i32 lo = -n / 2, hi = (n - 1) / 2;
+    pl.base = lo - 1;
+    const i32 span = hi + 1 - pl.base + 1;
+    const i32 nbz = (span + RB_Z - 1) / RB_Z;
+    pl.nby = (span + RB_Y - 1) / RB_Y;
+    pl.nbx = (n / 2 + 1 + RB_X - 1) / RB_X;
+    const double reach = cutoff * n + 1.0;
+    std::vector<std::pair<double, i32>> active;
+    for (i32 b = 0; b < nbz * pl.nby * pl.nbx; ++b) {
+        const double at[3] = {double(pl.base + b / pl.nbx / pl.nby * RB_Z), double(pl.base + b / pl.nbx % pl.nby * RB_Y),
+                              double(b % pl.nbx * RB_X)};
+        const double ext[3] = {RB_Z, RB_Y, RB_X};
+        double closest = 0, centre = 0;
+        for (int a = 0; a < 3; ++a) {
+            const double d = std::max({at[a], -(at[a] + ext[a]), 0.0}), c = at[a] + 0.5 * ext[a];
+            closest += d * d;
+            centre += c * c;
+        }
+        if (closest <= reach * reach) active.push_back({centre, b});
+    }
+    std::stable_sort(active.begin(), active.end());
+    std::vector<i32> boxes(active.size());
+    for (size_t k = 0; k < active.size(); ++k) boxes[k] = active[k].second;
+    pl.n_boxes = static_cast<i32>(boxes.size());
+    if (!boxes.empty() &&
+        (hipMalloc(&pl.boxes, boxes.size() * sizeof(i32)) != hipSuccess ||
+         hipMemcpy(pl.boxes, boxes.data(), boxes.size() * sizeof(i32), hipMemcpyHostToDevice) != hipSuccess)) {
+        err = "rasterize: could not upload the boxes";
+        return NOA_HIP_ERROR_RUNTIME;
+    }
+    g_box_plans[key] = pl;
+    plan = pl;
+    return NOA_HIP_OK;
+}
+
+// The boxed path (rasterize_box_kernel) where it applies: cubic volume and slices, no target shape, no Ewald sphere,
+// cutoff <= 0.5, Mat33<f32> or Quaternion<f32> rotations, Mat22 inverse scalings or none. It takes every such call: one
+// slice of 256^2 into its volume 38 us against 57 us with a lane per pixel, 8 slices of 64^2 26 us either way, 41 of
+// 192^2 109 against 665 us, 4,096 of 256^2 2.4 against 112 ms (with the clearing of the volume, 24 us at 256^3).
+// NOA_HIP_RASTERIZE_LAYOUT=direct selects the lane-per-pixel kernel; NOA_HIP_RASTERIZE_PAIRS sets the crossing slices
+// per work item.
 template<class In, class Out, class C, class W>
 int run_tiles(const ProjectDesc& d, const RasterParams<C, In, Out, W>& p, hipStream_t stream, std::string& err) {
     const i64 nn = p.grid[0], n_slices = d.in_shape[0];
     const bool cubic = p.grid[1] == nn && p.grid[2] == nn && d.in_shape[2] == nn && d.in_shape[3] == nn &&
                        d.target[0] == nn && d.target[1] == nn && d.target[2] == nn;
     const i64 stored = nn * nn * (nn / 2 + 1);
-    // The candidate list of a wave must hold a whole slice row (n/2 + 1 pixels) for any matrix.
     const bool flat = p.ews[0] == 0 && p.ews[1] == 0;
-    const bool eligible = cubic && flat && nn >= 16 && nn / 2 + 1 <= RS_LIST && d.cutoff <= 0.5 &&
+    const bool eligible = cubic && flat && nn >= 16 && nn <= RB_MAX_N && d.cutoff <= 0.5 &&
                           (p.rot.kind == NOA_HIP_MAT33_F32 || p.rot.kind == NOA_HIP_QUAT_F32) &&
                           stored < 0x7fffffffLL && n_slices <= 0x7fffffffLL;
     if (!eligible) return NOT_TILED;
     const char* env = std::getenv("NOA_HIP_RASTERIZE_LAYOUT");
-    const bool want = env ? std::strcmp(env, "tiles") == 0 : n_slices >= 64;
-    if (!want) return NOT_TILED;
+    if (env && std::strcmp(env, "tiles") != 0) return NOT_TILED;
     int device = 0;
     (void)hipGetDevice(&device);
-    i64 step = 1;
-    while (n_slices > 16 * step) step *= 2;
-    const i32 plan_slices = static_cast<i32>((n_slices + step - 1) / step * step);
-    const char* pe = std::getenv("NOA_HIP_RASTERIZE_PAIRS");
-    const i32 pairs = pe ? std::max(8, std::atoi(pe)) : -256;   // default: at most 256, fewer for small calls
-    TilePlan plan;
-    const int st = make_tile_plan(device, static_cast<i32>(nn), std::max(d.cutoff, 0.0), plan_slices, pairs, plan, err);
+    BoxPlan plan;
+    const int st = make_box_plan(device, static_cast<i32>(nn), std::max(d.cutoff, 0.0), plan, err);
     if (st != NOA_HIP_OK) return st;
-    if (plan.n_items == 0) return NOA_HIP_OK;
-    RasterTileParams<In, Out> q{};
+    if (plan.n_boxes == 0) return NOA_HIP_OK;
+    const char* pe = std::getenv("NOA_HIP_RASTERIZE_PAIRS");
+    // Crossing slices per item. An item costs its flush (9 x 9 x 17 atomics, most of them non-zero) and its slices, one
+    // after the other; the number of items falls and the length of one grows with this number, so the best one grows
+    // with the square root of the call's crossings, which are about n^2 / 150 per slice. Measured best (and their
+    // neighbours at half and double): 8 slices of 64^2 2, 41 of 192^2 4, 300 of 128^2 32, 300 of 256^2 32-64, 1,000 of
+    // 256^2 64-128, 4,096 of 256^2 128.
+    const double best = static_cast<double>(nn) * std::sqrt(static_cast<double>(n_slices)) / 110.0;
+    i64 per_item = pe ? std::max(1, std::atoi(pe)) : std::min<i64>(256, std::max<i64>(2, std::llround(best)));
+    const i64 most = 0x7fffffffLL / plan.n_boxes;              // parts of a box that the grid can hold
+    per_item = std::max(per_item, (n_slices + most - 1) / most);
+    const i64 max_items = (n_slices + per_item - 1) / per_item;
+    RasterBoxParams<In, Out> q{};
     q.in = p.in; q.is_b = p.is_b; q.is_y = p.is_y; q.is_x = p.is_x; q.in_is_value = p.in_is_value;
     q.in_value = p.in_value;
     q.win = p.win; q.wis_b = p.wis_b; q.wis_y = p.wis_y; q.wis_x = p.wis_x; q.win_present = p.win_present;
@@ -450,19 +740,39 @@ int run_tiles(const ProjectDesc& d, const RasterParams<C, In, Out, W>& p, hipStr
     q.rot = p.rot;
     q.scale = p.scale;
     q.scaled = p.general && p.scale.kind != NOA_HIP_XFORM_NONE;
-    q.items = plan.items;
+    q.boxes = plan.boxes;
+    q.n_boxes = plan.n_boxes;
+    q.per_item = static_cast<i32>(per_item);
+    q.max_items = static_cast<i32>(max_items);
     q.n = static_cast<i32>(nn);
-    q.nty = plan.nty; q.ntx = plan.ntx; q.base = plan.base;
+    q.nby = plan.nby; q.nbx = plan.nbx; q.base = plan.base;
     q.n_slices = static_cast<i32>(n_slices);
     q.pixels = p.pixels;
     q.inv_wr = 1.f / static_cast<float>(p.slice_wr);
+    q.inv_n = 1.f / static_cast<float>(nn);
     q.cutoff_sqd = p.cutoff_sqd;
     q.margin = 1e-3f + 1e-5f * static_cast<float>(nn);
     q.vol_centered = p.vol_centered;
     q.slice_centered = p.slices_centered;
-    hipLaunchKernelGGL((rasterize_tile_kernel<In, Out>), dim3(static_cast<u32>(plan.n_items)), dim3(256), 0, stream,
-                       q);
-    const hipError_t e = hipGetLastError();
+    const bool gen = q.scaled || p.rot.kind == NOA_HIP_QUAT_F32;
+    const dim3 boxes(static_cast<u32>(plan.n_boxes * max_items));
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(stream, &capture);
+    if (n_slices > 64 && capture == hipStreamCaptureStatusNone) {
+        if (hipMallocAsync(reinterpret_cast<void**>(&q.starts), static_cast<size_t>(plan.n_boxes) * max_items * sizeof(i32),
+                           stream) == hipSuccess)
+            hipLaunchKernelGGL((rasterize_items_kernel<In, Out>), dim3(static_cast<u32>(plan.n_boxes)), dim3(RB_SCAN), 0,
+                               stream, q);
+        else
+            (void)hipGetLastError(), q.starts = nullptr;
+    }
+    if (gen) hipLaunchKernelGGL((rasterize_box_kernel<In, Out, true>), boxes, dim3(64), 0, stream, q);
+    else hipLaunchKernelGGL((rasterize_box_kernel<In, Out, false>), boxes, dim3(64), 0, stream, q);
+    hipError_t e = hipGetLastError();
+    if (q.starts) {
+        const hipError_t fe = hipFreeAsync(q.starts, stream);
+        if (e == hipSuccess) e = fe;
+    }
     if (e != hipSuccess) { err = std::string("kernel launch failed: ") + hipGetErrorString(e); return NOA_HIP_ERROR_RUNTIME; }
     return NOA_HIP_OK;
 }

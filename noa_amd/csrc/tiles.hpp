@@ -1,5 +1,5 @@
-// Volume tiles of 16^3 sample positions, each visited by the slices whose plane crosses it: the enumeration shared by
-// the tiled extraction and the tiled rasterisation, and their work plan.
+// Volume tiles of 16^3 sample positions, each visited by the slices whose plane crosses it: the enumeration of the tiled
+// extraction and its work plan.
 //
 // Positions are the floor of a slice pixel's (flipped) coordinates in samples. With cutoff <= 0.5 every pixel inside
 // the cutoff has its floor within [lo - 1, hi + 1] along z and y and [0, n/2] along x, which the tiles cover. For a
@@ -44,27 +44,15 @@ __device__ __forceinline__ bool tile_crossed(const Rot<float>& r, float cz, floa
     return d <= (0.5f * XT) * sum + M * sum + 1e-6f;
 }
 
-// The same test for a box of EZ x 16 x 16 positions (a slab of a tile), centre c.
-template<int EZ>
-__device__ __forceinline__ bool slab_crossed(const Rot<float>& r, float cz, float cy, float cx, float M) {
-    const float nz = r.m[4] * r.m[8] - r.m[7] * r.m[5];
-    const float ny = r.m[7] * r.m[2] - r.m[1] * r.m[8];
-    const float nx = r.m[1] * r.m[5] - r.m[4] * r.m[2];
-    const float d = fabsf((nz * cz + ny * cy) + nx * cx);
-    const float sum = fabsf(nz) + fabsf(ny) + fabsf(nx);
-    return d <= (0.5f * EZ) * fabsf(nz) + (0.5f * XT) * (fabsf(ny) + fabsf(nx)) + M * sum + 1e-6f;
-}
-
-// The candidate pixels of one (box, crossing slice) pair; the box is [Z0, Z0 + EZ) x [Y0, Y0 + 16) x [X0, X0 + 16)
-// (a whole tile when EZ = 16). Cand: the caller's candidate type with a `bool ok`; fetch(fy, u, mirrored, Cand&)
-// evaluates one candidate, store(const Cand&) finishes it. `wl`: the wave's list of LIST words in LDS, which must
-// hold a whole row (n/2 + 1 <= LIST: rows enter the list whole). A degenerate transform (collapsed plane) makes every
+// The candidate pixels of one (tile, crossing slice) pair; the tile is [Z0, Z0 + 16) x [Y0, Y0 + 16) x [X0, X0 + 16).
+// Cand: the caller's candidate type with a `bool ok`; fetch(fy, u, mirrored, Cand&) evaluates one candidate,
+// store(const Cand&) finishes it. `wl`: the wave's list of XT_LIST words in LDS, which must hold a whole row
+// (n/2 + 1 <= XT_LIST: rows enter the list whole). A degenerate transform (collapsed plane) makes every
 // pixel of the slice a candidate.
-template<class Cand, int EZ = XT, int LIST = XT_LIST, class Fetch, class Store>
+template<class Cand, class Fetch, class Store>
 __device__ __forceinline__ void tile_candidates(const Rot<float>& r, i32 Z0, i32 Y0, i32 X0, i32 n, float M, i32 pixels,
                                                 float inv_wr, bool slice_centered, i32 lane, u32* wl, Fetch& fetch,
                                                 Store& store) {
-    constexpr i32 EXT[3] = {EZ, XT, XT};
     const i32 lo = -n / 2, hi = (n - 1) / 2, hix = n / 2;
     // Plane coordinates: F = Y a + U c (a, c: the 2nd and 3rd columns); on the plane Y = g . F with g the
     // first row of (G^T G)^-1 G^T, G = [a c].
@@ -97,8 +85,8 @@ __device__ __forceinline__ void tile_candidates(const Rot<float>& r, i32 Z0, i32
     float blo[3], bhi[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-        blo[i] = (mirrored ? -(P0[i] + EXT[i]) : P0[i]) - M;
-        bhi[i] = (mirrored ? -P0[i] : P0[i] + EXT[i]) + M;
+        blo[i] = (mirrored ? -(P0[i] + XT) : P0[i]) - M;
+        bhi[i] = (mirrored ? -P0[i] : P0[i] + XT) + M;
     }
     float ymin = 0.f, ymax = 0.f;
 #pragma unroll
@@ -135,7 +123,7 @@ __device__ __forceinline__ void tile_candidates(const Rot<float>& r, i32 Z0, i32
         const i32 total = __builtin_amdgcn_readlane(incl, 63);
         for (i32 done = 0; done < total;) {
             // Whole rows into the list, as many as fit (rows are short: at most n/2 + 1 pixels).
-            const bool fits = cnt > 0 && excl >= done && incl <= done + LIST;
+            const bool fits = cnt > 0 && excl >= done && incl <= done + XT_LIST;
             const unsigned long long fm = __ballot(fits);
             const i32 last = 63 - __clzll(static_cast<long long>(fm));
             const i32 upto = __builtin_amdgcn_readlane(incl, last);
@@ -178,10 +166,6 @@ struct TilePlan {
 inline std::mutex g_tile_mutex;
 inline std::map<std::tuple<int, i32, double, i32, i32>, TilePlan> g_tile_plans;
 
-// A negative `pairs` is a default: at most -pairs expected crossing slices per item, fewer when the call's expected
-// crossings would fill fewer than TILE_MIN_ITEMS items (small calls: more, shorter items keep every CU busy).
-constexpr double TILE_MIN_ITEMS = 512;
-
 inline int make_tile_plan(int device, i32 n, double cutoff, i32 n_slices, i32 pairs, TilePlan& plan, std::string& err) {
     const auto key = std::make_tuple(device, n, cutoff, n_slices, pairs);
     std::lock_guard<std::mutex> lock(g_tile_mutex);
@@ -197,8 +181,6 @@ inline int make_tile_plan(int device, i32 n, double cutoff, i32 n_slices, i32 pa
     pl.ntx = (n / 2 + 1 + XT - 1) / XT;
     const double rc = cutoff * n + 1.0;
     struct Entry { double work; int4 item; };
-    struct Active { i32 tile; double expected; };
-    std::vector<Active> active;
     std::vector<Entry> entries;
     for (i32 tz = 0; tz < pl.ntz; ++tz)
         for (i32 ty = 0; ty < pl.nty; ++ty)
@@ -214,22 +196,16 @@ inline int make_tile_plan(int device, i32 n, double cutoff, i32 n_slices, i32 pa
                 }
                 if (closest > rc * rc) continue;
                 const double frac = std::min(1.0, 1.5 * 0.5 * XT / std::max(std::sqrt(r2), 1e-9));
-                active.push_back({(tz * pl.nty + ty) * pl.ntx + tx, frac * n_slices});
+                const double expected = frac * n_slices;
+                const i32 n_seg = std::max<i32>(1, static_cast<i32>(std::ceil(expected / pairs)));
+                const i32 len = (n_slices + n_seg - 1) / n_seg;
+                for (i32 sgm = 0; sgm < n_seg; ++sgm) {
+                    const i32 b = sgm * len, e = std::min(n_slices, b + len);
+                    if (b < e)
+                        entries.push_back({expected / n_seg + (e - b) / 64.0,
+                                           make_int4((tz * pl.nty + ty) * pl.ntx + tx, b, e, 0)});
+                }
             }
-    double per_item = pairs;
-    if (pairs < 0) {
-        double total = 0;
-        for (const Active& a : active) total += a.expected;
-        per_item = std::min(static_cast<double>(-pairs), std::max(8.0, total / TILE_MIN_ITEMS));
-    }
-    for (const Active& a : active) {
-        const i32 n_seg = std::max<i32>(1, static_cast<i32>(std::ceil(a.expected / per_item)));
-        const i32 len = (n_slices + n_seg - 1) / n_seg;
-        for (i32 sgm = 0; sgm < n_seg; ++sgm) {
-            const i32 b = sgm * len, e = std::min(n_slices, b + len);
-            if (b < e) entries.push_back({a.expected / n_seg + (e - b) / 64.0, make_int4(a.tile, b, e, 0)});
-        }
-    }
     std::stable_sort(entries.begin(), entries.end(), [](const Entry& a, const Entry& b) { return a.work > b.work; });
     std::vector<int4> items(entries.size());
     for (size_t k = 0; k < entries.size(); ++k) items[k] = entries[k].item;

@@ -1,8 +1,8 @@
-"""The tiled rasterisation (LDS accumulators per 16^3 volume tile, each tile visited by the slices whose plane
+"""The tiled rasterisation (LDS accumulators per box of the volume, each box visited by the slices whose plane
 crosses it, one device-wide atomic flush per work item).
 
-It takes launches of 64 slices or more into a cubic volume with FP32 values and weights, Mat33<f32> or
-Quaternion<f32> rotations, Mat22 inverse scalings or none, no Ewald curvature and cutoff <= 0.5; NOA_HIP_RASTERIZE_LAYOUT=tiles|direct forces either path. Bars: rel-L2 1e-6 of values and weights
+It takes launches into a cubic volume with FP32 values and weights, Mat33<f32> or
+Quaternion<f32> rotations, Mat22 inverse scalings or none, no Ewald curvature and cutoff <= 0.5; NOA_HIP_RASTERIZE_LAYOUT=direct selects the other path. Bars: rel-L2 1e-6 of values and weights
 against the oracle (noa's per-pixel scatter; the sums are regrouped, by LDS and device atomics in both paths) and
 against the one-lane-per-pixel kernel.
 """
@@ -245,3 +245,76 @@ def test_tiles_take_inverse_scalings(monkeypatch, remap, n, b, quat):
     assert np.abs(want_v).max() > 0
     assert rel_l2(got["v"], want_v) < 1e-6 and rel_l2(got["w"], want_w) < 1e-6
     assert rel_l2(got["v"], direct["v"]) < 1e-6 and rel_l2(got["w"], direct["w"]) < 1e-6
+
+
+def _tilt_series(b, rng):
+    tilt = np.deg2rad(np.linspace(-60, 60, b))
+    return np.stack([nx().rotate_z(0.4) @ nx().rotate_y(t) for t in tilt]).astype(np.float32)
+
+
+@pytest.mark.parametrize("n,b,kind,per_item", [
+    (16, 1, "plain", None),         # the smallest size; fewer positions than a box
+    (17, 64, "plain", 3),           # the most slices without the items kernel
+    (40, 65, "quat", 2),            # the fewest with it
+    (41, 257, "scaled", 5),         # one slice past a scan of the items kernel
+    (24, 5, "strided", None),       # real slices with a pitch and a batch gap
+    (64, 300, "tilt", 7),           # boxes on the tilt axis: every slice, many items
+    (766, 1, "plain", None),        # the largest size
+])
+def test_boxes_match_the_oracle(monkeypatch, n, b, kind, per_item):
+    """Every pixel is rasterised once whatever the split into items: against the oracle, rel-L2 1e-6 (sums of at most a
+    few hundred FP32 terms in another order: 2^-24 times the square root of their number, about 1e-6 at the worst)."""
+    print(f"case rasterize boxes n={n} b={b} {kind} per_item={per_item}", flush=True)
+    rng = np.random.default_rng(2000 + n + b)
+    monkeypatch.delenv("NOA_HIP_RASTERIZE_LAYOUT", raising=False)
+    if per_item is not None:
+        monkeypatch.setenv("NOA_HIP_RASTERIZE_PAIRS", str(per_item))
+    wr = n // 2 + 1
+    real = kind == "strided"
+    sl = random_spectrum((b, 1, n, wr), rng)
+    sl = sl.real.copy() if real else sl
+    w = rng.uniform(0.1, 1.0, (b, 1, n, wr)).astype(np.float32)
+    rot = _tilt_series(b, rng) if kind == "tilt" else random_rotations(b, rng)
+    scale = _scalings(b, rng) if kind == "scaled" else None
+    if kind == "quat":
+        rot = nx().quaternion_from_matrix(rot.astype(np.float64)).astype(np.float32)
+    gsl = dev(sl)
+    if real:
+        room = torch.zeros((b, 2, n, wr + 3), dtype=torch.float32, device=DEV)
+        room[:, :1, :, :wr] = gsl
+        gsl = room[:, :1, :, :wr]
+    gw, grot = dev(w), (nx().Quaternions(dev(rot)) if kind == "quat" else nx().Mat33Array(dev(rot), DEV))
+    vol = torch.zeros((1, n, n, wr), dtype=gsl.dtype, device=DEV)
+    wv = torch.zeros((1, n, n, wr), dtype=torch.float32, device=DEV)
+
+    def call():
+        vol.zero_()
+        wv.zero_()
+        nx().rasterize_central_slices_3d("h2h", gsl, gw, (b, 1, n, n), vol, wv, (1, n, n, n),
+                                         None if scale is None else dev(scale), grot)
+
+    if n > 300:     # the lane-per-pixel kernel, itself checked against the oracle at the sizes above
+        monkeypatch.setenv("NOA_HIP_RASTERIZE_LAYOUT", "direct")
+        call()
+        want_v, want_w = vol.clone(), wv.clone()
+        monkeypatch.delenv("NOA_HIP_RASTERIZE_LAYOUT")
+    else:
+        want_v, want_w = np.zeros((1, n, n, wr), sl.dtype), np.zeros((1, n, n, wr), np.float32)
+        O.rasterize_central_slices_3d("h2h", sl, w, (b, 1, n, n), want_v, want_w, (1, n, n, n), scale, rot,
+                                      quaternion=kind == "quat", n_threads=8)
+        want_v, want_w = dev(want_v), dev(want_w)
+
+    def check():
+        for got, want in ((vol, want_v), (wv, want_w)):
+            assert float(torch.linalg.vector_norm(got - want) / torch.linalg.vector_norm(want)) < 1e-6
+
+    call()
+    check()
+    if scale is None and kind != "quat":         # captured: nothing is allocated, the items scan for their slices
+        stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call()
+        for _ in range(3):
+            vol.fill_(1)
+            graph.replay()
+            check()
