@@ -28,7 +28,7 @@ PROFILES = ROOT / "profiles"
 
 KERNELS = {
     "insert": {"one-wave": "insert_wave_kernel (+ insert_reduce_kernel)",
-               "slab": "insert_slab_kernel (+ slab_records_kernel and insert_reduce_kernel)"},
+               "slab": "insert_slab_kernel (+ insert_reduce_kernel)"},
     "extract": {"block-copy gather": "extract_c32_kernel (+ brick_volume_kernel)",
                 "row-major gather": "extract_c32_kernel",
                 "LDS tiles": "extract_tile_kernel (+ extract_outside_kernel)"},

@@ -265,7 +265,7 @@ int noa_hip_insert_central_slices_3d(const noa_hip_project_args* args, void* str
 
 /* No counterpart in noa: noa_hip_insert_central_slices_3d for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid allocation). Same arguments, rules and results
- * (bit-identical). The work plan, the per-slice records and the partial sums of split sub-bricks are carved from a
+ * (bit-identical). The work plan and the partial sums of split sub-bricks are carved from a
  * static device array of NOA_HIP_NOALLOC_SCRATCH_BYTES per GPU instead of being allocated; a call whose work needs
  * more returns NOA_HIP_ERROR_UNSUPPORTED with the size in noa_hip_last_error() (at 256^3, up to about 5,000 slices
  * fit). Every call on a GPU shares that GPU's array: calls that overlap on one GPU (different streams, or
@@ -324,7 +324,7 @@ int noa_hip_volume_blocks(const noa_hip_view* volume, void* blocks, int64_t capa
  *   NOA_HIP_OP_INSERT_BATCH:  values = {workgroups (default 3072); -; -; -}
  * Environment variables (NOA_HIP_EXTRACT_LAYOUT, NOA_HIP_EXTRACT_PAIRS, NOA_HIP_INSERT_KERNEL, NOA_HIP_INSERT_LIST,
  * NOA_HIP_INSERT_PAIRED, NOA_HIP_INSERT_ORDER) override the table; NOA_HIP_INSERT_SPAN sets the most slices of one
- * insertion work item (default 1024, 0: no bound; not applied by the allocation-free entry point or item order 3). */
+ * insertion work item (default a quarter of the slices, between 256 and 1024; 0: no bound; not applied by the allocation-free entry point or item order 3). */
 enum {
     NOA_HIP_OP_EXTRACT = 1,
     NOA_HIP_OP_INSERT = 2,

@@ -126,6 +126,13 @@ __device__ __forceinline__ i32 frequency2index(bool centered, i32 frequency, i32
     return frequency < 0 ? frequency + size : frequency;
 }
 
+// i / n rounded to nearest, for integers |i| <= n < 2^12 with inv_n = 1 / n rounded: one Newton step on the product
+// (the remainder is exact); the same as the division for every such pair.
+__device__ __forceinline__ float divide_index(float i, float n, float inv_n) {
+    const float q = i * inv_n;
+    return fmaf(fmaf(-q, n, i), inv_n, q);
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // Transforms. A transform is read from device memory (batched) or from the kernel arguments (broadcast).
 // ---------------------------------------------------------------------------------------------------------

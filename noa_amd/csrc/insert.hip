@@ -20,9 +20,9 @@
 //     balanced. A sub-brick with one segment adds its sum to the volume directly; a split sub-brick writes one
 //     partial sum per segment, and a second kernel adds the partials of each sub-brick in segment order. The
 //     result is deterministic; it differs from noa's strict slice order only by this regrouping of the sum.
-//   - insert_slab_kernel serves the common configuration (one power-of-two size, Mat33<f32> or Quaternion<f32>,
-//     LINEAR, cutoff <= 0.5, no scaling) with per-slice records and a leaner per-voxel path; insert_wave_kernel
-//     serves the others (inverse scalings, NEAREST, other sizes and cutoffs).
+//   - insert_slab_kernel serves the common configuration (one size for slices, volume and target, Mat33<f32>, LINEAR,
+//     cutoff <= 0.5, no scaling; Quaternion<f32> at a power of two) with a leaner enumeration and the loads of the next
+//     slice in flight; insert_wave_kernel serves the others (inverse scalings, NEAREST, other shapes and cutoffs).
 // General path (EWS, constant-value inputs, double precision): noa's per-voxel gather over every slice, one lane
 // per voxel.
 #include <type_traits>
@@ -72,6 +72,7 @@ struct InsertParams {
     bool wpoly;           // use wa; otherwise evaluate noa's expression
     float inv_fb;         // 1 / fftfreq_blackman
     u32 slice_bytes, wslice_bytes;   // byte extent of one slice and of its weights (buffer loads)
+    bool freq_order;      // sub-bricks cut in frequency order (slab kernel), not in index order
     int interp_mode;      // the method of the INTERP_WINDOW instantiation (CUBIC, CUBIC_BSPLINE, LANCZOS*)
 };
 
@@ -580,37 +581,6 @@ __global__ __launch_bounds__(64) void insert_wave_kernel(const InsertParams<C, I
     insert_wave_item<C, In, Out, W, INTERP, HOT>(p, item, acc_v, acc_w, cand);
 }
 
-// Batched insertion: several insertion calls (each its own volume, box size, layout, slice count and cutoff) in one
-// persistent launch of the one-wave kernel. The device image of a batch holds a header, one parameter block per call
-// and the work items of every call ({sub-brick, first slice, end slice, call}; the calls' slice ranges are not split,
-// so no partial sums); workgroup g takes the items g, g + G, ... (items of each call sorted by expected work, calls
-// interleaved by the host). Each item runs the one-wave kernel's code with its call's parameters: the results are
-// those of the calls made one by one (same per-voxel sums, in slice order).
-struct InsertBatchHeader {
-    i32 n_items, n_jobs;
-    i32 jobs_offset, items_offset;       // bytes from the start of the image
-    i32 pad[12];
-};
-static_assert(sizeof(InsertBatchHeader) == 64, "batch header");
-
-__global__ __launch_bounds__(64) void insert_batch_kernel(const unsigned char* __restrict__ image) {
-    using P = InsertParams<float, float2, float>;
-    __shared__ float2 acc_v[WVOX];
-    __shared__ float acc_w[WVOX];
-    __shared__ i32 cand[64 * WG];
-    const InsertBatchHeader* h = reinterpret_cast<const InsertBatchHeader*>(image);
-    const P* __restrict__ jobs = reinterpret_cast<const P*>(image + h->jobs_offset);
-    const int4* __restrict__ items = reinterpret_cast<const int4*>(image + h->items_offset);
-    const i32 n_items = h->n_items;
-    for (i32 i = static_cast<i32>(blockIdx.x); i < n_items; i += static_cast<i32>(gridDim.x)) {
-        int4 item = items[i];
-        const P& p = jobs[item.w];
-        item.w = -1;
-        __syncthreads();   // the previous item's flush has read the accumulator
-        insert_wave_item<float, float2, float2, float, NOA_HIP_INTERP_LINEAR, 0>(p, item, acc_v, acc_w, cand);
-    }
-}
-
 // Adds the partial sums of each split brick to the volume, in segment order.
 template<class C, class In, class Out, class W>
 __global__ __launch_bounds__(NT_REDUCE) void insert_reduce_kernel(const InsertParams<C, In, W> p) {
@@ -624,8 +594,13 @@ __global__ __launch_bounds__(NT_REDUCE) void insert_reduce_kernel(const InsertPa
     const i64 slot = static_cast<i64>(bd0) * bd1 * p.apitch;
     for (i32 v = static_cast<i32>(threadIdx.x); v < bd0 * bd1 * bd2; v += NT_REDUCE) {
         const i32 lz = v / (bd1 * bd2), ly = (v / bd2) % bd1, lx = v % bd2;
-        const i32 z = org[0] + lz, y = org[1] + ly, x = org[2] + lx;
+        i32 z = org[0] + lz, y = org[1] + ly;
+        const i32 x = org[2] + lx;
         if (z >= ext[0] || y >= ext[1] || x >= ext[2]) continue;
+        if (p.freq_order) {
+            z = frequency2index(p.vol_centered, z - p.grid[0] / 2, p.grid[0]);
+            y = frequency2index(p.vol_centered, y - p.grid[1] / 2, p.grid[1]);
+        }
         vec3<C> f;
         f.z = static_cast<C>(index2frequency(p.vol_centered, z, p.grid[0])) / p.target[0];
         f.y = static_cast<C>(index2frequency(p.vol_centered, y, p.grid[1])) / p.target[1];
@@ -649,27 +624,45 @@ __global__ __launch_bounds__(NT_REDUCE) void insert_reduce_kernel(const InsertPa
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Slab kernel: the common single-precision configuration (Mat33<f32> rotations, c32 or f32 slices with f32 or no
-// weights, LINEAR, one power-of-two size n for the slices, the volume and the target, cutoff <= 0.5, no scaling
-// or Ewald sphere). Same work items and sub-bricks as the one-wave kernel, with less work per pair and per voxel:
-//   - A prologue kernel writes one record per slice: the rotation, the volume axis A closest to the slab normal
-//     and the slab's centre and half-width along A as linear functions of the two other coordinates.
+// Slab kernel: the common single-precision configuration (Mat33<f32> or Quaternion<f32> rotations, c32 or f32 slices
+// with f32 or no weights, LINEAR, one size n for the slices, the volume and the target, cutoff <= 0.5, no scaling or
+// Ewald sphere). Sub-bricks as in the one-wave kernel, but cut in frequency order whatever the volume's layout (the
+// frequencies inside a sub-brick are contiguous for every n; the flush maps them to the layout), with less work per pair
+// and per voxel:
+//   - Lanes set up 64 slices at a time: the volume axis A closest to the slab normal, and the slab's centre and
+//     half-width along A as linear functions of the two other coordinates. A passing slice is broadcast from its lane.
 //   - Per (sub-brick, slice) pair, each lane takes one or two columns of the sub-brick face across A, clamps the
-//     slab range of its column to the sub-brick and to the cutoff sphere (exact integer test, precomputed per
-//     column), and the candidates are packed into an LDS list by ballots (one per candidate rank j).
-//   - Per candidate, the coordinates are noa's expressions in sample units: with n a power of two,
-//     R * (index / n) * n rounds exactly like R * index, so pz, py, px are noa's fz*n, f2y*n, f2x*n bit for bit.
-//     The window is a degree-9 polynomial in t = 2 (pz/fbT)^2 - 1 (fitted per window, error < 4e-7), folded
-//     into the bilinear weights; taps beyond noa's frequency bounds get weight 0 and never load outside the slice
-//     (buffer resources). Sums are added to the LDS accumulator (plain read-modify-write: a voxel is met at most
-//     once per slice and slices are processed in order, so the result is deterministic). The tap loads of the next
-//     passing slice are issued before the current slice's sums are added.
+//     slab range of its column to the sub-brick and to the cutoff sphere (precomputed per column), and the candidates
+//     are packed into an LDS list by ballots (one per candidate rank j).
+//   - Per candidate, the coordinates are noa's expressions: R * (index / n), then times n. With n a power of two (POW2)
+//     that rounds exactly like R * index, so they are computed in samples; otherwise the division is a product with the
+//     rounded reciprocal and one Newton step, which rounds like it.
+//   - The tap loads of all candidates of a pair (at most 128, in two groups; further ones are rare and wait) are issued
+//     together, then the sums of the previous pair are added. Together, because neighbouring candidates read the same
+//     lines while the L1 still holds them: the groups of several pairs in a ring, more of them in flight, read 31 % more
+//     from the L2 and took 5.1 instead of 4.7 ms (10,000 slices of 256^2). Taps beyond noa's frequency bounds, which
+//     only the pairs near the edge of the slice can have, read outside the slice's buffer, which returns 0. Sums are
+//     added to the LDS accumulator by plain read-modify-write: a voxel is met at most once per slice and slices are
+//     processed in order, so the result is deterministic.
+//   - Arithmetic of the sums, POW2: the window is a polynomial of degree 9 in t = 2 (pz/fbT)^2 - 1 (fitted per window,
+//     error < 4e-7), folded into the bilinear weights. Other sizes: the one-wave kernel's window polynomial and order of
+//     the taps, so both kernels give the same bits; the batched launches use it at every size (with n a power of two the
+//     division is exact).
+// Measured against the one-wave kernel at sizes that are not a power of two: 1,000 slices of 150^2 0.24 against 1.21 ms,
+// 41 tilts of 192^2 131 against 241 us (one item of the tilt axis after the other: latency), 2,000 tilts of 200^2 1.8
+// against 8.3 ms; 10,000 slices of 256^2 4.6 ms, bound by L2 misses (4.4 times the algorithmic bytes) at 1.8e9 VALU
+// instructions.
 // ---------------------------------------------------------------------------------------------------------
 constexpr i32 SLAB_NWIN = 9;        // degree of the window polynomial
+constexpr i32 SLAB_WAVES = 3;       // waves per SIMD: the 12 per CU that 13 KB of LDS each allow (at 2: 5.7 ms, not 4.6)
 // Candidates of one pair: at most 4 per column (the slab kernel runs for fbT <= 1.15 samples, so a column's slab
-// range is shorter than 2 * (1.15 * sqrt(3) + 2e-3) < 4 samples) over at most 128 columns (the 8 x 16 faces).
+// range is shorter than 2 * (1.15 * sqrt(3) + margin) < 4 samples) over at most 128 columns (the 8 x 16 faces).
 constexpr i32 SLAB_MAXC = 512;
 static_assert(WZ == 8 && WY == 8 && WX == 16, "slab candidate words decode lz = v >> 7, ly = (v >> 4) & 7, lx = v & 15");
+// Element index past the end of any slice or weight buffer of the slab kernel (below 2^30 bytes), also with the 16 bytes
+// of a paired load: such a load returns 0.
+constexpr u32 SLAB_OUTSIDE = 0x0FFFFFF0u;
+constexpr u32 SLAB_MAX_BYTES = 0x3FFFFF00u;
 
 template<class In, class W>
 struct SlabParams {
@@ -683,43 +676,18 @@ struct SlabParams {
     i32 nb[3];                          // sub-bricks along z, y, x
     const int4* items;                  // {sub-brick, first slice, end slice, partial slot or -1}
     float* partials;
-    const float4* rec;                  // 4 float4 per slice
+    XformArg<float> rot;
     i32 n_slices;
-    float fbT;                          // window half-width f_b * n, in samples
-    float tk;                           // 2 / fbT^2
-    float wa[SLAB_NWIN + 1];
-    float cut2;                         // cutoff^2 * n^2: a voxel is inside when iz^2 + iy^2 + ix^2 <= cut2
-    bool vol_centered;
+    float reach;                        // window half-width f_b * n, in samples
+    float margin;                       // samples: the rounding of the exact per-voxel test, with room
+    float fbT, tk;                      // window half-width in the units of pz (POW2: samples), 2 / fbT^2
+    float wa[NWIN + 1];                 // window polynomial (not POW2: the one-wave kernel's, degree NWIN)
+    float inv_fb, inv_n;
+    float cut2;                         // POW2: a voxel is inside when iz^2 + iy^2 + ix^2 <= cut2 (samples)
+    float cut2_columns;                 // the columns' bound, not below the exact one
+    float cutoff_sqd;
+    bool vol_centered, slice_centered;
 };
-
-// One record per slice: {R00, R01, R02, -}, {R10, R11, R12, ub}, {R20, R21, R22, uc}, {hw, A, passes, -}. With n =
-// the first row (pz = n . v in samples), A = argmax |n_a|, B < C the other axes: the slab |pz| <= fbT runs along A
-// around ub * v_B + uc * v_C (ub = -n_B / n_A, uc = -n_C / n_A) with half-width fbT / |n_A|, widened by 2e-3
-// samples to cover the rounding of the exact per-voxel test (a few 1e-5 samples). A column holds at most
-// floor(2 hw) + 1 candidates: at most 4 when the row is a unit vector (|n_A| >= 1/sqrt(3), fbT <= 1.15), more when
-// it is shorter; `passes` = the packing passes of 4 ranks each that the slice needs (1 for rotations).
-__global__ __launch_bounds__(256) void slab_records_kernel(const XformArg<float> rot, i32 n_slices, float fbT,
-                                                           float4* rec) {
-    const i32 s = static_cast<i32>(blockIdx.x) * 256 + static_cast<i32>(threadIdx.x);
-    if (s >= n_slices) return;
-    float m[9];
-    rot_matrix(load_rotation(rot, s), m);      // a quaternion's matrix: its rotation up to rounding
-    const float a0 = fabsf(m[0]), a1 = fabsf(m[1]), a2 = fabsf(m[2]);
-    i32 ax = 0;
-    if (a1 > a0) ax = 1;
-    if (a2 > (ax == 0 ? a0 : a1)) ax = 2;
-    const float nA = m[ax];
-    const float nB = ax == 0 ? m[1] : m[0];
-    const float nC = ax == 2 ? m[1] : m[2];
-    const float inv = 1.f / nA;
-    float4* o = rec + 4 * static_cast<i64>(s);
-    o[0] = make_float4(m[0], m[1], m[2], 0.f);
-    o[1] = make_float4(m[3], m[4], m[5], -nB * inv);
-    o[2] = make_float4(m[6], m[7], m[8], -nC * inv);
-    const float hw = fbT * fabsf(inv) + 2e-3f;
-    const i32 passes = (static_cast<i32>(fminf(2.f * hw, 15.f)) + 4) >> 2;
-    o[3] = make_float4(hw, __int_as_float(ax), __int_as_float(passes), 0.f);
-}
 
 // Largest integer m >= 0 with m^2 + r2 <= cut2 (all values exact in single precision), or -1 if none.
 __device__ __forceinline__ float sphere_half_extent(float r2, float cut2) {
@@ -768,6 +736,9 @@ __device__ __forceinline__ u32 lanes_below(unsigned long long m) {
     return __builtin_amdgcn_mbcnt_hi(static_cast<u32>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<u32>(m), 0u));
 }
 
+// Orders the LDS accesses of a one-wave workgroup for the compiler; LDS itself runs one wave's instructions in order.
+__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
+
 // Packs the candidates of ranks j0, j0 + 1, ... (at most `jn` ranks) of one face orientation into `cand` (ordered by
 // rank, then slot, then lane); returns their number. `u0`: the slab centre along A at face coordinates (0, 0),
 // relative to the sub-brick's first sample. Rotations: j0 = 0 and every rank (at most 4 per column, so at most
@@ -804,252 +775,322 @@ __device__ __forceinline__ u32 slab_candidates(unsigned short* cand, const SlabC
     return off;
 }
 
+// One group of candidates, its tap loads in flight. POW2: w00..w11 are the bilinear weights times the window;
+// otherwise w00, w01 are the fractions along y and x.
 template<class In, class W>
 struct SlabTaps {
     In v00, v01, v10, v11;
     W q00, q01, q10, q11;
-    float ty, tx, win;
-    u32 lv;
-    bool hit, flip, oky0, oky1, okx1;
+    float w00, w01, w10, w11, win;
+    u32 lv;                             // voxel | SLAB_FLIP | SLAB_EDGE
+    bool hit;
 };
+constexpr u32 SLAB_FLIP = 0x80000000u;  // early flip: the imaginary part is negated
+constexpr u32 SLAB_EDGE = 0x40000000u;  // the x + 1 taps lie beyond the stored half
 
-template<class In, class Out, class W, bool SC, bool PAIRED>
-__global__ __launch_bounds__(64) void insert_slab_kernel(const SlabParams<In, W> p) {
+template<class In, class Out, class W, bool HASW, bool POW2, bool PAIRED>
+__device__ __forceinline__ void insert_slab_item(const SlabParams<In, W>& p, int4 item, float* __restrict__ acc,
+                                                 unsigned short* __restrict__ cand) {
     constexpr bool CX = vt<In>::cx;
+    constexpr bool EXACT = !POW2;                      // the one-wave kernel's arithmetic
     constexpr i32 NCH = CX ? 3 : 2;                    // accumulator channels: re (, im), weight
-    __shared__ float acc[NCH * WVOX];
-    __shared__ unsigned short cand[SLAB_MAXC];
-
     const i32 lane = static_cast<i32>(threadIdx.x);
-    int4 item = p.items[blockIdx.x];
-    if (item.x < 0) return;                 // padding of an XCD-ordered plan
     item.z = min(item.z, p.n_slices);
     item.y = min(item.y, item.z);
     const i32 brick = item.x;
     const i32 bxi = brick % p.nb[2];
     const i32 rem = brick / p.nb[2];
-    const i32 byi = rem % p.nb[1];
-    const i32 bzi = rem / p.nb[1];
     const i32 n = p.n, half = n / 2, wr = half + 1;
-    const i32 org[3] = {bzi * WZ, byi * WY, bxi * WX};
-    const bool vc = p.vol_centered;
-    // First frequency of each axis of the sub-brick: frequencies are contiguous inside a sub-brick because n/2 is
-    // a multiple of the sub-brick sizes.
-    i32 f0[3], nin[3];
-    f0[0] = vc ? org[0] - half : (org[0] < half ? org[0] : org[0] - n);
-    f0[1] = vc ? org[1] - half : (org[1] < half ? org[1] : org[1] - n);
-    f0[2] = org[2];
-    nin[0] = WZ;
-    nin[1] = WY;
-    nin[2] = min(WX, wr - org[2]);
+    const i32 org[3] = {rem / p.nb[1] * WZ, rem % p.nb[1] * WY, bxi * WX};
+    // First frequency of each axis of the sub-brick, and its voxels inside the volume.
+    const i32 f0[3] = {org[0] - half, org[1] - half, org[2]};
+    const i32 nin[3] = {min(WZ, n - org[0]), min(WY, n - org[1]), min(WX, wr - org[2])};
 
     for (i32 v = lane; v < NCH * WVOX; v += 64) acc[v] = 0.f;
 
-    // Column data of the three face orientations (slot 1 of AX 0 and 1: the columns lane + 64).
+    // Column data of the three face orientations (slot 1 of AX 0 and 1: the next 8 columns along x).
     SlabColumn c0[2], c1[2], c2[2];
     // 8 x 8 patches of columns per slot: the 64 lanes of a candidate group project onto a compact patch of the
     // slice, whatever its in-plane rotation (fewer cache lines per tap load than 4 x 16 strips).
-    c0[0] = slab_column<0>(lane >> 3, lane & 7, f0, nin, p.cut2);
-    c0[1] = slab_column<0>(lane >> 3, (lane & 7) + 8, f0, nin, p.cut2);
-    c1[0] = slab_column<1>(lane >> 3, lane & 7, f0, nin, p.cut2);
-    c1[1] = slab_column<1>(lane >> 3, (lane & 7) + 8, f0, nin, p.cut2);
-    c2[0] = slab_column<2>(lane >> 3, lane & 7, f0, nin, p.cut2);
+    c0[0] = slab_column<0>(lane >> 3, lane & 7, f0, nin, p.cut2_columns);
+    c0[1] = slab_column<0>(lane >> 3, (lane & 7) + 8, f0, nin, p.cut2_columns);
+    c1[0] = slab_column<1>(lane >> 3, lane & 7, f0, nin, p.cut2_columns);
+    c1[1] = slab_column<1>(lane >> 3, (lane & 7) + 8, f0, nin, p.cut2_columns);
+    c2[0] = slab_column<2>(lane >> 3, lane & 7, f0, nin, p.cut2_columns);
     c2[1] = c2[0];
 
-    // Culling of a slice against the sub-brick box, in samples: |n . centre| <= fbT + |n| . half + slack.
-    const float cz = static_cast<float>(f0[0]) + 0.5f * static_cast<float>(nin[0] - 1);
-    const float cy = static_cast<float>(f0[1]) + 0.5f * static_cast<float>(nin[1] - 1);
-    const float cx = static_cast<float>(f0[2]) + 0.5f * static_cast<float>(nin[2] - 1);
+    // Culling of a slice against the sub-brick box, in samples: |n . centre| <= reach + |n| . half + slack.
     const float hz = 0.5f * static_cast<float>(nin[0] - 1), hy = 0.5f * static_cast<float>(nin[1] - 1);
     const float hx = 0.5f * static_cast<float>(nin[2] - 1);
-    const float fbT = p.fbT;
     const float f0zf = static_cast<float>(f0[0]), f0yf = static_cast<float>(f0[1]), f0xf = static_cast<float>(f0[2]);
+    const float cz = f0zf + hz, cy = f0yf + hy, cx = f0xf + hx;
+    const float reach = p.reach, margin = p.margin;
 
-    // Records of the current chunk of 64 slices (lane l: slice chunk0 + l) and of the next one.
-    auto load_rec = [&](i32 s, float4 (&r)[4]) {
-        if (s < item.z) {
+    // Lane l holds slice chunk0 + l: its rotation m, and with n the first row of m (pz = n . v in samples), A = argmax
+    // |n_a| and B < C the other axes, the slab |pz| <= reach along A: around ub * v_B + uc * v_C (ub = -n_B / n_A, uc =
+    // -n_C / n_A) with half-width reach / |n_A|, widened by the margin. A column holds at most floor(2 hw) + 1
+    // candidates: at most 4 when the row is a unit vector (|n_A| >= 1/sqrt(3), reach <= 1.15), more when it is shorter;
+    // `passes` = the packing passes of 4 ranks each that the slice needs (1 for rotations). The next chunk's rotations
+    // are loaded one chunk ahead.
+    float m[9] = {}, ub = 0.f, uc = 0.f, hw = 0.f;
+    i32 info = 0;                       // axis A | edge << 2 | passes << 3
+    // A slice's taps can reach beyond its bounds when the longest of its in-plane rows takes the voxel farthest from the
+    // origin there.
+    float far2 = 0.f;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) r[q] = p.rec[4 * static_cast<i64>(s) + q];
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) r[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    };
-    float4 cur[4], nxt[4];
+    for (i32 a = 0; a < 3; ++a) {
+        const float f = static_cast<float>(max(abs(f0[a]), abs(f0[a] + nin[a] - 1)));
+        far2 += f * f;
+    }
+    const float far = sqrtf(fminf(far2, p.cut2_columns)), near_edge = static_cast<float>(half) - 2.f;
+    float next[9] = {};
+    const bool quat = !EXACT && p.rot.kind == NOA_HIP_QUAT_F32;
     i32 chunk0 = item.y;
-    load_rec(chunk0 + lane, cur);
-    load_rec(chunk0 + 64 + lane, nxt);
+    auto load = [&](i32 s) {
+        if (s < item.z) {
+            const Rot<float> r = load_rotation(p.rot, s);
+#pragma unroll
+            for (i32 q = 0; q < 9; ++q) next[q] = r.m[q];
+        }
+    };
     auto scan = [&]() -> unsigned long long {
-        const float d = fabsf((cur[0].x * cz + cur[0].y * cy) + cur[0].z * cx);
-        const float bound = fbT + fabsf(cur[0].x) * hz + fabsf(cur[0].y) * hy + fabsf(cur[0].z) * hx;
-        return __ballot(chunk0 + lane < item.z && d <= bound + 2e-3f);
+        bool pass = false;
+        if (chunk0 + lane < item.z) {
+            Rot<float> r;
+            r.quat = quat;
+#pragma unroll
+            for (i32 q = 0; q < 9; ++q) r.m[q] = next[q];
+            rot_matrix(r, m);           // a quaternion's matrix: its rotation up to rounding
+            const float a0 = fabsf(m[0]), a1 = fabsf(m[1]), a2 = fabsf(m[2]);
+            i32 ax = 0;
+            if (a1 > a0) ax = 1;
+            if (a2 > (ax == 0 ? a0 : a1)) ax = 2;
+            const float nA = ax == 0 ? m[0] : (ax == 1 ? m[1] : m[2]);
+            const float nB = ax == 0 ? m[1] : m[0];
+            const float nC = ax == 2 ? m[1] : m[2];
+            const float inv = 1.f / nA;
+            ub = -nB * inv;
+            uc = -nC * inv;
+            hw = reach * fabsf(inv) + margin;
+            const float row1 = (m[3] * m[3] + m[4] * m[4]) + m[5] * m[5], row2 = (m[6] * m[6] + m[7] * m[7]) + m[8] * m[8];
+            const bool edge = !(sqrtf(fmaxf(row1, row2)) * far < near_edge);
+            info = ax | (edge ? 4 : 0) | (((static_cast<i32>(fminf(2.f * hw, 15.f)) + 4) >> 2) << 3);
+            const float d = fabsf((m[0] * cz + m[1] * cy) + m[2] * cx);
+            pass = d <= reach + ((a0 * hz + a1 * hy) + a2 * hx) + margin;
+        }
+        return __ballot(pass);
     };
+    load(chunk0 + lane);
     unsigned long long mask = scan();
+    load(chunk0 + 64 + lane);
 
-    const float wa0 = p.wa[0], wa1 = p.wa[1], wa2 = p.wa[2], wa3 = p.wa[3], wa4 = p.wa[4];
-    const float wa5 = p.wa[5], wa6 = p.wa[6], wa7 = p.wa[7], wa8 = p.wa[8], wa9 = p.wa[9];
-    const float tk = p.tk;
-    const i32 pitch = p.pitch;
-
-    // Phase 2 of a group of candidates: interpolation and accumulation (groups of non-hits skip).
-    auto finish = [&](const SlabTaps<In, W> (&t)[2]) {
+    const float fbT = p.fbT, tk = p.tk, inv_fb = p.inv_fb, inv_n = p.inv_n, nf = static_cast<float>(n);
+    float wa[NWIN + 1];
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            if (!t[g].hit) continue;
-            const float a0 = t[g].oky0 ? (1.f - t[g].ty) * t[g].win : 0.f;
-            const float a1 = t[g].oky1 ? t[g].ty * t[g].win : 0.f;
-            const float bx0 = 1.f - t[g].tx, bx1 = t[g].okx1 ? t[g].tx : 0.f;
-            const float w00 = a0 * bx0, w01 = a0 * bx1, w10 = a1 * bx0, w11 = a1 * bx1;
-            float re, im = 0.f;
-            if constexpr (CX) {
-                re = fmaf(w11, t[g].v11.x, fmaf(w10, t[g].v10.x, fmaf(w01, t[g].v01.x, w00 * t[g].v00.x)));
-                im = fmaf(w11, t[g].v11.y, fmaf(w10, t[g].v10.y, fmaf(w01, t[g].v01.y, w00 * t[g].v00.y)));
-                im = t[g].flip ? -im : im;
-            } else {
-                re = fmaf(w11, t[g].v11, fmaf(w10, t[g].v10, fmaf(w01, t[g].v01, w00 * t[g].v00)));
+    for (i32 k = 0; k <= (EXACT ? NWIN : SLAB_NWIN); ++k) wa[k] = p.wa[k];
+    const i32 pitch = p.pitch;
+    const i32 wrap_neg = p.slice_centered ? half : n, wrap_pos = p.slice_centered ? half : 0;
+
+    // The pair whose candidates are in the list.
+    float R[9] = {};
+    i32 slice = 0, pass = 0;
+    u32 total = 0;
+    bool edge = false;
+    // Packs the candidates of the next pair; false after the last one.
+    auto advance = [&]() -> bool {
+        do {
+            while (mask == 0) {
+                if (chunk0 >= item.z) return false;
+                chunk0 += 64;
+                if (chunk0 >= item.z) return false;
+                mask = scan();
+                load(chunk0 + 64 + lane);
             }
-            const float wt = p.win ? fmaf(w11, t[g].q11, fmaf(w10, t[g].q10, fmaf(w01, t[g].q01, w00 * t[g].q00)))
-                                   : t[g].win;
-            // A voxel is a candidate at most once per slice, and one wave adds its slices in order: plain
-            // read-modify-write.
-            acc[t[g].lv] += re;
-            if constexpr (CX) acc[WVOX + t[g].lv] += im;
-            acc[(NCH - 1) * WVOX + t[g].lv] += wt;
+            const i32 k = __ffsll(static_cast<long long>(mask)) - 1;
+            mask &= mask - 1;
+            slice = chunk0 + k;
+#pragma unroll
+            for (i32 q = 0; q < 9; ++q) R[q] = bcast(m[q], k);
+            const float sub = bcast(ub, k), suc = bcast(uc, k), shw = bcast(hw, k);
+            const i32 sinfo = __builtin_amdgcn_readlane(info, k);
+            // Rotations pack a slice's candidates in one pass (at most 4 per column). Rows that are not unit vectors
+            // thicken the slab: such a slice takes one pass per 4 ranks (a voxel is a candidate at most once per slice,
+            // so the passes add distinct voxels); its bit of the mask is set again until the last pass.
+            const i32 ax = sinfo & 3, passes = sinfo >> 3;
+            edge = (sinfo & 4) != 0;
+            const i32 j0 = 4 * pass, jn = passes > 1 ? 4 : 16;
+            if (passes > 1) {
+                if (++pass < passes) mask |= 1ull << k;
+                else pass = 0;
+            }
+            wave_lds_order();   // the list's previous reads come before it is rewritten
+            if (ax == 0) {
+                const float u0 = fmaf(sub, f0yf, fmaf(suc, f0xf, -f0zf));
+                total = slab_candidates<0, 2>(cand, c0, u0, sub, suc, shw, j0, jn);
+            } else if (ax == 1) {
+                const float u0 = fmaf(sub, f0zf, fmaf(suc, f0xf, -f0yf));
+                total = slab_candidates<1, 2>(cand, c1, u0, sub, suc, shw, j0, jn);
+            } else {
+                const float u0 = fmaf(sub, f0zf, fmaf(suc, f0yf, -f0xf));
+                total = slab_candidates<2, 1>(cand, c2, u0, sub, suc, shw, j0, jn);
+            }
+            wave_lds_order();
+        } while (total == 0);
+        return true;
+    };
+
+    // Coordinates, window, and every tap load of the candidates [base, base + 64) issued.
+    auto issue = [&](u32 base, SlabTaps<In, W>& t) {
+        t.hit = false;
+        if (base >= total) return;      // uniform
+        const SliceBuf sb(p.in + static_cast<i64>(slice) * p.is_b, p.slice_bytes);
+        const u32 pos = base + static_cast<u32>(lane);
+        const bool real = pos < total;
+        const u32 e = cand[real ? pos : 0u];
+        float iz = f0zf + static_cast<float>(e >> 7);           // WX * WY = 128 voxels per z
+        float iy = f0yf + static_cast<float>((e >> 4) & 7u);
+        float ix = f0xf + static_cast<float>(e & 15u);
+        if constexpr (!POW2) {
+            iz = divide_index(iz, nf, inv_n);
+            iy = divide_index(iy, nf, inv_n);
+            ix = divide_index(ix, nf, inv_n);
+        }
+        // noa's grid2slice (FourierProject.hpp:71-95).
+        const float pz = (R[0] * iz + R[1] * iy) + R[2] * ix;
+        float py = (R[3] * iz + R[4] * iy) + R[5] * ix;
+        float px = (R[6] * iz + R[7] * iy) + R[8] * ix;
+        if constexpr (!POW2) {
+            py *= nf;
+            px *= nf;
+        }
+        t.hit = real && fabsf(pz) <= fbT;
+        float wv;
+        if constexpr (EXACT) {
+            wv = window_poly(pz, inv_fb, wa);
+        } else {
+            const float tt = fmaf(pz * pz, tk, -1.f);
+            wv = wa[SLAB_NWIN];
+#pragma unroll
+            for (i32 k = SLAB_NWIN - 1; k >= 0; --k) wv = fmaf(wv, tt, wa[k]);
+        }
+        // Early flip of LINEAR spectrum interpolation (Interpolation.hpp:459-463).
+        const bool flip = px < 0.f;
+        py = flip ? -py : py;
+        px = fabsf(px);
+        const float fy = floorf(py), fx = floorf(px);
+        const float ty = py - fy, tx = px - fx;
+        const i32 y0 = static_cast<i32>(fy), x0 = static_cast<i32>(fx);
+        t.lv = e | (flip ? SLAB_FLIP : 0u);
+        const i32 row0 = y0 + (y0 < 0 ? wrap_neg : wrap_pos), row1 = y0 + 1 + (y0 + 1 < 0 ? wrap_neg : wrap_pos);
+        // Element offsets of the two tap rows (24-bit products: rows and pitch are below 2^24), then byte
+        // offsets; the x + 1 taps use the loads' immediate offset.
+        u32 e0 = __umul24(static_cast<u32>(row0), static_cast<u32>(pitch)) + static_cast<u32>(x0);
+        u32 e1 = __umul24(static_cast<u32>(row1), static_cast<u32>(pitch)) + static_cast<u32>(x0);
+        if (edge) {                     // uniform
+            // Bounds of the rfft slice (Frequency.hpp:258-288): y in [-(n/2), (n-1)/2], x in [0, n/2].
+            if (x0 > half || static_cast<u32>(y0 + half) >= static_cast<u32>(n)) e0 = SLAB_OUTSIDE;
+            if (x0 > half || static_cast<u32>(y0 + 1 + half) >= static_cast<u32>(n)) e1 = SLAB_OUTSIDE;
+            if (x0 >= half) t.lv |= SLAB_EDGE;
+        }
+        // PAIRED lets the compiler merge the two x taps of a row into one load; otherwise the second offset
+        // is hidden from it and each tap is its own load.
+        const u32 b0 = e0 * static_cast<u32>(sizeof(In)), b1 = e1 * static_cast<u32>(sizeof(In));
+        const u32 b0x = PAIRED ? b0 + static_cast<u32>(sizeof(In)) : pin(b0 + static_cast<u32>(sizeof(In)));
+        const u32 b1x = PAIRED ? b1 + static_cast<u32>(sizeof(In)) : pin(b1 + static_cast<u32>(sizeof(In)));
+        t.v00 = sb.template load_bytes<In>(b0);
+        t.v01 = sb.template load_bytes<In>(b0x);
+        t.v10 = sb.template load_bytes<In>(b1);
+        t.v11 = sb.template load_bytes<In>(b1x);
+        if constexpr (HASW) {
+            const SliceBuf wb(p.win + static_cast<i64>(slice) * p.wis_b, p.wslice_bytes);
+            const u32 d0 = e0 * 4u, d1 = e1 * 4u;
+            const u32 d0x = PAIRED ? d0 + 4u : pin(d0 + 4u), d1x = PAIRED ? d1 + 4u : pin(d1 + 4u);
+            t.q00 = wb.template load_bytes<W>(d0);
+            t.q01 = wb.template load_bytes<W>(d0x);
+            t.q10 = wb.template load_bytes<W>(d1);
+            t.q11 = wb.template load_bytes<W>(d1x);
+        }
+        if constexpr (EXACT) {
+            t.w00 = ty;
+            t.w01 = tx;
+            t.win = wv;
+        } else {
+            const float a0 = (1.f - ty) * wv, a1 = ty * wv, bx0 = 1.f - tx;
+            t.w00 = a0 * bx0;
+            t.w01 = a0 * tx;
+            t.w10 = a1 * bx0;
+            t.w11 = a1 * tx;
+            if constexpr (!HASW) t.win = wv;
         }
     };
-    // Cross-pair pipeline: the taps of the last pair whose sums are not added yet.
-    SlabTaps<In, W> pend[2];
-    bool have = false;
-    i32 pass = 0;          // pass of the current slice (more than one only for rows that are not unit vectors)
-
-    while (true) {
-        while (mask == 0) {
-            chunk0 += 64;
-            if (chunk0 >= item.z) break;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) cur[q] = nxt[q];
-            load_rec(chunk0 + 64 + lane, nxt);
-            mask = scan();
-        }
-        if (mask == 0) break;
-        const i32 k = __ffsll(static_cast<long long>(mask)) - 1;
-        mask &= mask - 1;
-        const i32 s = chunk0 + k;
-        // The slice's record, broadcast from the lane that scanned it.
-        const float R00 = bcast(cur[0].x, k), R01 = bcast(cur[0].y, k), R02 = bcast(cur[0].z, k);
-        const float R10 = bcast(cur[1].x, k), R11 = bcast(cur[1].y, k), R12 = bcast(cur[1].z, k);
-        const float R20 = bcast(cur[2].x, k), R21 = bcast(cur[2].y, k), R22 = bcast(cur[2].z, k);
-        const float ub = bcast(cur[1].w, k), uc = bcast(cur[2].w, k), hw = bcast(cur[3].x, k);
-        const i32 ax = __builtin_amdgcn_readlane(__float_as_int(cur[3].y), k);
-        // Rotations pack a slice's candidates in one pass (at most 4 per column). Rows that are not unit vectors
-        // thicken the slab: such a slice takes one pass per 4 ranks (a voxel is a candidate at most once per slice,
-        // so the passes add distinct voxels); its bit of the mask is set again until the last pass.
-        const i32 passes = __builtin_amdgcn_readlane(__float_as_int(cur[3].z), k);
-        const i32 j0 = 4 * pass, jn = passes > 1 ? 4 : 16;
-        if (passes > 1) {
-            if (++pass < passes) mask |= 1ull << k;
-            else pass = 0;
-        }
-
-        __syncthreads();   // the previous pair's candidate reads are done before the list is rewritten
-        u32 total;
-        if (ax == 0) {
-            const float u0 = fmaf(ub, static_cast<float>(f0[1]), fmaf(uc, static_cast<float>(f0[2]), -f0zf));
-            total = slab_candidates<0, 2>(cand, c0, u0, ub, uc, hw, j0, jn);
-        } else if (ax == 1) {
-            const float u0 = fmaf(ub, static_cast<float>(f0[0]), fmaf(uc, static_cast<float>(f0[2]), -f0yf));
-            total = slab_candidates<1, 2>(cand, c1, u0, ub, uc, hw, j0, jn);
-        } else {
-            const float u0 = fmaf(ub, static_cast<float>(f0[0]), fmaf(uc, static_cast<float>(f0[1]), -f0xf));
-            total = slab_candidates<2, 1>(cand, c2, u0, ub, uc, hw, j0, jn);
-        }
-        __syncthreads();
-
-        const SliceBuf sb(p.in + static_cast<i64>(s) * p.is_b, p.slice_bytes);
-        const SliceBuf wb(p.win ? static_cast<const void*>(p.win + static_cast<i64>(s) * p.wis_b)
-                                : static_cast<const void*>(p.in), p.win ? p.wslice_bytes : 0u);
-        // Phase 1 of candidates [base, base + 128): coordinates, window, and every tap load issued.
-        auto issue = [&](u32 base, SlabTaps<In, W> (&t)[2]) {
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                t[g].hit = false;
-                if (base + 64u * g >= total) continue;            // uniform
-                const u32 pos = base + 64u * g + static_cast<u32>(lane);
-                const bool real = pos < total;
-                const u32 e = cand[real ? pos : 0u];
-                const float iz = f0zf + static_cast<float>(e >> 7);           // WX * WY = 128 voxels per z
-                const float iy = f0yf + static_cast<float>((e >> 4) & 7u);
-                const float ix = f0xf + static_cast<float>(e & 15u);
-                t[g].lv = e;
-                // noa's grid2slice in samples (FourierProject.hpp:71-95 with R * (index / n) * n == R * index).
-                const float pz = (R00 * iz + R01 * iy) + R02 * ix;
-                float py = (R10 * iz + R11 * iy) + R12 * ix;
-                float px = (R20 * iz + R21 * iy) + R22 * ix;
-                t[g].hit = real && fabsf(pz) <= fbT;
-                const float u = pz * pz;
-                const float tt = fmaf(u, tk, -1.f);
-                float wv = wa9;
-                wv = fmaf(wv, tt, wa8); wv = fmaf(wv, tt, wa7); wv = fmaf(wv, tt, wa6); wv = fmaf(wv, tt, wa5);
-                wv = fmaf(wv, tt, wa4); wv = fmaf(wv, tt, wa3); wv = fmaf(wv, tt, wa2); wv = fmaf(wv, tt, wa1);
-                wv = fmaf(wv, tt, wa0);
-                t[g].win = wv;
-                // Early flip of LINEAR spectrum interpolation (Interpolation.hpp:459-463).
-                t[g].flip = px < 0.f;
-                py = t[g].flip ? -py : py;
-                px = fabsf(px);
-                const float fy = floorf(py), fx = floorf(px);
-                t[g].ty = py - fy;
-                t[g].tx = px - fx;
-                const i32 y0 = static_cast<i32>(fy), x0 = static_cast<i32>(fx);
-                // Bounds of the rfft slice (Frequency.hpp:258-288): y in [-n/2, n/2 - 1], x in [0, n/2].
-                t[g].oky0 = static_cast<u32>(y0 + half) < static_cast<u32>(n);
-                t[g].oky1 = static_cast<u32>(y0 + half) < static_cast<u32>(n - 1);
-                t[g].okx1 = x0 < half;
-                const i32 row0 = SC ? y0 + half : (y0 & (n - 1));
-                const i32 row1 = SC ? row0 + 1 : ((y0 + 1) & (n - 1));
-                // Element offsets of the two tap rows (24-bit products: rows and pitch are below 2^24), then byte
-                // offsets; the x + 1 taps use the loads' immediate offset.
-                const u32 e0 = __umul24(static_cast<u32>(row0), static_cast<u32>(pitch)) + static_cast<u32>(x0);
-                const u32 e1 = __umul24(static_cast<u32>(row1), static_cast<u32>(pitch)) + static_cast<u32>(x0);
-                // PAIRED lets the compiler merge the two x taps of a row into one load; otherwise the second offset
-                // is hidden from it and each tap is its own load.
-                const u32 b0 = e0 * static_cast<u32>(sizeof(In)), b1 = e1 * static_cast<u32>(sizeof(In));
-                const u32 b0x = PAIRED ? b0 + static_cast<u32>(sizeof(In)) : pin(b0 + static_cast<u32>(sizeof(In)));
-                const u32 b1x = PAIRED ? b1 + static_cast<u32>(sizeof(In)) : pin(b1 + static_cast<u32>(sizeof(In)));
-                t[g].v00 = sb.template load_bytes<In>(b0);
-                t[g].v01 = sb.template load_bytes<In>(b0x);
-                t[g].v10 = sb.template load_bytes<In>(b1);
-                t[g].v11 = sb.template load_bytes<In>(b1x);
-                if (p.win) {
-                    const u32 c0 = e0 * 4u, c1 = e1 * 4u;
-                    const u32 c0x = PAIRED ? c0 + 4u : pin(c0 + 4u), c1x = PAIRED ? c1 + 4u : pin(c1 + 4u);
-                    t[g].q00 = wb.template load_bytes<W>(c0);
-                    t[g].q01 = wb.template load_bytes<W>(c0x);
-                    t[g].q10 = wb.template load_bytes<W>(c1);
-                    t[g].q11 = wb.template load_bytes<W>(c1x);
-                }
+    // Interpolation and accumulation of a group.
+    auto finish = [&](SlabTaps<In, W>& t, bool at_edge) {
+        if (!t.hit) return;
+        if (at_edge) {                  // uniform
+            // Past the last stored column: what follows it in memory is no tap.
+            if (t.lv & SLAB_EDGE) {
+                t.v01 = t.v11 = vzero<In>();
+                if constexpr (HASW) t.q01 = t.q11 = W(0);
             }
-        };
-        SlabTaps<In, W> now[2];
-        issue(0u, now);
-        // The previous pair's sums are added while this pair's loads are in flight; per voxel, slices still add in
-        // order.
-        if (have) finish(pend);
-        if (total > 128u) {
-            finish(now);
+        }
+        const u32 at = t.lv & 1023u;
+        float re, im = 0.f, wt;
+        if constexpr (EXACT) {
+            // combine_taps: noa's order, x innermost, then y, then the flip and the window.
+            const float ty = t.w00, tx = t.w01, sx = 1 - tx, sy = 1 - ty;
+            auto mix = [&](float a, float b, float c, float d) { return (a * sx + b * tx) * sy + (c * sx + d * tx) * ty; };
+            if constexpr (CX) {
+                re = mix(t.v00.x, t.v01.x, t.v10.x, t.v11.x);
+                im = mix(t.v00.y, t.v01.y, t.v10.y, t.v11.y);
+            } else {
+                re = mix(t.v00, t.v01, t.v10, t.v11);
+            }
+            re *= t.win;
+            im *= t.win;
+            if constexpr (HASW) wt = mix(t.q00, t.q01, t.q10, t.q11) * t.win;
+            else wt = t.win;
+        } else {
+            if constexpr (CX) {
+                re = fmaf(t.w11, t.v11.x, fmaf(t.w10, t.v10.x, fmaf(t.w01, t.v01.x, t.w00 * t.v00.x)));
+                im = fmaf(t.w11, t.v11.y, fmaf(t.w10, t.v10.y, fmaf(t.w01, t.v01.y, t.w00 * t.v00.y)));
+            } else {
+                re = fmaf(t.w11, t.v11, fmaf(t.w10, t.v10, fmaf(t.w01, t.v01, t.w00 * t.v00)));
+            }
+            if constexpr (HASW) wt = fmaf(t.w11, t.q11, fmaf(t.w10, t.q10, fmaf(t.w01, t.q01, t.w00 * t.q00)));
+            else wt = t.win;
+        }
+        if constexpr (CX) im = __uint_as_float(__float_as_uint(im) ^ (t.lv & SLAB_FLIP));
+        acc[at] += re;
+        if constexpr (CX) acc[WVOX + at] += im;
+        acc[(NCH - 1) * WVOX + at] += wt;
+    };
+
+    // Two pairs in turn: the loads of one are in flight while the sums of the other are added. At the end, an empty
+    // pair pushes the last one through.
+    SlabTaps<In, W> taps[2][2];
+    bool edges[2] = {false, false};
+#pragma unroll
+    for (i32 d = 0; d < 4; ++d) taps[d >> 1][d & 1].hit = false;
+    for (bool more = true; more;) {
+#pragma unroll
+        for (i32 d = 0; d < 2; ++d) {
+            total = 0;
+            more = more && advance();
+            edges[d] = edge;
+            issue(0, taps[d][0]);
+            issue(64, taps[d][1]);
+            finish(taps[1 - d][0], edges[1 - d]);
+            finish(taps[1 - d][1], edges[1 - d]);
+            taps[1 - d][0].hit = taps[1 - d][1].hit = false;
             for (u32 base = 128; base < total; base += 128) {
-                issue(base, now);
-                finish(now);
+                finish(taps[d][0], edge);
+                finish(taps[d][1], edge);
+                issue(base, taps[d][0]);
+                issue(base + 64, taps[d][1]);
             }
-            have = false;
-        } else {
-#pragma unroll
-            for (int g = 0; g < 2; ++g) pend[g] = now[g];
-            have = true;
         }
     }
-    if (have) finish(pend);
-    __syncthreads();
+    wave_lds_order();
 
     if (item.w >= 0) {
         // Split sub-brick: this segment's sums, in the layout of insert_reduce_kernel's partial slots.
@@ -1065,10 +1106,15 @@ __global__ __launch_bounds__(64) void insert_slab_kernel(const SlabParams<In, W>
     // Sums of the voxels inside the stored volume and the cutoff are added to the volume (:516-518).
     for (i32 v = lane; v < WVOX; v += 64) {
         const i32 lz = v / (WY * WX), ly = (v / WX) % WY, lx = v % WX;
-        if (lx >= nin[2]) continue;
-        const float iz = f0zf + static_cast<float>(lz), iy = f0yf + static_cast<float>(ly), ix = f0xf + static_cast<float>(lx);
-        if ((iz * iz + iy * iy) + ix * ix > p.cut2) continue;
-        const i32 z = org[0] + lz, y = org[1] + ly, x = org[2] + lx;
+        if (lz >= nin[0] || ly >= nin[1] || lx >= nin[2]) continue;
+        vec3<float> f;
+        f.z = f0zf + static_cast<float>(lz); f.y = f0yf + static_cast<float>(ly); f.x = f0xf + static_cast<float>(lx);
+        if constexpr (!POW2) {
+            f.z /= nf; f.y /= nf; f.x /= nf;
+        }
+        if (dot3(f) > (POW2 ? p.cut2 : p.cutoff_sqd)) continue;
+        const i32 z = frequency2index(p.vol_centered, f0[0] + lz, n), y = frequency2index(p.vol_centered, f0[1] + ly, n);
+        const i32 x = org[2] + lx;
         In sum;
         if constexpr (CX) sum = make_float2(acc[v], acc[WVOX + v]);
         else sum = acc[v];
@@ -1077,6 +1123,76 @@ __global__ __launch_bounds__(64) void insert_slab_kernel(const SlabParams<In, W>
         if (p.wvol) {
             W* w = p.wvol + (z * p.wvs0 + y * p.wvs1 + x * p.wvs2);
             *w = *w + acc[(NCH - 1) * WVOX + v];
+        }
+    }
+}
+
+template<class In, class Out, class W, bool HASW, bool POW2, bool PAIRED>
+__global__ __launch_bounds__(64, SLAB_WAVES) void insert_slab_kernel(const SlabParams<In, W> p) {
+    __shared__ float acc[(vt<In>::cx ? 3 : 2) * WVOX];
+    __shared__ unsigned short cand[SLAB_MAXC];
+    const int4 item = p.items[blockIdx.x];
+    if (item.x < 0) return;                 // padding of an XCD-ordered plan
+    insert_slab_item<In, Out, W, HASW, POW2, PAIRED>(p, item, acc, cand);
+}
+
+// Batched insertion: several insertion calls (each its own volume, box size, layout, slice count and cutoff) in one
+// persistent launch. The device image of a batch holds a header, one parameter block per call and the work items of
+// every call ({sub-brick, first slice, end slice, call}; the calls' slice ranges are not split, so no partial sums);
+// workgroup g takes the items g, g + G, ... (items of each call sorted by expected work, calls interleaved by the
+// host). A call of the slab kernel's configuration runs its enumeration and pipeline with the one-wave kernel's
+// arithmetic (EXACT), any other call the one-wave kernel's code: the results are those of unsplit one-wave calls made one
+// by one, bit for bit.
+struct InsertBatchHeader {
+    i32 n_items, n_jobs;
+    i32 jobs_offset, items_offset;       // bytes from the start of the image
+    i32 pad[12];
+};
+static_assert(sizeof(InsertBatchHeader) == 64, "batch header");
+
+struct InsertBatchJob {
+    enum Kind : i32 { WAVE, SLAB, SLAB_NO_WEIGHTS };
+    InsertParams<float, float2, float> wave;
+    SlabParams<float2, float> slab;
+    i32 kind;
+};
+
+// A parameter block at a wave-uniform address, read through the scalar cache (the image does not change while a batch
+// runs) into scalar registers.
+template<class T> __device__ __forceinline__ T load_uniform(const T* at) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    using Words = const u32 __attribute__((address_space(4)));
+    Words* src = (Words*)(reinterpret_cast<uintptr_t>(at));
+    u32 words[sizeof(T) / 4];
+#pragma unroll
+    for (u32 i = 0; i < sizeof(T) / 4; ++i) words[i] = src[i];
+    T out;
+    __builtin_memcpy(&out, words, sizeof(T));
+    return out;
+}
+
+__global__ __launch_bounds__(64, SLAB_WAVES) void insert_batch_kernel(const unsigned char* __restrict__ image) {
+    __shared__ float2 acc_v[WVOX + WVOX / 2];          // values and weights (one-wave items), or the slab's channels
+    __shared__ i32 cand[SLAB_MAXC / 2];
+    const InsertBatchHeader* h = reinterpret_cast<const InsertBatchHeader*>(image);
+    const InsertBatchJob* __restrict__ jobs = reinterpret_cast<const InsertBatchJob*>(image + h->jobs_offset);
+    const int4* __restrict__ items = reinterpret_cast<const int4*>(image + h->items_offset);
+    const i32 n_items = h->n_items;
+    float* acc = reinterpret_cast<float*>(acc_v);
+    for (i32 i = static_cast<i32>(blockIdx.x); i < n_items; i += static_cast<i32>(gridDim.x)) {
+        int4 item = items[i];
+        const InsertBatchJob* job = jobs + __builtin_amdgcn_readfirstlane(item.w);
+        item.w = -1;
+        __syncthreads();   // the previous item's flush has read the accumulator
+        const i32 kind = __builtin_amdgcn_readfirstlane(job->kind);
+        if (kind == InsertBatchJob::SLAB) {
+            const SlabParams<float2, float> p = load_uniform(&job->slab);
+            insert_slab_item<float2, float2, float, true, false, true>(p, item, acc, reinterpret_cast<unsigned short*>(cand));
+        } else if (kind == InsertBatchJob::SLAB_NO_WEIGHTS) {
+            const SlabParams<float2, float> p = load_uniform(&job->slab);
+            insert_slab_item<float2, float2, float, false, false, true>(p, item, acc, reinterpret_cast<unsigned short*>(cand));
+        } else {
+            insert_wave_item<float, float2, float2, float, NOA_HIP_INTERP_LINEAR, 0>(job->wave, item, acc_v, acc + 2 * WVOX, cand);
         }
     }
 }
@@ -1569,8 +1685,8 @@ struct KernelChoice {
     bool paired;          // slab kernel: one 16-byte (8-byte) load for the two x taps of a slice (weight) row
     int order;            // order of the work items (make_plan)
     double list_target;   // expected passing slices per work item; 0: the kernel's default
-    i32 max_span;         // most slices per work item (0: no bound; not for the allocation-free entry point or the
-                          // pose-adaptive order, whose segments come from the counts)
+    i32 max_span;         // most slices per work item (0: no bound, -1: default_span; not for the allocation-free entry
+                          // point or the pose-adaptive order, whose segments come from the counts)
 };
 KernelChoice kernel_choice(const ProjectDesc& d) {
     KernelChoice k{};
@@ -1590,13 +1706,17 @@ KernelChoice kernel_choice(const ProjectDesc& d) {
     }
     if (const char* pr = std::getenv("NOA_HIP_INSERT_PAIRED")) k.paired = std::string(pr) != "0";
     if (const char* l = std::getenv("NOA_HIP_INSERT_LIST")) k.list_target = std::max(16.0, std::atof(l));
-    // At most 1,024 slices per work item: a sub-brick crossed by many more slices than the uniform model expects
-    // (a tilt series: 13.4 -> 6.1 ms at 256^3 with 10,000 slices) still gets several items, for uniform poses within
-    // the noise (more partial sums, 591 against 140 MiB at 10,000 slices).
-    k.max_span = 1024;
+    k.max_span = -1;
     if (const char* sp = std::getenv("NOA_HIP_INSERT_SPAN")) k.max_span = std::max(0, std::atoi(sp));
     return k;
 }
+
+// Most slices of the range per work item: a sub-brick crossed by many more slices than the uniform model expects (a tilt
+// series) still gets several items. A quarter of the slices, between 256 and 1,024: fewer cost uniform poses partial sums
+// (1,000 slices of 256^2: 0.62 ms, 0.71 ms with a bound of 128, which takes a tilt series from 2.5 to 1.0 ms); 2,000
+// slices of 200^2, uniform and tilt series, with bounds of 128 0.73 and 0.97 ms, 256 0.60 and 1.09 ms, 512 0.57 and 1.75
+// ms, 1,024 0.60 and 3.05 ms; 10,000 of 256^2 4.60 ms with 1,024, 4.87 with 512.
+i32 default_span(i32 n_slices) { return std::clamp(n_slices / 4, 256, 1024); }
 
 // Window of the slab kernel: windowed_sinc(pz / n, fs, fb) (FourierProject.hpp:99-110) as a polynomial of degree
 // SLAB_NWIN in t = 2 (pz / fbT)^2 - 1, pz in samples (fbT = fb * n): Chebyshev interpolation at the Chebyshev nodes,
@@ -1742,6 +1862,57 @@ bool fill_params(const ProjectDesc& d, InsertParams<C, In, W>& p) {
     return buffers_ok;
 }
 
+// The slab kernel's parameters of one call (but the work plan and the partial sums), from those of the one-wave kernel;
+// false where it does not apply. `exact`: the arithmetic of sizes that are not a power of two, whatever the size. It takes
+// Mat33<f32> rotations (or, with a power of two, Quaternion<f32> through their matrix: the coordinates are noa's
+// quaternion rotation up to rounding, within the insertion's tolerance), LINEAR, one size 32 <= n < 4096 for the slices, the volume and the target, cutoff <= 0.5, a
+// window of at most ~1.15 samples (at most 4 candidates per column) that the polynomial fits, unit x strides and one row
+// pitch for the slices and their weights.
+template<class In, class W>
+bool fill_slab(const ProjectDesc& d, const InsertParams<float, In, W>& p, bool exact, SlabParams<In, W>& sp) {
+    const i64 nn = d.target[0];
+    const bool cubic = d.target[1] == nn && d.target[2] == nn && p.grid[0] == nn && p.grid[1] == nn && p.grid[2] == nn &&
+                       p.slice_shape[0] == nn && p.slice_shape[1] == nn;
+    const bool pow2 = !exact && (nn & (nn - 1)) == 0;
+    const bool rot_ok = p.rot.kind == NOA_HIP_MAT33_F32 || (pow2 && p.rot.kind == NOA_HIP_QUAT_F32);
+    const float cutoff = std::max(static_cast<float>(d.cutoff), 0.f);
+    if (p.general || d.interp != NOA_HIP_INTERP_LINEAR || !cubic || nn < 32 || nn >= 4096 || !rot_ok || cutoff > 0.5f ||
+        p.in_is_value || p.win_is_value || p.is_x != 1 || p.is_y < 0 || p.is_y >= (1 << 24) ||
+        (p.win_present && (p.wis_x != 1 || p.wis_y != p.is_y)) || p.slice_bytes > SLAB_MAX_BYTES || p.slice_bytes == 0 ||
+        p.wslice_bytes > SLAB_MAX_BYTES)
+        return false;
+    const float n = static_cast<float>(nn);
+    SlabWindow sw{};
+    if (pow2) sw = fit_slab_window(p.fftfreq_sinc, p.fftfreq_blackman, static_cast<i32>(nn));
+    sp = SlabParams<In, W>{};
+    sp.reach = p.fftfreq_blackman * n;
+    if (sp.reach > 1.15f || !(pow2 ? sw.ok : p.wpoly)) return false;
+    sp.in = p.in; sp.is_b = p.is_b;
+    sp.win = p.win_present ? p.win : nullptr; sp.wis_b = p.wis_b;
+    sp.pitch = p.is_y;
+    sp.slice_bytes = p.slice_bytes; sp.wslice_bytes = p.wslice_bytes;
+    sp.vol = p.vol; sp.vs0 = p.vs0; sp.vs1 = p.vs1; sp.vs2 = p.vs2;
+    sp.wvol = p.has_wvol ? p.wvol : nullptr; sp.wvs0 = p.wvs0; sp.wvs1 = p.wvs1; sp.wvs2 = p.wvs2;
+    sp.n = p.grid[0];
+    for (int i = 0; i < 3; ++i) sp.nb[i] = p.nb[i];
+    sp.rot = p.rot;
+    sp.n_slices = p.n_slices;
+    // The exact test's pz carries at most four roundings of 2^-24 n (with those of the range's centre, below 1e-6 n
+    // samples along A).
+    sp.margin = 1e-3f + 2e-6f * n;
+    sp.fbT = pow2 ? sw.fbT : p.fftfreq_blackman;
+    sp.tk = sw.tk;
+    for (int k = 0; k <= NWIN; ++k) sp.wa[k] = !pow2 ? p.wa[k] : (k <= SLAB_NWIN ? sw.a[k] : 0.f);
+    sp.inv_fb = p.inv_fb;
+    sp.inv_n = 1.f / n;
+    sp.cutoff_sqd = p.cutoff_sqd;
+    sp.cut2 = p.cutoff_sqd * n * n;
+    sp.cut2_columns = pow2 ? sp.cut2 : sp.cut2 * (1.f + 2e-6f);
+    sp.vol_centered = p.vol_centered;
+    sp.slice_centered = p.slices_centered;
+    return true;
+}
+
 template<class C, class In, class Out, class W>
 int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratch* scratch) {
     InsertParams<C, In, W> p;
@@ -1766,25 +1937,12 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
             i32 step = 8;
             while (p.n_slices > 16 * step) step *= 2;
             const i32 plan_slices = std::max<i32>(64, (p.n_slices + step - 1) / step * step);
-            // The slab kernel: Mat33<f32> rotations (or Quaternion<f32>, through their matrix: the coordinates are
-            // noa's quaternion rotation up to rounding, within the insertion's tolerance), LINEAR, one power-of-two size n >= 32 for the slices, the
-            // volume and the target, cutoff <= 0.5, a window of at most ~1.15 samples (at most 4 candidates per column)
-            // that the degree-9 polynomial fits, unit x strides and one row pitch for the slices and their weights.
             bool slab = false;
-            SlabWindow sw{};
+            SlabParams<In, W> sp{};
             if constexpr (std::is_same_v<C, float>) {
-                const i64 nn = d.target[0];
-                const bool cubic = d.target[1] == nn && d.target[2] == nn && p.grid[0] == nn && p.grid[1] == nn &&
-                                   p.grid[2] == nn && p.slice_shape[0] == nn && p.slice_shape[1] == nn;
-                if (!kc.force_wave && !p.general && d.interp == NOA_HIP_INTERP_LINEAR && cubic && p.pow2 && nn >= 32 &&
-                    (p.rot.kind == NOA_HIP_MAT33_F32 || p.rot.kind == NOA_HIP_QUAT_F32) && cutoff <= C(0.5) && p.is_x == 1 &&
-                    (!p.win_present || (p.wis_x == 1 && p.wis_y == p.is_y)) && p.slice_bytes < 0x7ffffff0u &&
-                    p.wslice_bytes < 0x7ffffff0u) {
-                    sw = fit_slab_window(static_cast<float>(p.fftfreq_sinc), static_cast<float>(p.fftfreq_blackman),
-                                         static_cast<i32>(nn));
-                    slab = sw.ok && sw.fbT <= 1.15f;
-                }
+                slab = !kc.force_wave && fill_slab(d, p, false, sp);
             }
+            p.freq_order = slab;
             // Expected passing slices per work item: the table's value, else 512 for the slab kernel (12 resident
             // waves per CU: 4.6-4.7 ms against 5.0 ms at 256 for 10,000 slices at 256^3) and 256 for the one-wave
             // kernel.
@@ -1792,10 +1950,12 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
             // value, whose partial sums fit its scratch.
             const double cap = slab ? 512.0 : 256.0;
             const double list_target = kc.list_target > 0 ? kc.list_target : (scratch == nullptr ? -cap : cap);
-            const int st = make_plan(device, p.grid, d.target, static_cast<double>(cutoff), p.vol_centered,
+            const int st = make_plan(device, p.grid, d.target, static_cast<double>(cutoff), slab || p.vol_centered,
                                      plan_slices, static_cast<double>(p.fftfreq_blackman), p.bd, list_target,
                                      scratch == nullptr, planp, err, kc.order,
-                                     scratch == nullptr && kc.order != 3 ? kc.max_span : 0);
+                                     scratch != nullptr || kc.order == 3 ? 0
+                                     : kc.max_span >= 0                  ? kc.max_span
+                                                                         : default_span(plan_slices));
             if (st != NOA_HIP_OK) return st;
             // Pose-adaptive plan (item order 3; not for the allocation-free entry point): the passing slices of each
             // active sub-brick are counted on the device, and the segments are cut from the counts.
@@ -1837,7 +1997,7 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                     cp.target[a] = p.target[a];
                 }
                 cp.fb = p.fftfreq_blackman;
-                cp.vol_centered = p.vol_centered;
+                cp.vol_centered = slab || p.vol_centered;
                 hipLaunchKernelGGL((insert_count_kernel<C>),
                                    dim3(static_cast<u32>((nbk + CNT_BRICKS - 1) / CNT_BRICKS),
                                         static_cast<u32>((p.n_slices + cp.range_w - 1) / cp.range_w)),
@@ -1885,11 +2045,11 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
             if (plan.n_items == 0) return NOA_HIP_OK;
             const size_t partial_bytes = static_cast<size_t>(plan.n_partials) * p.bd[0] * p.bd[1] * p.apitch * 3 *
                                          sizeof(float);
-            const size_t record_bytes = static_cast<size_t>(p.n_slices) * 4 * sizeof(float4);
+            // The allocation-free entry point's limit counts 64 bytes per slice beside the plan and the partial sums.
+            const size_t record_bytes = static_cast<size_t>(p.n_slices) * 64;
             void* partials = nullptr;
-            void* records = nullptr;     // slab kernel only
             if (scratch) {
-                // Allocation-free: plan, records and partial sums in the caller-independent scratch, in that order.
+                // Allocation-free: plan and partial sums in the caller-independent scratch, in that order.
                 auto round = [](size_t b) { return (b + 255) & ~static_cast<size_t>(255); };
                 const size_t items_bytes = round(plan.h_items.size() * sizeof(int4));
                 const size_t reduce_bytes = round(plan.h_reduce.size() * sizeof(int4));
@@ -1905,8 +2065,6 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                 at += items_bytes;
                 int4* reduce = plan.h_reduce.empty() ? nullptr : reinterpret_cast<int4*>(at);
                 at += reduce_bytes;
-                records = at;
-                at += round(record_bytes);
                 partials = plan.n_partials > 0 ? at : nullptr;
                 p.items = items;
                 p.reduce = reduce;
@@ -1934,43 +2092,18 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                                   p.is_y == p.wis_y && p.slice_bytes < 0x7ffffff0u && p.wslice_bytes < 0x7ffffff0u;
             const int hot = hot_opts ? (p.vol_centered ? 2 : 1) : 0;
             if (slab) {
-                if (!scratch && hipMallocAsync(&records, record_bytes, stream) != hipSuccess) {
-                    if (partials) (void)hipFreeAsync(partials, stream);
-                    err = "insert: could not allocate the slice records";
-                    return NOA_HIP_ERROR_RUNTIME;
-                }
                 if constexpr (std::is_same_v<C, float>) {
-                    hipLaunchKernelGGL(slab_records_kernel, dim3(static_cast<unsigned>((p.n_slices + 255) / 256)),
-                                       dim3(256), 0, stream, p.rot, p.n_slices, sw.fbT, static_cast<float4*>(records));
-                    SlabParams<In, W> sp{};
-                    sp.in = p.in; sp.is_b = p.is_b;
-                    sp.win = p.win_present ? p.win : nullptr; sp.wis_b = p.wis_b;
-                    sp.pitch = p.is_y;
-                    sp.slice_bytes = p.slice_bytes; sp.wslice_bytes = p.wslice_bytes;
-                    sp.vol = p.vol; sp.vs0 = p.vs0; sp.vs1 = p.vs1; sp.vs2 = p.vs2;
-                    sp.wvol = p.has_wvol ? p.wvol : nullptr; sp.wvs0 = p.wvs0; sp.wvs1 = p.wvs1; sp.wvs2 = p.wvs2;
-                    sp.n = p.grid[0];
-                    for (int i = 0; i < 3; ++i) sp.nb[i] = p.nb[i];
                     sp.items = p.items;
                     sp.partials = p.partials;
-                    sp.rec = static_cast<const float4*>(records);
-                    sp.n_slices = p.n_slices;
-                    sp.fbT = sw.fbT;
-                    sp.tk = sw.tk;
-                    for (int k = 0; k <= SLAB_NWIN; ++k) sp.wa[k] = sw.a[k];
-                    sp.cut2 = static_cast<float>(p.cutoff_sqd) * static_cast<float>(p.grid[0]) * static_cast<float>(p.grid[0]);
-                    sp.vol_centered = p.vol_centered;
-                    if (kc.paired) {
-                        if (p.slices_centered)
-                            hipLaunchKernelGGL((insert_slab_kernel<In, Out, W, true, true>), grid_items, dim3(64), 0, stream, sp);
-                        else
-                            hipLaunchKernelGGL((insert_slab_kernel<In, Out, W, false, true>), grid_items, dim3(64), 0, stream, sp);
-                    } else {
-                        if (p.slices_centered)
-                            hipLaunchKernelGGL((insert_slab_kernel<In, Out, W, true, false>), grid_items, dim3(64), 0, stream, sp);
-                        else
-                            hipLaunchKernelGGL((insert_slab_kernel<In, Out, W, false, false>), grid_items, dim3(64), 0, stream, sp);
-                    }
+                    const bool pow2 = (p.grid[0] & (p.grid[0] - 1)) == 0;
+                    auto launch = [&](auto has_w) {
+                        constexpr bool HW = decltype(has_w)::value;
+                        if (!pow2) hipLaunchKernelGGL((insert_slab_kernel<In, Out, W, HW, false, true>), grid_items, dim3(64), 0, stream, sp);
+                        else if (kc.paired) hipLaunchKernelGGL((insert_slab_kernel<In, Out, W, HW, true, true>), grid_items, dim3(64), 0, stream, sp);
+                        else hipLaunchKernelGGL((insert_slab_kernel<In, Out, W, HW, true, false>), grid_items, dim3(64), 0, stream, sp);
+                    };
+                    if (sp.win) launch(std::true_type{});
+                    else launch(std::false_type{});
                 }
             } else {
                 if (nearest) {
@@ -1986,9 +2119,8 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
             if (plan.n_reduce > 0)
                 hipLaunchKernelGGL((insert_reduce_kernel<C, In, Out, W>), dim3(plan.n_reduce), dim3(NT_REDUCE), 0, stream, p);
             hipError_t e = hipGetLastError();
-            for (void* buf : {partials, records}) {
-                if (!buf || scratch) continue;
-                const hipError_t fe = hipFreeAsync(buf, stream);
+            if (partials && !scratch) {
+                const hipError_t fe = hipFreeAsync(partials, stream);
                 if (e == hipSuccess) e = fe;
             }
             if (e != hipSuccess) { err = std::string("kernel launch failed: ") + hipGetErrorString(e); return NOA_HIP_ERROR_RUNTIME; }
@@ -2055,8 +2187,9 @@ int scratch_address(int device, void*& ptr, std::string& err) {
 int insert_batch_prepare(const ProjectDesc* descs, i32 n_jobs, void* image, i64 capacity, i64& bytes,
                          std::string& err) {
     using P = InsertParams<float, float2, float>;
+    using Job = InsertBatchJob;
     auto round = [](i64 b) { return (b + 255) & ~static_cast<i64>(255); };
-    std::vector<P> params(static_cast<size_t>(n_jobs));
+    std::vector<Job> params(static_cast<size_t>(n_jobs));
     struct Item { float work; int4 item; };
     std::vector<Item> items;
     int device = 0;
@@ -2072,16 +2205,20 @@ int insert_batch_prepare(const ProjectDesc* descs, i32 n_jobs, void* image, i64 
                        "interpolation and single-precision transforms without scaling or Ewald sphere are batched";
             return NOA_HIP_ERROR_UNSUPPORTED;
         }
-        P& p = params[static_cast<size_t>(k)];
+        Job& job = params[static_cast<size_t>(k)];
+        std::memset(static_cast<void*>(&job), 0, sizeof(Job));
+        P& p = job.wave;
         if (!fill_params(d, p)) { err = at + "the slices exceed the 4 GiB of a buffer load"; return NOA_HIP_ERROR_UNSUPPORTED; }
         if (p.n_slices == 0) continue;
+        const bool slab = fill_slab(d, p, true, job.slab);
+        job.kind = !slab ? Job::WAVE : (job.slab.win ? Job::SLAB : Job::SLAB_NO_WEIGHTS);
         i32 step = 8;
         while (p.n_slices > 16 * step) step *= 2;
         const i32 plan_slices = std::max<i32>(64, (p.n_slices + step - 1) / step * step);
         const Plan* plan = nullptr;
         // One segment per sub-brick (no partial sums): list target above any slice count.
         const int st = make_plan(device, p.grid, d.target, static_cast<double>(std::max(static_cast<float>(d.cutoff), 0.f)),
-                                 p.vol_centered, plan_slices, static_cast<double>(p.fftfreq_blackman), p.bd, 1e30, false,
+                                 slab || p.vol_centered, plan_slices, static_cast<double>(p.fftfreq_blackman), p.bd, 1e30, false,
                                  plan, err);
         if (st != NOA_HIP_OK) return st;
         for (size_t i = 0; i < plan->h_items.size(); ++i) {
@@ -2093,7 +2230,7 @@ int insert_batch_prepare(const ProjectDesc* descs, i32 n_jobs, void* image, i64 
     // Largest expected work first, across the calls.
     std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& b) { return a.work > b.work; });
     const i64 jobs_offset = round(static_cast<i64>(sizeof(InsertBatchHeader)));
-    const i64 items_offset = round(jobs_offset + static_cast<i64>(sizeof(P)) * n_jobs);
+    const i64 items_offset = round(jobs_offset + static_cast<i64>(sizeof(Job)) * n_jobs);
     bytes = items_offset + static_cast<i64>(items.size()) * static_cast<i64>(sizeof(int4));
     if (!image || capacity < bytes) {
         err = "insert batch: the image needs " + std::to_string(bytes) + " bytes";
@@ -2108,7 +2245,7 @@ int insert_batch_prepare(const ProjectDesc* descs, i32 n_jobs, void* image, i64 
     h.jobs_offset = static_cast<i32>(jobs_offset);
     h.items_offset = static_cast<i32>(items_offset);
     std::memcpy(out, &h, sizeof(h));
-    if (n_jobs > 0) std::memcpy(out + jobs_offset, params.data(), sizeof(P) * static_cast<size_t>(n_jobs));
+    if (n_jobs > 0) std::memcpy(out + jobs_offset, params.data(), sizeof(Job) * static_cast<size_t>(n_jobs));
     int4* dst = reinterpret_cast<int4*>(out + items_offset);
     for (size_t i = 0; i < items.size(); ++i) dst[i] = items[i].item;
     return NOA_HIP_OK;

@@ -274,13 +274,6 @@ __global__ __launch_bounds__(RB_SCAN) void rasterize_items_kernel(const RasterBo
     for (i32 j = (seen + p.per_item - 1) / p.per_item + t; j < p.max_items; j += RB_SCAN) starts[j] = RB_DONE;
 }
 
-// i / n rounded to nearest, for integers |i| <= n < 2^12 with inv_n = 1 / n rounded: one Newton step on the product
-// (the remainder is exact), checked for every such pair on the CPU.
-__device__ __forceinline__ float divide_index(float i, float n, float inv_n) {
-    const float q = i * inv_n;
-    return fmaf(fmaf(-q, n, i), inv_n, q);
-}
-
 // GEN: quaternions or inverse scalings (noa's expressions at run time); otherwise Mat33 rotations.
 template<class In, class Out, bool GEN>
 __global__ __launch_bounds__(64) void rasterize_box_kernel(const RasterBoxParams<In, Out> p) {

@@ -160,3 +160,44 @@ def test_slab_adds_to_the_volume_and_leaves_voxels_beyond_the_cutoff():
     r = np.sqrt(fr[:, None, None] ** 2 + fr[None, :, None] ** 2 + (np.arange(n // 2 + 1) / n)[None, None, :] ** 2)
     outside = np.broadcast_to(r > 0.4 + 1e-6, got.shape)
     np.testing.assert_array_equal(got[outside], start[outside])
+
+
+@pytest.mark.parametrize("n,remap,sdt,odt,weights", [
+    (33, "h2h", np.complex64, np.complex64, True),        # the smallest odd size: a sub-brick across the wrap
+    (40, "hc2h", np.complex64, np.float32, False),        # n/2 not a multiple of a sub-brick
+    (47, "h2hc", np.float32, np.float32, True),
+    (64, "h2h", np.complex64, np.complex64, True),        # a power of two
+    (150, "hc2hc", np.complex64, np.complex64, True),
+])
+def test_slab_sizes_match_the_wave_kernel_with_nonfinite_pixels(monkeypatch, n, remap, sdt, odt, weights):
+    """Every size takes the slab kernel; with one item per sub-brick, sizes that are not a power of two give the one-wave
+    kernel's bits (same expressions, same order) and a power of two is within 1e-6 of it (another order and window
+    polynomial). A NaN and an infinity in a slice's first column and last row reach the same voxels: a tap past the
+    stored half or beyond the last row reads none of them."""
+    print(f"case slab sizes n={n} {remap}", flush=True)
+    monkeypatch.setenv("NOA_HIP_INSERT_LIST", "1000000000")
+    monkeypatch.setenv("NOA_HIP_INSERT_SPAN", "0")
+    rng = np.random.default_rng(500 + n)
+    b = 21
+    sl = random_spectrum((b, 1, n, n // 2 + 1), rng)
+    sl = (sl.real if sdt == np.float32 else sl).astype(sdt)
+    sl[3, 0, n // 3, 0] = np.nan
+    sl[5, 0, n // 2 + 1, 0] = np.inf
+    sl[7, 0, n - 1, n // 4] = np.nan
+    w = rng.uniform(0.1, 1.0, sl.shape).astype(np.float32) if weights else None
+    inv = np.ascontiguousarray(np.transpose(random_rotations(b, rng), (0, 2, 1)))
+    inv[2] = np.eye(3)                       # taps on the slice's last column
+    inv[8] *= 1.04                           # rows longer than unit vectors: taps beyond the slice
+    args = (remap, dev(sl), dev(w) if weights else None, (b, 1, n, n), n, dev(inv),
+            torch.complex64 if odt == np.complex64 else torch.float32)
+    got_v, got_w = run_gpu(*args)
+    monkeypatch.setenv("NOA_HIP_INSERT_KERNEL", "wave")
+    want_v, want_w = run_gpu(*args)
+    bad = ~np.isfinite(want_v)
+    assert bad.any() and np.isfinite(want_w).all()
+    np.testing.assert_array_equal(~np.isfinite(got_v), bad)
+    if n == 64:
+        assert rel_l2(got_v[~bad], want_v[~bad]) < 1e-6 and rel_l2(got_w, want_w) < 1e-6
+    else:
+        np.testing.assert_array_equal(got_v, want_v)
+        np.testing.assert_array_equal(got_w, want_w)
