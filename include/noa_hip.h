@@ -275,6 +275,10 @@ int noa_hip_insert_central_slices_3d_noalloc(const noa_hip_project_args* args, v
 /* Replaces the GPU branch of noa::xform::extract_central_slices_3d (FourierProject.hpp:1869-1914). */
 int noa_hip_extract_central_slices_3d(const noa_hip_project_args* args, void* stream);
 
+/* The calls keep their device workspaces (volume copies, partial sums, work items) for the next call, at most 1 GiB per
+ * GPU. Gives those that no call is using back (waiting for the work that used them); returns their bytes. */
+int64_t noa_hip_workspace_trim(int32_t device);
+
 /* ---- Batched calls (no counterpart in noa, whose only asynchrony is Stream::enqueue,
  * runtime/cuda/Stream.hpp:205-239) --------------------------------------------------------------------------------
  * Several extraction (or insertion) calls, each with its own arrays, box size, layout, slice count and cutoff, run

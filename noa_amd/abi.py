@@ -218,6 +218,8 @@ def declare(lib: ctypes.CDLL) -> ctypes.CDLL:
         f = getattr(lib, name)
         f.argtypes = [P, c_void_p]
         f.restype = ctypes.c_int
+    lib.noa_hip_workspace_trim.argtypes = [c_int32]
+    lib.noa_hip_workspace_trim.restype = c_int64
     lib.noa_hip_volume_blocks_bytes.argtypes = [ctypes.POINTER(c_int64)]
     lib.noa_hip_volume_blocks_bytes.restype = c_int64
     lib.noa_hip_volume_blocks.argtypes = [ctypes.POINTER(View), c_void_p, c_int64, c_void_p]

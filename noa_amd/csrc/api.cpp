@@ -19,6 +19,7 @@
 
 #include "../../include/noa_hip.h"
 #include "kernels.hpp"
+#include "workspace.hpp"
 
 namespace noa_hip {
 namespace {
@@ -1493,6 +1494,8 @@ int32_t noa_hip_fft_clear_cache(int32_t device) { return noa_hip::fft_clear_cach
 int32_t noa_hip_fft_set_cache_limit(int32_t count, int32_t device) { return noa_hip::fft_set_cache_limit(count, device); }
 int32_t noa_hip_fft_cache_limit(int32_t device) { return noa_hip::fft_cache_limit(device); }
 int32_t noa_hip_fft_cache_size(int32_t device) { return noa_hip::fft_cache_size(device); }
+int64_t noa_hip_workspace_trim(int32_t device) { return static_cast<int64_t>(noa_hip::workspace_trim(device)); }
+
 int64_t noa_hip_fft_workspace_left_to_allocate(int32_t device) {
     return noa_hip::fft_workspace_left_to_allocate(device);
 }

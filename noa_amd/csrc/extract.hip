@@ -19,6 +19,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "tiles.hpp"
+#include "workspace.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -789,13 +790,10 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err) {
             if (env && std::strcmp(env, "linear") == 0) bricks = false;
             if (env && std::strcmp(env, "bricks") == 0) bricks = true;
             bricks = bricks && brick_elems < 0x7fffffffLL;
-            void* brick = nullptr;
-            if (bricks) {
-                if (hipMallocAsync(&brick, static_cast<size_t>(brick_elems) * sizeof(S), stream) != hipSuccess) {
-                    (void)hipGetLastError();
-                    brick = nullptr;   // not enough memory for the copy: gather from the row-major volume
-                }
-            }
+            // Without memory for the copy: gather from the row-major volume.
+            CallWorkspace copy;
+            if (bricks) copy = CallWorkspace(static_cast<size_t>(brick_elems) * sizeof(S), stream);
+            void* brick = copy.data();
             // Pixel patches (extract_c32_kernel<PATCH>): rows and the columns but the last in blocks of 8, four
             // patches per workgroup.
             const i32 pr = p.slice_h / 8, pc = (p.slice_wr - 1) / 8;
@@ -826,7 +824,6 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err) {
                     else if (q.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, true, S>), grid, block, 0, stream, q);
                     else hipLaunchKernelGGL((extract_c32_kernel<0, true, S>), grid, block, 0, stream, q);
                 }
-                (void)hipFreeAsync(brick, stream);
             } else {
                 if (p.shift_mode == 0) hipLaunchKernelGGL((extract_c32_kernel<1, false, S>), grid, block, 0, stream, p);
                 else if (p.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, false, S>), grid, block, 0, stream, p);

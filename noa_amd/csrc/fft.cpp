@@ -25,6 +25,7 @@
 
 #include "../../include/noa_hip.h"
 #include "kernels.hpp"
+#include "workspace.hpp"
 
 namespace noa_hip {
 namespace {
@@ -306,20 +307,20 @@ int launch_fft(const FftDesc& d, hipStream_t stream, std::string& err) {
     if (!plan->has_workspace) { err = "Trying to run a plan without a workspace"; return NOA_HIP_ERROR_RUNTIME; }
 
     // Staging buffer (stream-ordered): the contiguous copy of the real operand.
-    void* tmp = nullptr;
+    CallWorkspace staging;
     const i64 contiguous[4] = {d.shape[1] * d.shape[2] * d.shape[3], d.shape[2] * d.shape[3], d.shape[3], 1};
     if (stage) {
         const size_t bytes = static_cast<size_t>(d.shape[0] * contiguous[0]) * (d.f64 ? 8 : 4);
-        if (hipMallocAsync(&tmp, bytes, stream) != hipSuccess) {
-            (void)hipGetLastError();
+        staging = CallWorkspace(bytes, stream);
+        if (!staging) {
             err = "Could not allocate the staging buffer of a strided real FFT operand";
             return NOA_HIP_ERROR_RUNTIME;
         }
-        if (real_in && (st = launch_strided_copy(d.in, d.in_s, tmp, contiguous, d.shape, d.f64, stream, err)) != NOA_HIP_OK) {
-            (void)hipFreeAsync(tmp, stream);
+        if (real_in &&
+            (st = launch_strided_copy(d.in, d.in_s, staging.data(), contiguous, d.shape, d.f64, stream, err)) != NOA_HIP_OK)
             return st;
-        }
     }
+    void* tmp = staging.data();
     rocfft_status s = rocfft_execution_info_set_stream(plan->info, stream);
     if (s == rocfft_status_success) {
         void* in_buf[1] = {stage && real_in ? tmp : d.in};
@@ -330,7 +331,6 @@ int launch_fft(const FftDesc& d, hipStream_t stream, std::string& err) {
         st = launch_strided_copy(tmp, contiguous, d.out, d.out_s, d.shape, d.f64, stream, err);
     else
         st = NOA_HIP_OK;
-    if (tmp) (void)hipFreeAsync(tmp, stream);
     if (s != rocfft_status_success) {
         err = std::string("rocfft_execute: ") + rocfft_status_str(s);
         return NOA_HIP_ERROR_RUNTIME;

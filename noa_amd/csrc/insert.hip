@@ -29,6 +29,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "workspace.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -1435,7 +1436,6 @@ struct Plan {
     std::vector<i32> h_bricks;             // active sub-bricks (pose-adaptive plans count their passing slices)
     std::vector<i32> h_nseg;               // segments of each active sub-brick in this plan
     i32* bricks{};                         // device copy of h_bricks, uploaded on first use
-    bool owned{};                          // device arrays freed with the plan (pose-adaptive plans, one call)
     double target{};                       // expected passing slices per item the plan was cut for
 };
 
@@ -1973,8 +1973,9 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                     }
                 }
                 const i32 nbk = static_cast<i32>(shared.h_bricks.size());
-                i32* dcounts = nullptr;
-                if (hipMallocAsync(&dcounts, static_cast<size_t>(nbk) * CNT_BINS * sizeof(i32), stream) != hipSuccess) {
+                const CallWorkspace counts_ws(static_cast<size_t>(nbk) * CNT_BINS * sizeof(i32), stream);
+                i32* dcounts = counts_ws.data<i32>();
+                if (!dcounts) {
                     err = "insert: could not allocate the pass counts";
                     return NOA_HIP_ERROR_RUNTIME;
                 }
@@ -2006,7 +2007,6 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                 const bool ok = hipMemcpyAsync(counts.data(), dcounts, counts.size() * sizeof(i32), hipMemcpyDeviceToHost,
                                                stream) == hipSuccess &&
                                 hipStreamSynchronize(stream) == hipSuccess;
-                (void)hipFreeAsync(dcounts, stream);
                 if (!ok) { err = "insert: could not read the pass counts"; return NOA_HIP_ERROR_RUNTIME; }
                 // The model plan stays when no sub-brick needs more than twice its segments.
                 bool skewed = false;
@@ -2017,36 +2017,29 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                 }
                 if (skewed) make_pose_plan(shared.h_bricks, counts, p.n_slices, shared.target, pose);
             }
+            CallWorkspace pose_items, pose_reduce;
             if (pose.n_items > 0) {
-                if (hipMallocAsync(&pose.items, pose.h_items.size() * sizeof(int4), stream) != hipSuccess ||
-                    hipMemcpyAsync(pose.items, pose.h_items.data(), pose.h_items.size() * sizeof(int4),
-                                   hipMemcpyHostToDevice, stream) != hipSuccess ||
+                pose_items = CallWorkspace(pose.h_items.size() * sizeof(int4), stream);
+                pose.items = pose_items.data<int4>();
+                if (!pose.h_reduce.empty()) pose_reduce = CallWorkspace(pose.h_reduce.size() * sizeof(int4), stream);
+                pose.reduce = pose_reduce.data<int4>();
+                if (!pose.items || hipMemcpyAsync(pose.items, pose.h_items.data(), pose.h_items.size() * sizeof(int4),
+                                                  hipMemcpyHostToDevice, stream) != hipSuccess ||
                     (!pose.h_reduce.empty() &&
-                     (hipMallocAsync(&pose.reduce, pose.h_reduce.size() * sizeof(int4), stream) != hipSuccess ||
-                      hipMemcpyAsync(pose.reduce, pose.h_reduce.data(), pose.h_reduce.size() * sizeof(int4),
-                                     hipMemcpyHostToDevice, stream) != hipSuccess))) {
+                     (!pose.reduce || hipMemcpyAsync(pose.reduce, pose.h_reduce.data(), pose.h_reduce.size() * sizeof(int4),
+                                                     hipMemcpyHostToDevice, stream) != hipSuccess))) {
                     err = "insert: could not upload the pose-adaptive plan";
                     return NOA_HIP_ERROR_RUNTIME;
                 }
-                pose.owned = true;
                 planp = &pose;
             }
             const Plan& plan = *planp;
-            // The pose-adaptive plan's device arrays are released after this call's kernels (stream-ordered).
-            struct PoseRelease {
-                Plan& pl;
-                hipStream_t st;
-                ~PoseRelease() {
-                    if (!pl.owned) return;
-                    if (pl.items) (void)hipFreeAsync(pl.items, st);
-                    if (pl.reduce) (void)hipFreeAsync(pl.reduce, st);
-                }
-            } pose_release{pose, stream};
             if (plan.n_items == 0) return NOA_HIP_OK;
             const size_t partial_bytes = static_cast<size_t>(plan.n_partials) * p.bd[0] * p.bd[1] * p.apitch * 3 *
                                          sizeof(float);
             // The allocation-free entry point's limit counts 64 bytes per slice beside the plan and the partial sums.
             const size_t record_bytes = static_cast<size_t>(p.n_slices) * 64;
+            CallWorkspace partial_ws;
             void* partials = nullptr;
             if (scratch) {
                 // Allocation-free: plan and partial sums in the caller-independent scratch, in that order.
@@ -2078,7 +2071,9 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
             } else {
                 p.items = plan.items;
                 p.reduce = plan.reduce;
-                if (plan.n_partials > 0 && hipMallocAsync(&partials, partial_bytes, stream) != hipSuccess) {
+                if (plan.n_partials > 0) partial_ws = CallWorkspace(partial_bytes, stream);
+                partials = partial_ws.data();
+                if (plan.n_partials > 0 && !partials) {
                     err = "insert: could not allocate the partial sums";
                     return NOA_HIP_ERROR_RUNTIME;
                 }
@@ -2118,11 +2113,7 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
             }
             if (plan.n_reduce > 0)
                 hipLaunchKernelGGL((insert_reduce_kernel<C, In, Out, W>), dim3(plan.n_reduce), dim3(NT_REDUCE), 0, stream, p);
-            hipError_t e = hipGetLastError();
-            if (partials && !scratch) {
-                const hipError_t fe = hipFreeAsync(partials, stream);
-                if (e == hipSuccess) e = fe;
-            }
+            const hipError_t e = hipGetLastError();
             if (e != hipSuccess) { err = std::string("kernel launch failed: ") + hipGetErrorString(e); return NOA_HIP_ERROR_RUNTIME; }
             return NOA_HIP_OK;
         }

@@ -14,6 +14,7 @@
 // instead: the accumulation happens in LDS and reaches the volume once per work item.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "workspace.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -751,21 +752,16 @@ int run_tiles(const ProjectDesc& d, const RasterParams<C, In, Out, W>& p, hipStr
     const dim3 boxes(static_cast<u32>(plan.n_boxes * max_items));
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     (void)hipStreamIsCapturing(stream, &capture);
-    if (n_slices > 64 && capture == hipStreamCaptureStatusNone) {
-        if (hipMallocAsync(reinterpret_cast<void**>(&q.starts), static_cast<size_t>(plan.n_boxes) * max_items * sizeof(i32),
-                           stream) == hipSuccess)
-            hipLaunchKernelGGL((rasterize_items_kernel<In, Out>), dim3(static_cast<u32>(plan.n_boxes)), dim3(RB_SCAN), 0,
-                               stream, q);
-        else
-            (void)hipGetLastError(), q.starts = nullptr;
-    }
+    CallWorkspace starts;
+    if (n_slices > 64 && capture == hipStreamCaptureStatusNone)
+        starts = CallWorkspace(static_cast<size_t>(plan.n_boxes) * max_items * sizeof(i32), stream);
+    q.starts = starts.data<i32>();
+    if (q.starts)
+        hipLaunchKernelGGL((rasterize_items_kernel<In, Out>), dim3(static_cast<u32>(plan.n_boxes)), dim3(RB_SCAN), 0,
+                           stream, q);
     if (gen) hipLaunchKernelGGL((rasterize_box_kernel<In, Out, true>), boxes, dim3(64), 0, stream, q);
     else hipLaunchKernelGGL((rasterize_box_kernel<In, Out, false>), boxes, dim3(64), 0, stream, q);
-    hipError_t e = hipGetLastError();
-    if (q.starts) {
-        const hipError_t fe = hipFreeAsync(q.starts, stream);
-        if (e == hipSuccess) e = fe;
-    }
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) { err = std::string("kernel launch failed: ") + hipGetErrorString(e); return NOA_HIP_ERROR_RUNTIME; }
     return NOA_HIP_OK;
 }

@@ -738,6 +738,13 @@ def cubic_bspline_prefilter(input, output) -> None:
         raise NoaError(last_error())
 
 
+def workspace_trim(device=None) -> int:
+    """Gives the device workspaces that the calls keep for the next ones (at most 1 GiB per GPU) back; returns their
+    bytes."""
+    index = torch.cuda.current_device() if device is None else torch.device(device).index or 0
+    return int(lib().noa_hip_workspace_trim(index))
+
+
 def rfft_shape(shape: Sequence[int]) -> tuple[int, int, int, int]:
     """Shape4::rfft (src/noa/runtime/core/Shape.hpp:380): (B, D, H, W//2+1)."""
     b, d, h, w = _shape4(shape, "shape")
