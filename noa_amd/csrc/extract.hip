@@ -218,25 +218,42 @@ __global__ __launch_bounds__(256) void extract_kernel(const ExtractParams<C> p) 
 // work that the general kernel does for every pixel: the integer division of the pixel index (here a float
 // reciprocal, exact for slices below 2^21 pixels, checked on the host), the runtime selection between the plain and
 // the scaled/EWS transforms, the weight paths, and the runtime choice of the shift precision.
-// Copy of a complex volume (unit x stride; c32 or a pair of 16-bit floats) into the block layout of BrickLayout:
-// one lane per element of the stored (nz, ny, wr) volume; the block padding (sizes not multiples of the block) is
-// never read.
+// Copy of a complex volume (unit x stride; c32 or a pair of 16-bit floats) into the block layout of BrickLayout, in the
+// order of the copy: a wave writes two whole blocks, next to each other along x, and reads them as 64-byte (c32) pieces
+// of 8 rows. The block padding (sizes not multiples of the block) is never read and not written. In the order of the
+// volume, each lane's element written where it belongs (32-byte pieces), the copy of 256^3 took 40 us, this one 35.
+constexpr u32 BRICK_EPT = 4;
 template<class S>
 __global__ __launch_bounds__(256) void brick_volume_kernel(const S* __restrict__ in, i32 vs0, i32 vs1,
-                                                           S* __restrict__ out, i32 ny, i32 wr, i64 total,
+                                                           S* __restrict__ out, u32 nz, u32 ny, u32 wr, u32 total,
                                                            BrickLayout L) {
-    const i64 i = static_cast<i64>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= total) return;
-    const i32 x = static_cast<i32>(i % wr);
-    const i64 r = i / wr;
-    const i32 y = static_cast<i32>(r % ny), z = static_cast<i32>(r / ny);
-    out[L.z(z) + L.y(y) + L.x(x)] = in[static_cast<i64>(z) * vs0 + static_cast<i64>(y) * vs1 + x];
+    constexpr u32 IN = BrickLayout::LX + BrickLayout::LY + BrickLayout::LZ;
+    const u32 first = blockIdx.x * (256u * BRICK_EPT) + threadIdx.x;
+    const u32 bx = static_cast<u32>(L.by) >> IN, by = static_cast<u32>(L.bz / L.by);   // blocks along x and y
+    S v[BRICK_EPT];
+    bool live[BRICK_EPT];
+#pragma unroll
+    for (u32 e = 0; e < BRICK_EPT; ++e) {
+        const u32 i = first + e * 256u, block = i >> IN, in_block = i & ((1u << IN) - 1);
+        const u32 row = block / bx, page = row / by;
+        const u32 x = ((block - row * bx) << BrickLayout::LX) + (in_block & ((1u << BrickLayout::LX) - 1));
+        const u32 y = ((row - page * by) << BrickLayout::LY) +
+                      ((in_block >> BrickLayout::LX) & ((1u << BrickLayout::LY) - 1));
+        const u32 z = (page << BrickLayout::LZ) + (in_block >> (BrickLayout::LX + BrickLayout::LY));
+        live[e] = i < total && x < wr && y < ny && z < nz;
+        if (live[e]) v[e] = in[static_cast<i64>(z) * vs0 + static_cast<i64>(y) * vs1 + x];
+    }
+#pragma unroll
+    for (u32 e = 0; e < BRICK_EPT; ++e)
+        if (live[e]) out[first + e * 256u] = v[e];
 }
 
 // PATCH: each wave takes an 8 x 8 patch of pixels (rows y0..y0+7, columns u0..u0+7) instead of 64 consecutive
 // pixels of a row: the patch samples a compact piece of the plane, so each tap load touches fewer cache lines of the
-// volume. Workgroups [0, patch_wgs) of a slice hold four patches each (columns 0..wr-2); the next ones take the last
-// column (u = wr - 1), 256 rows per workgroup.
+// volume. Workgroups [0, patch_wgs) of a slice hold four patches each, the last ones of a row or column partly outside
+// the slice; where one column would be left over (wr = 8 k + 1, the half of a size that is a multiple of 16), the next
+// workgroups take it, 256 rows each.
+constexpr i32 NPATCH = 2;              // patches per wave, next to each other along x, their loads in flight together
 template<int SHIFT, bool BRICK, class S, bool PATCH = false>
 __global__ __launch_bounds__(256) void extract_c32_kernel(const ExtractParams<float> p) {
     const u32 lb = xcd_swizzle(blockIdx.x, gridDim.x);
@@ -256,7 +273,7 @@ __global__ __launch_bounds__(256) void extract_c32_kernel(const ExtractParams<fl
     const S* __restrict__ vol = static_cast<const S*>(p.vol);
     float2* __restrict__ out = static_cast<float2*>(p.out) + static_cast<i64>(b) * p.os_b;
 
-    constexpr i32 MAXP = PATCH ? 1 : 4;
+    constexpr i32 MAXP = PATCH ? NPATCH : 4;
     Taps3<float2, float> tv[MAXP];
     bool inside[MAXP];
     i32 ys[MAXP], us[MAXP];
@@ -270,12 +287,14 @@ __global__ __launch_bounds__(256) void extract_c32_kernel(const ExtractParams<fl
             if (tile < p.patch_wgs) {
                 const i32 q = tile * 4 + wave, pr = q / p.patch_pc, pc = q - pr * p.patch_pc;
                 y = pr * 8 + (lane >> 3);
-                u = pc * 8 + (lane & 7);
-                live = true;
+                u = (pc * NPATCH + k) * 8 + (lane & 7);
+                live = y < p.slice_h && u < p.slice_wr;
+                y = live ? y : 0;
+                u = live ? u : 0;
             } else {
                 y = (tile - p.patch_wgs) * 256 + static_cast<i32>(threadIdx.x);
                 u = p.slice_wr - 1;
-                live = y < p.slice_h;
+                live = k == 0 && y < p.slice_h;
                 y = live ? y : 0;
             }
         } else {
@@ -291,8 +310,8 @@ __global__ __launch_bounds__(256) void extract_c32_kernel(const ExtractParams<fl
         us[k] = u;
         vec2<float> f2;
         const i32 fy = index2frequency(p.slice_centered, y, p.slice_h);
-        f2.y = static_cast<float>(fy) / p.slice_f[0];
-        f2.x = static_cast<float>(u) / p.slice_f[1];
+        f2.y = divide_index(static_cast<float>(fy), p.slice_f[0], p.norm_f[0]);
+        f2.x = divide_index(static_cast<float>(u), p.slice_f[1], p.norm_f[1]);
         const vec3<float> f = slice2grid<false>(f2, sc, rot, 0.f, 0.f);
         inside[k] = live && dot3(f) <= p.cutoff_sqd;
         const float fz = f.z * p.target[0], fyv = f.y * p.target[1], fx = f.x * p.target[2];
@@ -794,40 +813,48 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err) {
             CallWorkspace copy;
             if (bricks) copy = CallWorkspace(static_cast<size_t>(brick_elems) * sizeof(S), stream);
             void* brick = copy.data();
-            // Pixel patches (extract_c32_kernel<PATCH>): rows and the columns but the last in blocks of 8, four
-            // patches per workgroup.
-            const i32 pr = p.slice_h / 8, pc = (p.slice_wr - 1) / 8;
-            bool patch = p.slice_h % 8 == 0 && (p.slice_wr - 1) % 8 == 0 && (pr * pc) % 4 == 0 && pr * pc > 0;
-            if (const char* pe = std::getenv("NOA_HIP_EXTRACT_PATCH")) patch = patch && pe[0] != '0';
-            const i64 patch_tiles = pr * pc / 4 + (p.slice_h + 255) / 256;
-            patch = patch && n_slices * patch_tiles <= 0x7fffffffLL;
+            // Pixel patches (extract_c32_kernel<PATCH>), four per workgroup.
+            const bool last_column = p.slice_wr % 8 == 1 && p.slice_wr > 1;
+            const i32 pr = (p.slice_h + 7) / 8, pc = ((last_column ? p.slice_wr / 8 : (p.slice_wr + 7) / 8) + NPATCH - 1) / NPATCH;
+            const i32 patch_wgs = (pr * pc + 3) / 4;
+            const i64 patch_tiles = patch_wgs + (last_column ? (p.slice_h + 255) / 256 : 0);
+            // Where the patches cover up to an eighth more than the slice. Patches and rows: 4,096 slices of 256^2 0.95
+            // and 1.09 ms, 1,000 of 250^2 0.27 and 0.31, 500 of 384^2 from the row-major volume 0.46 and 0.60, 500 of
+            // 180^2 (8 % more) 84 and 82 us, 3,000 of 40^2 (52 % more) 40 and 37 us.
+            const i64 covered = static_cast<i64>(pr) * pc * 64 * NPATCH + (last_column ? p.slice_h : 0);
+            bool patch = n_slices * patch_tiles <= 0x7fffffffLL && 8 * covered <= 9 * static_cast<i64>(p.pixels);
+            if (const char* pe = std::getenv("NOA_HIP_EXTRACT_PATCH"))
+                patch = pe[0] != '0' && n_slices * patch_tiles <= 0x7fffffffLL;
+            auto launch = [&](ExtractParams<C> q, auto from_brick) {
+                constexpr bool B = decltype(from_brick)::value;
+                if (patch) {
+                    q.ppt = 1;
+                    q.patch_wgs = patch_wgs;
+                    q.patch_pc = pc;
+                    q.tiles = static_cast<i32>(patch_tiles);
+                    const dim3 pgrid(static_cast<u32>(n_slices * patch_tiles));
+                    if (q.shift_mode == 0) hipLaunchKernelGGL((extract_c32_kernel<1, B, S, true>), pgrid, block, 0, stream, q);
+                    else if (q.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, B, S, true>), pgrid, block, 0, stream, q);
+                    else hipLaunchKernelGGL((extract_c32_kernel<0, B, S, true>), pgrid, block, 0, stream, q);
+                } else {
+                    if (q.shift_mode == 0) hipLaunchKernelGGL((extract_c32_kernel<1, B, S, false>), grid, block, 0, stream, q);
+                    else if (q.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, B, S, false>), grid, block, 0, stream, q);
+                    else hipLaunchKernelGGL((extract_c32_kernel<0, B, S, false>), grid, block, 0, stream, q);
+                }
+            };
             if (brick) {
                 const BrickLayout L{static_cast<i32>(bz), static_cast<i32>(by)};
-                hipLaunchKernelGGL((brick_volume_kernel<S>), dim3(static_cast<u32>((stored + 255) / 256)), dim3(256), 0,
-                                   stream, static_cast<const S*>(p.vol), p.vs0, p.vs1, static_cast<S*>(brick),
-                                   ny, wr, stored, L);
+                hipLaunchKernelGGL((brick_volume_kernel<S>), dim3(static_cast<u32>((brick_elems + 256 * BRICK_EPT - 1) / (256 * BRICK_EPT))),
+                                   dim3(256), 0, stream, static_cast<const S*>(p.vol), p.vs0, p.vs1, static_cast<S*>(brick),
+                                   static_cast<u32>(nz), static_cast<u32>(ny), static_cast<u32>(wr),
+                                   static_cast<u32>(brick_elems), L);
                 ExtractParams<C> q = p;
                 q.vol = brick;
                 q.vs0 = L.bz;
                 q.vs1 = L.by;
-                if (patch) {
-                    q.ppt = 1;
-                    q.patch_wgs = pr * pc / 4;
-                    q.patch_pc = pc;
-                    q.tiles = static_cast<i32>(patch_tiles);
-                    const dim3 pgrid(static_cast<u32>(n_slices * patch_tiles));
-                    if (q.shift_mode == 0) hipLaunchKernelGGL((extract_c32_kernel<1, true, S, true>), pgrid, block, 0, stream, q);
-                    else if (q.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, true, S, true>), pgrid, block, 0, stream, q);
-                    else hipLaunchKernelGGL((extract_c32_kernel<0, true, S, true>), pgrid, block, 0, stream, q);
-                } else {
-                    if (q.shift_mode == 0) hipLaunchKernelGGL((extract_c32_kernel<1, true, S>), grid, block, 0, stream, q);
-                    else if (q.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, true, S>), grid, block, 0, stream, q);
-                    else hipLaunchKernelGGL((extract_c32_kernel<0, true, S>), grid, block, 0, stream, q);
-                }
+                launch(q, std::true_type{});
             } else {
-                if (p.shift_mode == 0) hipLaunchKernelGGL((extract_c32_kernel<1, false, S>), grid, block, 0, stream, p);
-                else if (p.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, false, S>), grid, block, 0, stream, p);
-                else hipLaunchKernelGGL((extract_c32_kernel<0, false, S>), grid, block, 0, stream, p);
+                launch(p, std::false_type{});
             }
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) { err = std::string("kernel launch failed: ") + hipGetErrorString(e); return NOA_HIP_ERROR_RUNTIME; }
@@ -964,9 +991,10 @@ int volume_blocks(const void* volume, i64 s_z, i64 s_y, const int64_t rfft_shape
     }
     if (stored == 0) return NOA_HIP_OK;
     const BrickLayout L{static_cast<i32>(bz), static_cast<i32>(by)};
-    hipLaunchKernelGGL((brick_volume_kernel<float2>), dim3(static_cast<u32>((stored + 255) / 256)), dim3(256), 0, stream,
-                       static_cast<const float2*>(volume), static_cast<i32>(s_z), static_cast<i32>(s_y),
-                       static_cast<float2*>(blocks), static_cast<i32>(ny), static_cast<i32>(wr), stored, L);
+    hipLaunchKernelGGL((brick_volume_kernel<float2>), dim3(static_cast<u32>((count + 256 * BRICK_EPT - 1) / (256 * BRICK_EPT))),
+                       dim3(256), 0, stream, static_cast<const float2*>(volume), static_cast<i32>(s_z), static_cast<i32>(s_y),
+                       static_cast<float2*>(blocks), static_cast<u32>(nz), static_cast<u32>(ny), static_cast<u32>(wr),
+                       static_cast<u32>(count), L);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) { err = std::string("kernel launch failed: ") + hipGetErrorString(e); return NOA_HIP_ERROR_RUNTIME; }
     return NOA_HIP_OK;

@@ -163,3 +163,31 @@ def test_tuning_table_selects_tiles(monkeypatch):
         autotune.apply([])
     for o in outs:
         np.testing.assert_array_equal(o.view(np.uint32), forced.view(np.uint32))
+
+
+@pytest.mark.parametrize("layout", ["linear", "bricks"])
+@pytest.mark.parametrize("n,shifts", [(32, True), (47, False), (62, True), (64, False), (65, True), (94, False), (180, True)])
+def test_pixel_patches_equal_the_rows(monkeypatch, layout, n, shifts):
+    """Waves of two 8x8 pixel patches (with pixels outside the slice at its ends, or a last column of its own) and waves of
+    64 pixels of a row evaluate the same expressions per pixel: the same bits."""
+    print(f"case extract patches n={n} {layout}", flush=True)
+    rng = np.random.default_rng(600 + n)
+    b, wr = 9, n // 2 + 1
+    volume = dev(random_spectrum((1, n, n, wr), rng))
+    rot = dev(random_rotations(b, rng))
+    sh = dev(rng.uniform(-5, 5, (b, 2)).astype(np.float32))
+    monkeypatch.setenv("NOA_HIP_EXTRACT_LAYOUT", layout)
+    outs = []
+    for patch in ("1", "0"):
+        monkeypatch.setenv("NOA_HIP_EXTRACT_PATCH", patch)
+        room = torch.full((b, 1, n, wr + 2), float("nan"), dtype=torch.complex64, device=DEV)
+        out = room[..., :wr]
+        if shifts:
+            nx().extract_central_slices_3d_shifted("hc2h", volume, None, (1, n, n, n), out, None, (b, 1, n, n), None, rot, sh)
+        else:
+            nx().extract_central_slices_3d("h2hc", volume, None, (1, n, n, n), out, None, (b, 1, n, n), None, rot)
+        torch.cuda.synchronize()
+        assert bool(torch.isnan(room[..., wr:].real).all())
+        outs.append(out.cpu().numpy())
+    assert np.isfinite(outs[0]).all()
+    np.testing.assert_array_equal(outs[0], outs[1])
