@@ -7,16 +7,20 @@
 //
 // The recursion is sequential along a line, so one lane owns one line, with noa's expressions in noa's order
 // (bit-identical to the CPU path). What differs from a lane-per-line loop over memory is the access pattern:
-//  - lines along y and z: the 64 lanes of a wave own 64 neighbouring x, so every step of the recursion is one
+//  - lines along x that fit in LDS (up to 2,048 samples of 4 bytes), and along y and z where there are few: a workgroup copies a tile of whole lines into LDS with all of
+//    its lanes, one lane per line runs both recursions there, and the workgroup stores the tile: each pass reads and
+//    writes the array once, with all loads of a tile in flight (bspline_tile_kernel);
+//  - other lines along y and z: the 64 lanes of a wave own 64 neighbouring x, so every step of the recursion is one
 //    coalesced 64-element access; steps are loaded in batches of 16, the next batch in flight while the current
 //    one's dependent arithmetic runs;
-//  - lines along x (the contiguous axis): a wave owns 64 rows and walks them in 32-column chunks staged through
+//  - longer lines along x (the contiguous axis): a wave owns 64 rows and walks them in 32-column chunks staged through
 //    LDS, loaded and stored as whole row segments; the lanes then run their row's recursion out of LDS while the
-//    next chunk's loads are in flight.
-// Each pass reads and writes the array once; the anticausal half re-reads the causal half's output, which the
-// column passes do straight from the L2/last-level cache and the row pass from LDS for the last chunk.
+//    next chunk's loads are in flight. In both, the anticausal half re-reads the causal half's output.
 #include "common.hpp"
 #include "kernels.hpp"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace noa_hip {
 
@@ -241,6 +245,167 @@ __global__ __launch_bounds__(256) void bspline_lines_kernel(const LinesParams<T>
     }
 }
 
+// Whole lines in LDS. ROWS: the lines run along the contiguous axis, and a wave copies stretches of one line at a time
+// (LDS lines of an odd pitch, so that the lanes of the recursion read different banks); otherwise neighbouring lines are
+// neighbours in memory, and a wave copies pieces of 128 bytes across them.
+// Bound by the copies and by the latency of the recursion, which one half-wave per workgroup runs (about 16 clocks per
+// sample and direction) while other workgroups of the CU copy. Rows of 181 x 300 x 275 f32 44 us (92 us in chunks,
+// the lanes waiting for each), of 24 x 24 x 24, all three passes, 17 against 24 us. 64 bytes across the lines or 512 lanes
+// were no faster.
+constexpr i32 TILE_LANES = 256;
+constexpr size_t TILE_LDS = 64 * 1024;
+// Across the contiguous axis, a lane per line in memory is as fast once there are three waves of lines per CU or more
+// (49,775 lines of 300 samples 48 against 54 us, 65,536 of 256 45 against 43; 720 of 320 and 9,600 of 24, both passes, 40
+// against 17 us).
+constexpr i64 TILE_MAX_LINES = 49152;
+
+template<class T, bool ROWS, i32 WIDTH>
+__global__ __launch_bounds__(TILE_LANES) void bspline_tile_kernel(const LinesParams<T> p, i32 tiles_c) {
+    using R = typename vt<T>::real;
+    using K = BSplineConst<R>;
+    extern __shared__ __align__(16) unsigned char lds_bytes[];
+    T* const lds = reinterpret_cast<T*>(lds_bytes);
+    const i32 t = static_cast<i32>(threadIdx.x), n = p.n;
+    // The tile's lines: WIDTH consecutive lines (ROWS), or the ones at c0 .. c0 + WIDTH - 1 of the fastest line index.
+    i64 first;
+    i32 lines;
+    if constexpr (ROWS) {
+        first = static_cast<i64>(blockIdx.x) * WIDTH;
+        lines = static_cast<i32>(min<i64>(WIDTH, p.lines - first));
+    } else {
+        const i64 outer = blockIdx.x / static_cast<u32>(tiles_c);
+        const i32 c0 = static_cast<i32>(blockIdx.x % static_cast<u32>(tiles_c)) * WIDTH;
+        first = outer * p.n2 + c0;
+        lines = min(WIDTH, p.n2 - c0);
+    }
+    auto base_of = [&](i64 line, const i64 (&s)[3]) {
+        const i64 c = line % p.n2, u = line / p.n2;
+        return u / p.n1 * s[0] + u % p.n1 * s[1] + c * s[2];
+    };
+    const i32 pitch = ROWS ? (n | 1) : 1;              // LDS strides of lines and of samples
+    constexpr i32 step = ROWS ? 1 : WIDTH;
+    // The copies: EACH elements per lane in flight. ROWS: a wave takes EACH lines and 64 samples of each at a time;
+    // otherwise WIDTH lanes take one sample each of neighbouring lines.
+    constexpr i32 EACH = ROWS ? WIDTH / (TILE_LANES / 64) : 8;
+    static_assert(EACH >= 1, "whole lines per wave");
+    const i32 wave = t >> 6, lane = t & 63;
+    const i32 l = t % WIDTH, per = TILE_LANES / WIDTH;
+    const i64 at_in = base_of(first, p.in_s), at_out = base_of(first, p.out_s);
+    auto copy = [&](auto move) {
+        if constexpr (ROWS) {
+            for (i32 j = lane; j < n; j += 64) move(wave * EACH, j);
+        } else {
+            if (l < lines)
+                for (i32 j = t / WIDTH; j < n; j += per * EACH) move(l, j);
+        }
+    };
+    i64 row_in[ROWS ? EACH : 1], row_out[ROWS ? EACH : 1];
+    if constexpr (ROWS) {
+#pragma unroll
+        for (i32 q = 0; q < EACH; ++q) {
+            const i64 line = min(first + wave * EACH + q, p.lines - 1);
+            row_in[q] = base_of(line, p.in_s);
+            row_out[q] = base_of(line, p.out_s);
+        }
+    }
+    copy([&](i32 at, i32 j) {
+        T v[EACH];
+#pragma unroll
+        for (i32 q = 0; q < EACH; ++q) {
+            if constexpr (ROWS) {
+                if (at + q < lines) v[q] = p.in[row_in[q] + static_cast<i64>(j) * p.in_step];
+            } else {
+                if (j + q * per < n)
+                    v[q] = p.in[at_in + static_cast<i64>(at) * p.in_s[2] + static_cast<i64>(j + q * per) * p.in_step];
+            }
+        }
+#pragma unroll
+        for (i32 q = 0; q < EACH; ++q) {
+            if constexpr (ROWS) {
+                if (at + q < lines) lds[(at + q) * pitch + j] = v[q];
+            } else {
+                if (j + q * per < n) lds[(j + q * per) * WIDTH + at] = v[q];
+            }
+        }
+    });
+    __syncthreads();
+    if (t < lines) {
+        T* const line = lds + t * pitch;
+        constexpr i32 U = sizeof(T) <= 8 ? 16 : 8;
+        // Causal initialisation (:87-100) and recursion (:67-73).
+        const i32 horizon = min(12, n);
+        R zn = K::POLE;
+        T sum = line[0];
+        for (i32 k = 0; k < horizon; ++k) {
+            sum = vadd(sum, vmul(line[k * step], zn));
+            zn *= K::POLE;
+        }
+        T prev = vmul(sum, K::LAMBDA);
+        line[0] = prev;
+        i32 j = 1;
+        T cur[U], nxt[U];
+        if (j + U <= n) {
+#pragma unroll
+            for (i32 k = 0; k < U; ++k) cur[k] = line[(j + k) * step];
+        }
+        for (; j + U <= n; j += U) {
+            if (j + 2 * U <= n) {
+#pragma unroll
+                for (i32 k = 0; k < U; ++k) nxt[k] = line[(j + U + k) * step];
+            }
+#pragma unroll
+            for (i32 k = 0; k < U; ++k) {
+                prev = vadd(vmul(cur[k], K::LAMBDA), vmul(prev, K::POLE));
+                line[(j + k) * step] = prev;
+            }
+#pragma unroll
+            for (i32 k = 0; k < U; ++k) cur[k] = nxt[k];
+        }
+        for (; j < n; ++j) {
+            prev = vadd(vmul(line[j * step], K::LAMBDA), vmul(prev, K::POLE));
+            line[j * step] = prev;
+        }
+        // Anticausal initialisation (:102-106) from c[n-1], which `prev` holds, and recursion (:75-79).
+        prev = vmul(prev, K::ANTI);
+        line[(n - 1) * step] = prev;
+        j = n - 2;
+        if (j - U + 1 >= 0) {
+#pragma unroll
+            for (i32 k = 0; k < U; ++k) cur[k] = line[(j - k) * step];
+        }
+        for (; j - U + 1 >= 0; j -= U) {
+            if (j - 2 * U + 1 >= 0) {
+#pragma unroll
+                for (i32 k = 0; k < U; ++k) nxt[k] = line[(j - U - k) * step];
+            }
+#pragma unroll
+            for (i32 k = 0; k < U; ++k) {
+                prev = vmul(vsub(prev, cur[k]), K::POLE);
+                line[(j - k) * step] = prev;
+            }
+#pragma unroll
+            for (i32 k = 0; k < U; ++k) cur[k] = nxt[k];
+        }
+        for (; j >= 0; --j) {
+            prev = vmul(vsub(prev, line[j * step]), K::POLE);
+            line[j * step] = prev;
+        }
+    }
+    __syncthreads();
+    copy([&](i32 at, i32 j) {
+#pragma unroll
+        for (i32 q = 0; q < EACH; ++q) {
+            if constexpr (ROWS) {
+                if (at + q < lines) p.out[row_out[q] + static_cast<i64>(j) * p.out_step] = lds[(at + q) * pitch + j];
+            } else {
+                if (j + q * per < n)
+                    p.out[at_out + static_cast<i64>(at) * p.out_s[2] + static_cast<i64>(j + q * per) * p.out_step] =
+                        lds[(j + q * per) * WIDTH + at];
+            }
+        }
+    });
+}
+
 namespace {
 
 // Launch of one pass over `lines` lines of `n` samples; the outer dimensions are (lines / (n1 * n2), n1, n2).
@@ -258,7 +423,24 @@ int pass(bool rows, const T* in, const i64 in_s[3], i64 in_step, T* out, const i
     p.lines = n0 * n1 * n2;
     p.n = static_cast<i32>(n);
     if (p.lines == 0 || n == 0) return NOA_HIP_OK;
-    if (rows) {
+    // Tiles of 128 bytes across the lines (and at least as many lines of the rows), halved until a tile fits.
+    i64 width = std::max<i64>(8, 128 / static_cast<i64>(sizeof(T)));
+    const i64 pitch = rows ? (n | 1) : n;
+    while (width > 8 && static_cast<size_t>(width * pitch) * sizeof(T) > TILE_LDS) width /= 2;
+    const size_t lds = static_cast<size_t>(width * pitch) * sizeof(T);
+    const i64 tiles_c = (n2 + width - 1) / width;
+    const i64 tiles = rows ? (p.lines + width - 1) / width : n0 * n1 * tiles_c;
+    if (lds <= TILE_LDS && tiles <= 0x7fffffffLL && (rows || p.lines < TILE_MAX_LINES)) {
+        auto launch = [&](auto w) {
+            constexpr i32 W = decltype(w)::value;
+            const dim3 grid(static_cast<u32>(tiles)), block(TILE_LANES);
+            if (rows) hipLaunchKernelGGL((bspline_tile_kernel<T, true, W>), grid, block, lds, stream, p, 1);
+            else hipLaunchKernelGGL((bspline_tile_kernel<T, false, W>), grid, block, lds, stream, p, static_cast<i32>(tiles_c));
+        };
+        if (width == 32) launch(std::integral_constant<i32, 32>{});
+        else if (width == 16) launch(std::integral_constant<i32, 16>{});
+        else launch(std::integral_constant<i32, 8>{});
+    } else if (rows) {
         const i64 blocks = (p.lines + 63) / 64;
         hipLaunchKernelGGL((bspline_rows_kernel<T>), dim3(static_cast<u32>(blocks)), dim3(64), 0, stream, p);
     } else {

@@ -122,3 +122,23 @@ def test_prefilter_256_cube_interpolates_its_samples():
     rec = _spline_at_samples(c.double())
     err = (rec - v.double()).abs().max().item()
     assert err < 2e-5 * v.abs().max().item(), err
+
+
+@pytest.mark.parametrize("dt,shape", [
+    ("f32", (1, 3, 5, 2047)), ("f32", (1, 3, 5, 2049)),         # the longest rows in LDS, and past them
+    ("f64", (1, 2, 1030, 9)), ("c64", (1, 515, 3, 9)),         # columns and pages of 16 and 8 neighbours
+    ("c32", (2, 33, 65, 31)), ("f32", (1, 17, 224, 224)),       # ends of tiles; 50,176 lines along z: a lane per line
+    ("f32", (3, 1, 1, 1)), ("c32", (1, 2, 13, 17)),
+])
+def test_prefilter_tiles_match_the_oracle(dt, shape):
+    """Lines in LDS, in every tile width, at the ends of tiles and on both sides of the rules: noa's recursion in noa's
+    order, bit for bit; and in place."""
+    print(f"case bspline tiles {dt} {shape}", flush=True)
+    x = _random(shape, DTYPES[dt][0], 900 + sum(shape))
+    want = _expected(x)
+    xin = torch.from_numpy(x).to(DEV)
+    out = torch.empty_like(xin)
+    nx().cubic_bspline_prefilter(xin, out)
+    nx().cubic_bspline_prefilter(xin, xin)
+    np.testing.assert_array_equal(_cpu(out), want)
+    np.testing.assert_array_equal(_cpu(xin), want)
