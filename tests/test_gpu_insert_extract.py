@@ -121,6 +121,54 @@ def test_insert_extract_matches_the_oracle(remap, tin, tout, weights, interp, ex
     close(got_w, want_w, rel=tol, elem=tol * 100)
 
 
+@pytest.mark.parametrize("n,n_out,b_in,b_out,weights,centered,sinc", [
+    (6, 6, 1, 1, False, True, None),               # smaller than a tile, one slice
+    (16, 16, 65, 3, True, True, (0.06, 0.13)),     # the first size with two tile columns; two scans of slices
+    (33, 33, 64, 2, True, False, None),            # odd, an odd number of tiles in y, one full scan
+    (40, 25, 70, 5, True, False, (0.05, 0.08)),    # output slices of another size
+    (46, 46, 129, 4, False, True, (0.02, 0.3)),    # an even number of tiles in y, three scans, wide window
+])
+def test_pipelined_candidates_match_the_oracle(n, n_out, b_in, b_out, weights, centered, sinc):
+    """Contiguous and padded/transposed inputs give the same bits, and the oracle's values and non-finite pixels.
+
+    The window polynomial is within 4e-7 of the window, which the weights and values scale with, and the sums of up
+    to 129 terms run in the oracle's order: 1e-6 relative L2 holds the polynomial and the sine of another library.
+    """
+    print(f"case insert_extract pipelined n={n}->{n_out} b={b_in}->{b_out} w={weights} {centered} {sinc}", flush=True)
+    rng = np.random.default_rng(1000 * n + b_in)
+    remap = "hc2hc" if centered else "h2h"
+    slices = random_spectrum((b_in, 1, n, n // 2 + 1), rng)
+    slices[b_in // 2, 0, 0, -1] = np.nan           # the last column and the first row: a corner of the buffer
+    slices[b_in - 1, 0, -1, 0] = np.inf
+    w_in = rng.uniform(0.1, 2, (b_in, 1, n, n // 2 + 1)).astype(np.float32) if weights else None
+    rot_in, rot_out = random_rotations(b_in, rng), random_rotations(b_out, rng)
+    shape_out = (b_out, 1, n_out, n_out // 2 + 1)
+    want, want_w = np.zeros(shape_out, np.complex64), np.zeros(shape_out, np.float32)
+    kw = {} if sinc is None else dict(input_fftfreq_sinc=sinc[0], input_fftfreq_blackman=sinc[1])
+    with np.errstate(invalid="ignore"):
+        O.insert_and_extract_central_slices_3d(remap, slices, w_in, (b_in, 1, n, n), want, want_w,
+                                               (b_out, 1, n_out, n_out), None, rot_in, None, rot_out, **kw)
+    padded = torch.full((b_in, 1, n + 2, n // 2 + 4), float("nan"), dtype=torch.complex64, device=DEV)
+    padded[:, :, 1:-1, 2:-1] = to_dev(slices)
+    w_strided = None if w_in is None else to_dev(w_in).transpose(2, 3).contiguous().transpose(2, 3)
+    results = []
+    for src, w in ((to_dev(slices), None if w_in is None else to_dev(w_in)), (padded[:, :, 1:-1, 2:-1], w_strided)):
+        out = torch.zeros(shape_out, dtype=torch.complex64, device=DEV)
+        out_w = torch.zeros(shape_out, dtype=torch.float32, device=DEV)
+        opts = nx().InsertAndExtractCentralSlicesOptions(
+            **({} if sinc is None else dict(input_windowed_sinc=nx().WindowedSinc(*sinc))))
+        nx().insert_and_extract_central_slices_3d(remap, src, w, (b_in, 1, n, n), out, out_w,
+                                                  (b_out, 1, n_out, n_out), None, to_dev(rot_in), None,
+                                                  to_dev(rot_out), opts)
+        results.append((cpu(out), cpu(out_w)))
+    (got, got_w), (strided, strided_w) = results
+    assert np.array_equal(got.view(np.uint32), strided.view(np.uint32)) and np.array_equal(got_w, strided_w)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    finite = np.isfinite(want)
+    close(got[finite], want[finite])
+    close(got_w, want_w)
+
+
 def test_culling_keeps_every_contribution_with_the_default_window():
     """Many slices and the narrowest window (1/n): the tile culling must not drop any pixel's contribution."""
     print("case insert_extract culling n=64 b_in=300", flush=True)
