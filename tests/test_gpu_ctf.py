@@ -117,6 +117,39 @@ def test_fused_weighted_equals_the_two_calls(remap):
     assert rel_l2(cpu(v1), want_v) <= 1e-5 and rel_l2(cpu(w1), want_w) <= 1e-5
 
 
+@pytest.mark.parametrize("b,h,w", [(1, 2, 2), (70, 3, 4), (300, 2, 3), (5, 33, 62), (3, 129, 254), (130, 2, 9)])
+@pytest.mark.parametrize("batched", [True, False])
+def test_elements_of_many_images_per_wave(b, h, w, batched):
+    """Images smaller than a wave, rows of two elements, waves and blocks that end within an image, the axes and the
+    diagonals, and astigmatism angles of several turns.
+
+    Half the waves' images are strongly astigmatic (1 um at up to 0.25 / A^2 and 0.0197 A: 150 rad), whose cosine is
+    right to about 4 roundings of 6e-8 here and in the oracle: 8 x 6e-8 x 150 = 7e-5 per element.
+    """
+    print(f"case ctf images {b}x{h}x{w} batched={batched}", flush=True)
+    rng = np.random.default_rng(1000 * b + h)
+    ctfs = [sig().CTFAnisotropic((1.5, 1.45), (rng.uniform(0.5, 3.0), (i % 2) * rng.uniform(-1, 1), rng.uniform(-10, 10)),
+                                 300, 0.07, 2.7, bfactor=-20.0 * (i % 3), dtype=np.float32) for i in range(b)]
+    arg = ctfs if batched else ctfs[0]
+    raw = [c.to_bytes() for c in ctfs] if batched else ctfs[0].to_bytes()
+    shape, half = (b, 1, h, w), (b, 1, h, w // 2 + 1)
+    x = random_spectrum(half, rng)
+    want_v, want_w = np.zeros(half, np.complex64), np.zeros(half, np.float32)
+    O.ctf_anisotropic_2d("hc2h", x, want_v, shape, raw)
+    O.ctf_anisotropic_2d("hc2h", None, want_w, shape, raw, ctf_squared=True)
+    v1 = torch.full(half, float("nan"), dtype=torch.complex64, device=DEV)
+    w1 = torch.full(half, float("nan"), dtype=torch.float32, device=DEV)
+    sig().ctf_anisotropic_weighted("hc2h", to_dev(x), v1, w1, shape, arg)
+    v2, w2 = torch.empty_like(v1), torch.empty_like(w1)
+    sig().ctf_anisotropic("hc2h", to_dev(x), v2, shape, arg)
+    sig().ctf_anisotropic("hc2h", None, w2, shape, arg, sig().CTFOptions(ctf_squared=True))
+    torch.cuda.synchronize()
+    assert torch.equal(v1, v2) and torch.equal(w1, w2)
+    scale = max(1.0, float(np.abs(x).max()))
+    assert float(np.abs(cpu(v1) - want_v).max()) <= 1e-4 * scale
+    assert float(np.abs(cpu(w1) - want_w).max()) <= 2e-4      # (c + d)^2 - c^2 <= 2 d for |c| <= 1
+
+
 def test_ctf_in_place_and_errors():
     b, h, w = 2, 32, 32
     ctfs = _ctfs(b)

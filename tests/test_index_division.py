@@ -1,5 +1,6 @@
-"""The division of a frequency index by the box size in the rasterisation: a product with the rounded reciprocal and one
-Newton step, in fused multiply-adds, rounds like the division for every index and size it is used for."""
+"""The divisions of indices that the kernels replace by products: a frequency index by the box size (the rounded
+reciprocal and one Newton step, in fused multiply-adds, rounds like the division for every index and size it is used
+for) and an element index by a row length (a 32-bit multiplier and a shift)."""
 import numpy as np
 import pytest
 
@@ -16,3 +17,18 @@ def test_newton_step_rounds_like_the_division(sizes):
         assert (r.astype(np.float32) == r).all()
         got = (q.astype(np.float64) + r * np.float64(inv)).astype(np.float32)
         assert (got == i / np.float32(n)).all()
+
+
+def test_element_index_quotient_is_exact():
+    sizes = list(range(1, 2050)) + [4097, 65535, 65536, 65537, 2**30 - 1, 2**30, 2**30 + 1, 2**31 - 1]
+    rng = np.random.default_rng(0)
+    for d in sizes:
+        shift = 31 + (d - 1).bit_length()
+        mul = -(-(1 << shift) // d)
+        assert mul < 1 << 32
+        # The error grows with the index, so the last multiples below 2^31 and the index before each decide.
+        last = (2**31 - 1) // d
+        multiples = np.concatenate([np.arange(max(0, last - 64), last + 1), rng.integers(0, last + 1, 64)]) * d
+        t = np.concatenate([multiples, multiples - 1, [2**31 - 1]])
+        t = t[t >= 0].astype(np.uint64)
+        assert ((t * np.uint64(mul)) >> np.uint64(shift) == t // np.uint64(d)).all(), d
