@@ -7,9 +7,10 @@
 //
 // The recursion is sequential along a line, so one lane owns one line, with noa's expressions in noa's order
 // (bit-identical to the CPU path). What differs from a lane-per-line loop over memory is the access pattern:
-//  - lines along x that fit in LDS (up to 2,048 samples of 4 bytes), and along y and z where there are few: a workgroup copies a tile of whole lines into LDS with all of
-//    its lanes, one lane per line runs both recursions there, and the workgroup stores the tile: each pass reads and
-//    writes the array once, with all loads of a tile in flight (bspline_tile_kernel);
+//  - lines along x that fit in LDS (up to 2,048 samples of 4 bytes), and along y and z where there are few: a
+//    workgroup copies a tile of whole lines into LDS with all of its lanes, one lane per line runs both recursions
+//    there, and the workgroup stores the tile: each pass reads and writes the array once, with all loads of a tile in
+//    flight (bspline_tile_kernel);
 //  - other lines along y and z: the 64 lanes of a wave own 64 neighbouring x, so every step of the recursion is one
 //    coalesced 64-element access; steps are loaded in batches of 16, the next batch in flight while the current
 //    one's dependent arithmetic runs;
