@@ -1290,6 +1290,19 @@ struct Plan {
 // expected passing (sub-brick, slice) pairs fill about this many items (a few per resident wave of the GPU), so that
 // calls of a few hundred or thousand slices keep every CU busy instead of a few long items.
 constexpr double PLAN_MIN_ITEMS = 4096;
+
+// Most slices per work item where the active sub-bricks leave resident waves (12 on each of 256 CUs) without one: the
+// slices are cut into as many segments as fill them, of at least 8 slices. The longest item, up to all slices where a
+// tilt series crosses its axis, bounds such a call (one segment and cut: 41 tilts at 64^3 81 and 52 us, 61 at 128^3 169
+// and 82 us, at 150^3 188 and 112 us; uniform poses 57 and 48, 74 and 65, 77 and 67 us). With more sub-bricks than half
+// the waves the partial sums cost uniform poses more (41 at 192^3 in two segments: 70 and 91 us).
+// Only for the default item size: a size from the tuning table stays as it is.
+i32 few_bricks_span(i32 most, i32 n_slices, i64 bricks) {
+    constexpr i64 WAVES = 12 * 256;
+    if (bricks < 1 || 2 * bricks > WAVES) return most;
+    const i32 segments = static_cast<i32>(WAVES / bricks);
+    return std::min(most, std::max(8, (n_slices + segments - 1) / segments));
+}
 using PlanKey = std::tuple<int, i32, i32, i32, i64, i64, i64, double, bool, i32, double, i32, i32, i32, double, int, i32>;
 std::mutex g_plan_mutex;
 std::map<PlanKey, Plan> g_plans;
@@ -1374,6 +1387,7 @@ int make_plan(int device, const i32 grid[3], const i64 target[3], double cutoff,
         for (const Active& a : active) total += a.expected;
         per_item = std::min(-list_target, std::max(16.0, total / PLAN_MIN_ITEMS));
     }
+    if (max_span < 0) max_span = few_bricks_span(-max_span, n_slices, static_cast<i64>(active.size()));
     for (const Active& a : active) {
                 const i32 brick = a.brick;
                 const double expected = a.expected;
@@ -1802,7 +1816,8 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                                      scratch == nullptr, planp, err, kc.order,
                                      scratch != nullptr || kc.order == 3 ? 0
                                      : kc.max_span >= 0                  ? kc.max_span
-                                                                         : default_span(plan_slices));
+                                     : kc.list_target > 0                ? default_span(plan_slices)
+                                                                         : -default_span(plan_slices));
             if (st != NOA_HIP_OK) return st;
             // Pose-adaptive plan (item order 3; not for the allocation-free entry point): the passing slices of each
             // active sub-brick are counted on the device, and the segments are cut from the counts.

@@ -162,6 +162,22 @@ def test_slab_adds_to_the_volume_and_leaves_voxels_beyond_the_cutoff():
     np.testing.assert_array_equal(got[outside], start[outside])
 
 
+@pytest.mark.parametrize("n,b", [(16, 9), (33, 8), (64, 17), (150, 61)])
+def test_segments_of_boxes_with_few_sub_bricks(monkeypatch, n, b):
+    """Small boxes cut into segments of at least 8 slices, the last one shorter, give the sums of whole items (another
+    order of the sums: 1e-6)."""
+    print(f"case few sub-bricks n={n} b={b}", flush=True)
+    rng = np.random.default_rng(n + b)
+    sl = random_spectrum((b, 1, n, n // 2 + 1), rng)
+    w = rng.uniform(0.1, 1.0, sl.shape).astype(np.float32)
+    inv = np.ascontiguousarray(np.transpose(random_rotations(b, rng), (0, 2, 1)))
+    args = ("h2h", dev(sl), dev(w), (b, 1, n, n), n, dev(inv), torch.complex64)
+    got_v, got_w = run_gpu(*args)
+    monkeypatch.setenv("NOA_HIP_INSERT_SPAN", "0")
+    want_v, want_w = run_gpu(*args)
+    assert rel_l2(got_v, want_v) < 1e-6 and rel_l2(got_w, want_w) < 1e-6
+
+
 @pytest.mark.parametrize("n,remap,sdt,odt,weights", [
     (33, "h2h", np.complex64, np.complex64, True),        # the smallest odd size: a sub-brick across the wrap
     (40, "hc2h", np.complex64, np.float32, False),        # n/2 not a multiple of a sub-brick
