@@ -1,5 +1,5 @@
-// Taps of 2D interpolations of slices read through buffer resources, and the polynomial window: shared by the culled
-// insertion kernels and the virtual volume.
+// Taps of 2D interpolations of slices read through buffer resources, shared by the culled insertion kernels and the
+// virtual volume, and the culled kernels' polynomial window.
 #pragma once
 
 #include "common.hpp"
