@@ -431,7 +431,7 @@ int pass(bool rows, const T* in, const i64 in_s[3], i64 in_step, T* out, const i
     const size_t lds = static_cast<size_t>(width * pitch) * sizeof(T);
     const i64 tiles_c = (n2 + width - 1) / width;
     const i64 tiles = rows ? (p.lines + width - 1) / width : n0 * n1 * tiles_c;
-    if (lds <= TILE_LDS && tiles <= 0x7fffffffLL && (rows || p.lines < TILE_MAX_LINES)) {
+    if (lds <= TILE_LDS && tiles * TILE_LANES <= MAX_LANES && (rows || p.lines < TILE_MAX_LINES)) {
         auto launch = [&](auto w) {
             constexpr i32 W = decltype(w)::value;
             const dim3 grid(static_cast<u32>(tiles)), block(TILE_LANES);

@@ -718,7 +718,7 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err) {
     const i64 n_slices = d.out_shape[0];
     const i64 blocks = n_slices * p.tiles;
     if (blocks == 0) return NOA_HIP_OK;
-    if (blocks > 0x7fffffffLL) { err = "too many slices for one launch"; return NOA_HIP_ERROR_UNSUPPORTED; }
+    if (blocks * 256 > MAX_LANES) { err = "too many slices for one launch"; return NOA_HIP_ERROR_UNSUPPORTED; }
 
     const dim3 grid(static_cast<unsigned>(blocks)), block(256);
     // c32 volumes and the 16-bit pair storages (FP32 math after the load, as in the general kernel).
@@ -750,7 +750,7 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err) {
                 tiled = cubic && nn >= 16 && nn <= 1000 && static_cast<double>(cutoff) <= 0.5 && p.os_x == 1 &&
                         p.rot.kind == NOA_HIP_MAT33_F32 && stored_elems < 0x7fffffffLL;
             const i64 tiles_px = (p.pixels + 1023) / 1024;   // outside kernel: 1024 pixels per workgroup
-            if (tiled && n_slices * tiles_px <= 0x7fffffffLL) {
+            if (tiled && n_slices * tiles_px * 256 <= MAX_LANES) {
                 int device = 0;
                 (void)hipGetDevice(&device);
                 // Plans are kept per slice count rounded up to m * 2^k, 8 <= m < 16 (items are clamped to the
@@ -822,9 +822,9 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err) {
             // and 1.09 ms, 1,000 of 250^2 0.27 and 0.31, 500 of 384^2 from the row-major volume 0.46 and 0.60, 500 of
             // 180^2 (8 % more) 84 and 82 us, 3,000 of 40^2 (52 % more) 40 and 37 us.
             const i64 covered = static_cast<i64>(pr) * pc * 64 * NPATCH + (last_column ? p.slice_h : 0);
-            bool patch = n_slices * patch_tiles <= 0x7fffffffLL && 8 * covered <= 9 * static_cast<i64>(p.pixels);
+            bool patch = n_slices * patch_tiles * 256 <= MAX_LANES && 8 * covered <= 9 * static_cast<i64>(p.pixels);
             if (const char* pe = std::getenv("NOA_HIP_EXTRACT_PATCH"))
-                patch = pe[0] != '0' && n_slices * patch_tiles <= 0x7fffffffLL;
+                patch = pe[0] != '0' && n_slices * patch_tiles * 256 <= MAX_LANES;
             auto launch = [&](ExtractParams<C> q, auto from_brick) {
                 constexpr bool B = decltype(from_brick)::value;
                 if (patch) {

@@ -397,7 +397,7 @@ int run(const InsertExtractDesc& d, hipStream_t stream, std::string& err) {
 
     const i64 tiles = static_cast<i64>(p.tiles_y) * p.tiles_x * p.n_out;
     const i64 blocks = (tiles + IE_WAVES - 1) / IE_WAVES;
-    if (blocks > 0x7fffffff) { err = "insert_and_extract: too many output slices"; return NOA_HIP_ERROR_UNSUPPORTED; }
+    if (blocks * IE_TILE * IE_TILE * IE_WAVES > MAX_LANES) { err = "insert_and_extract: too many output slices"; return NOA_HIP_ERROR_UNSUPPORTED; }
     const dim3 grid(static_cast<u32>(blocks)), block(IE_TILE * IE_TILE * IE_WAVES);
     p.interp_mode = d.interp;
     auto launch = [&](auto interp_tag) {

@@ -15,6 +15,10 @@ namespace noa_hip {
 using i32 = int32_t;
 using i64 = int64_t;
 
+// Most lanes of one launch along x: the dispatch packet counts them in 32 bits, and a larger launch runs a part of its
+// workgroups without reporting an error.
+constexpr i64 MAX_LANES = 0xffffffffLL;
+
 // A flattened strided array: slices use (batch, y, x) strides, volumes (z, y, x) strides.
 struct Arr {
     void* data{};

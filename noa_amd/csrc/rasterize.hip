@@ -721,7 +721,7 @@ int run_tiles(const ProjectDesc& d, const RasterParams<C, In, Out, W>& p, hipStr
     // 256^2 64-128, 4,096 of 256^2 128.
     const double best = static_cast<double>(nn) * std::sqrt(static_cast<double>(n_slices)) / 110.0;
     i64 per_item = pe ? std::max(1, std::atoi(pe)) : std::min<i64>(256, std::max<i64>(2, std::llround(best)));
-    const i64 most = 0x7fffffffLL / plan.n_boxes;              // parts of a box that the grid can hold
+    const i64 most = MAX_LANES / 64 / plan.n_boxes;             // parts of a box that the grid can hold
     per_item = std::max(per_item, (n_slices + most - 1) / most);
     const i64 max_items = (n_slices + per_item - 1) / per_item;
     RasterBoxParams<In, Out> q{};
@@ -809,7 +809,7 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err) {
         const int st = run_tiles<In, Out>(d, p, stream, err);
         if (st != NOT_TILED) return st;
     }
-    if (blocks > 0x7fffffffLL) { err = "too many slices for one launch"; return NOA_HIP_ERROR_UNSUPPORTED; }
+    if (blocks * 256 > MAX_LANES) { err = "too many slices for one launch"; return NOA_HIP_ERROR_UNSUPPORTED; }
     hipLaunchKernelGGL((rasterize_kernel<C, In, Out, W>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, p);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) { err = std::string("kernel launch failed: ") + hipGetErrorString(e); return NOA_HIP_ERROR_RUNTIME; }

@@ -142,3 +142,18 @@ def test_prefilter_tiles_match_the_oracle(dt, shape):
     nx().cubic_bspline_prefilter(xin, xin)
     np.testing.assert_array_equal(_cpu(out), want)
     np.testing.assert_array_equal(_cpu(xin), want)
+
+
+def test_prefilter_more_lines_than_a_launch_of_whole_line_tiles():
+    """More than 2^24 tiles of 32 short lines (2^32 lanes, which one launch does not hold): the rows go to the kernel with
+    a line per lane. Every line against the same lines filtered in a small call, bit for bit."""
+    print("case bspline 2^29 lines", flush=True)
+    lines, part = (1 << 29) + 96, 1 << 16
+    few = torch.randn((part, 1, 1, 2), device=DEV, generator=torch.Generator(device=DEV).manual_seed(6))
+    want = torch.empty_like(few)
+    nx().cubic_bspline_prefilter(few, want)
+    x = few.expand(lines // part + 1, part, 1, 1, 2).reshape(-1, 1, 1, 2)[:lines].contiguous()
+    nx().cubic_bspline_prefilter(x, x)
+    whole = x[:lines // part * part].reshape(-1, part, 2)
+    assert bool((whole == want.reshape(1, part, 2)).all())
+    assert torch.equal(x[lines // part * part:], want[:lines % part])
