@@ -5,16 +5,17 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <list>
 
 namespace noa_hip {
 
 // A device buffer for the work enqueued on `stream` until this object is destroyed. data() is null where no memory was
-// left. Freeing a stream-ordered allocation waits for the stream here (hipFreeAsync returned after the kernel that used
-// the buffer: the host then enqueues nothing while the GPU runs), and allocating takes 0.1 to 0.4 ms once the runtime has
-// given the memory back, so the buffers are kept: at most WORKSPACE_LIMIT bytes per device, the ones of other streams
-// given back first when that is reached; larger buffers, and all of them while a stream is being captured, are allocated
-// and freed in stream order. Safe from several threads: a buffer belongs to one call at a time, and a call waits, on its
-// stream, for the event recorded behind the buffer's last use.
+// left. Allocating takes 0.1 to 0.4 ms once the runtime has given freed memory back, and a free in stream order can hold
+// the host until the stream has caught up, so the buffers are kept: at most WORKSPACE_LIMIT bytes per device, over all
+// streams. When that is reached, the stream's own buffers and those whose last use has ended on the GPU make room, the
+// longest unused first; a buffer still in use by another stream's work is neither taken nor waited for, and the call
+// allocates and frees its own in stream order, as do larger calls and all calls on a stream that is being captured. Safe from several threads: a buffer
+// belongs to one call at a time, and a call waits, on its stream, for the event recorded behind the buffer's last use.
 class CallWorkspace {
 public:
     CallWorkspace() = default;
@@ -28,13 +29,19 @@ public:
     template<class T = void> T* data() const { return static_cast<T*>(m_data); }
     explicit operator bool() const { return m_data != nullptr; }
 
+    struct Kept {
+        void* data;
+        size_t bytes;
+        hipStream_t stream;        // of the last use
+        hipEvent_t event;          // behind it
+    };
+
 private:
-    void release();
+    void release() noexcept;
 
     void* m_data{};
-    size_t m_bytes{};
     hipStream_t m_stream{};
-    hipEvent_t m_event{};      // null: not kept
+    std::list<Kept> m_kept;        // one element, moved from and to the idle buffers; empty: not kept
     int m_device{};
 };
 
