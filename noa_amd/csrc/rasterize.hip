@@ -636,7 +636,8 @@ constexpr int NOT_TILED = -1000;
 
 // The boxes that the cutoff sphere reaches, for one size and cutoff: every pixel inside the cutoff has its floor within
 // [lo - 1, hi + 1] along z and y and [0, n/2] along x. The ones nearest to the origin, which most slices cross, come
-// first. Kept per (device, size, cutoff) for the process lifetime.
+// first. Kept per (device, size, cutoff) for the process lifetime. False where they are not resident and cannot be uploaded:
+// while the stream is captured, which allows neither the allocation nor the copy, or without memory.
 struct BoxPlan {
     i32* boxes{};
     i32 n_boxes{}, nby{}, nbx{}, base{};
@@ -644,14 +645,15 @@ struct BoxPlan {
 std::mutex g_box_mutex;
 std::map<std::tuple<int, i32, double>, BoxPlan> g_box_plans;
 
-int make_box_plan(int device, i32 n, double cutoff, BoxPlan& plan, std::string& err) {
+bool make_box_plan(int device, i32 n, double cutoff, bool captured, BoxPlan& plan) {
     std::lock_guard<std::mutex> lock(g_box_mutex);
     const auto key = std::make_tuple(device, n, cutoff);
     const auto it = g_box_plans.find(key);
     if (it != g_box_plans.end()) {
         plan = it->second;
-        return NOA_HIP_OK;
+        return true;
     }
+    if (captured) return false;
     BoxPlan pl;
     const i32 lo = -n / 2, hi = (n - 1) / 2;
     pl.base = lo - 1;
@@ -680,16 +682,18 @@ int make_box_plan(int device, i32 n, double cutoff, BoxPlan& plan, std::string& 
     if (!boxes.empty() &&
         (hipMalloc(&pl.boxes, boxes.size() * sizeof(i32)) != hipSuccess ||
          hipMemcpy(pl.boxes, boxes.data(), boxes.size() * sizeof(i32), hipMemcpyHostToDevice) != hipSuccess)) {
-        err = "rasterize: could not upload the boxes";
-        return NOA_HIP_ERROR_RUNTIME;
+        if (pl.boxes) (void)hipFree(pl.boxes);
+        (void)hipGetLastError();
+        return false;
     }
     g_box_plans[key] = pl;
     plan = pl;
-    return NOA_HIP_OK;
+    return true;
 }
 
 // The boxed path (rasterize_box_kernel) where it applies: cubic volume and slices, no target shape, no Ewald sphere,
-// cutoff <= 0.5, Mat33<f32> or Quaternion<f32> rotations, Mat22 inverse scalings or none. It takes every such call: one
+// cutoff <= 0.5, Mat33<f32> or Quaternion<f32> rotations, Mat22 inverse scalings or none. It takes every such call but the
+// first one of a size and cutoff where that one is captured (the lane-per-pixel kernel needs nothing resident): one
 // slice of 256^2 into its volume 38 us against 57 us with a lane per pixel, 8 slices of 64^2 26 us either way, 41 of
 // 192^2 109 against 665 us, 4,096 of 256^2 2.4 against 112 ms (with the clearing of the volume, 24 us at 256^3).
 // NOA_HIP_RASTERIZE_LAYOUT=direct selects the lane-per-pixel kernel; NOA_HIP_RASTERIZE_PAIRS sets the crossing slices
@@ -709,9 +713,11 @@ int run_tiles(const ProjectDesc& d, const RasterParams<C, In, Out, W>& p, hipStr
     if (env && std::strcmp(env, "tiles") != 0) return NOT_TILED;
     int device = 0;
     (void)hipGetDevice(&device);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(stream, &capture);
+    const bool captured = capture != hipStreamCaptureStatusNone;
     BoxPlan plan;
-    const int st = make_box_plan(device, static_cast<i32>(nn), std::max(d.cutoff, 0.0), plan, err);
-    if (st != NOA_HIP_OK) return st;
+    if (!make_box_plan(device, static_cast<i32>(nn), std::max(d.cutoff, 0.0), captured, plan)) return NOT_TILED;
     if (plan.n_boxes == 0) return NOA_HIP_OK;
     const char* pe = std::getenv("NOA_HIP_RASTERIZE_PAIRS");
     // Crossing slices per item. An item costs its flush (9 x 9 x 17 atomics, most of them non-zero) and its slices, one
@@ -750,10 +756,8 @@ int run_tiles(const ProjectDesc& d, const RasterParams<C, In, Out, W>& p, hipStr
     q.slice_centered = p.slices_centered;
     const bool gen = q.scaled || p.rot.kind == NOA_HIP_QUAT_F32;
     const dim3 boxes(static_cast<u32>(plan.n_boxes * max_items));
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    (void)hipStreamIsCapturing(stream, &capture);
     CallWorkspace starts;
-    if (n_slices > 64 && capture == hipStreamCaptureStatusNone)
+    if (n_slices > 64 && !captured)
         starts = CallWorkspace(static_cast<size_t>(plan.n_boxes) * max_items * sizeof(i32), stream);
     q.starts = starts.data<i32>();
     if (q.starts)

@@ -318,3 +318,34 @@ def test_boxes_match_the_oracle(monkeypatch, n, b, kind, per_item):
             vol.fill_(1)
             graph.replay()
             check()
+
+
+@pytest.mark.parametrize("b", [7, 100])
+def test_first_call_of_a_size_can_be_captured(b, monkeypatch):
+    """A size and cutoff that no call had before, in a graph: the boxes are not resident and nothing may be uploaded
+    then, so the lane-per-pixel kernel serves the call. Replays against an eager call, rel-L2 1e-6 (other sums)."""
+    print(f"case rasterize first call captured b={b}", flush=True)
+    monkeypatch.delenv("NOA_HIP_RASTERIZE_LAYOUT", raising=False)
+    n, cutoff = 44, 0.40625 + 0.0001 * b
+    rng = np.random.default_rng(b)
+    sl, rot = dev(random_spectrum((b, 1, n, n // 2 + 1), rng)), nx().Mat33Array(random_rotations(b, rng), DEV)
+    vol = torch.zeros((1, n, n, n // 2 + 1), dtype=torch.complex64, device=DEV)
+    wv = torch.zeros((1, n, n, n // 2 + 1), dtype=torch.float32, device=DEV)
+    opts = nx().RasterizeCentralSlicesOptions(fftfreq_cutoff=cutoff)
+
+    def call():
+        vol.zero_()
+        wv.zero_()
+        nx().rasterize_central_slices_3d("h2h", sl, None, (b, 1, n, n), vol, wv, (1, n, n, n), None, rot, opts)
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    call()
+    torch.cuda.synchronize()
+    want_v, want_w = vol.cpu().numpy(), wv.cpu().numpy()
+    for _ in range(3):
+        vol.fill_(1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(vol.cpu().numpy(), want_v) < 1e-6 and rel_l2(wv.cpu().numpy(), want_w) < 1e-6
