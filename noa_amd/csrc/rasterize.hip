@@ -692,12 +692,17 @@ bool make_box_plan(int device, i32 n, double cutoff, bool captured, BoxPlan& pla
 }
 
 // The boxed path (rasterize_box_kernel) where it applies: cubic volume and slices, no target shape, no Ewald sphere,
-// cutoff <= 0.5, Mat33<f32> or Quaternion<f32> rotations, Mat22 inverse scalings or none. It takes every such call but the
-// first one of a size and cutoff where that one is captured (the lane-per-pixel kernel needs nothing resident): one
-// slice of 256^2 into its volume 38 us against 57 us with a lane per pixel, 8 slices of 64^2 26 us either way, 41 of
-// 192^2 109 against 665 us, 4,096 of 256^2 2.4 against 112 ms (with the clearing of the volume, 24 us at 256^3).
-// NOA_HIP_RASTERIZE_LAYOUT=direct selects the lane-per-pixel kernel; NOA_HIP_RASTERIZE_PAIRS sets the crossing slices
-// per work item.
+// cutoff <= 0.5, Mat33<f32> or Quaternion<f32> rotations, Mat22 inverse scalings or none. Of these calls it takes all but
+//  - the smallest ones, where the lane-per-pixel kernel's single step (about 8 us less than a box's chain of set-up, rows
+//    and queue) counts for more than its atomics: up to 16 slices of fewer than 2^14 pixels together. One call with a
+//    synchronisation behind it, lane per pixel and boxed: 16 slices of 16^2 35 and 41 us, 8 of 32^2 35 and 42, 4 of 64^2 38
+//    and 44, 1 of 128^2 35 and 41; just above the line 8 of 64^2 43 and 43, 2 of 128^2 45 and 42, 16 of 48^2 46 and 44; more
+//    slices meet in the same voxels (41 of 16^2 48 and 41 us);
+//  - the first one of a size and cutoff where that one is captured (the lane-per-pixel kernel needs nothing resident).
+// 41 slices of 192^2 take 109 against 665 us, 4,096 of 256^2 2.4 against 112 ms (with the clearing of the volume, 24 us at
+// 256^3). NOA_HIP_RASTERIZE_LAYOUT=direct selects the lane-per-pixel kernel, =tiles the boxed one where it applies;
+// NOA_HIP_RASTERIZE_PAIRS sets the crossing slices per work item.
+constexpr i64 RB_FEW_SLICES = 16, RB_FEW_PIXELS = 1 << 14;
 template<class In, class Out, class C, class W>
 int run_tiles(const ProjectDesc& d, const RasterParams<C, In, Out, W>& p, hipStream_t stream, std::string& err) {
     const i64 nn = p.grid[0], n_slices = d.in_shape[0];
@@ -711,6 +716,7 @@ int run_tiles(const ProjectDesc& d, const RasterParams<C, In, Out, W>& p, hipStr
     if (!eligible) return NOT_TILED;
     const char* env = std::getenv("NOA_HIP_RASTERIZE_LAYOUT");
     if (env && std::strcmp(env, "tiles") != 0) return NOT_TILED;
+    if (!env && n_slices <= RB_FEW_SLICES && n_slices * p.pixels < RB_FEW_PIXELS) return NOT_TILED;
     int device = 0;
     (void)hipGetDevice(&device);
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;

@@ -169,12 +169,13 @@ def test_tiles_with_a_degenerate_transform(monkeypatch):
 
 
 def test_default_selection_by_slice_count(monkeypatch):
-    """Without the switch, 64 slices or more take the tiled path and fewer the direct kernel; both agree."""
+    """Without the switch, calls of at most 16 slices with fewer than 2^14 pixels take the direct kernel and larger ones the
+    boxes; on both sides of the line (7 slices of 64^2 have 14,784 pixels, 8 have 16,896) and well above it."""
     print("case rasterize default selection", flush=True)
     monkeypatch.delenv("NOA_HIP_RASTERIZE_LAYOUT", raising=False)
     rng = np.random.default_rng(1750)
     n = 64
-    for b in (63, 64):
+    for b in (7, 8, 17, 64):
         sl = random_spectrum((b, 1, n, n // 2 + 1), rng)
         rot = random_rotations(b, rng)
         vol = torch.zeros((1, n, n, n // 2 + 1), dtype=torch.complex64, device=DEV)
@@ -266,7 +267,7 @@ def test_boxes_match_the_oracle(monkeypatch, n, b, kind, per_item):
     few hundred FP32 terms in another order: 2^-24 times the square root of their number, about 1e-6 at the worst)."""
     print(f"case rasterize boxes n={n} b={b} {kind} per_item={per_item}", flush=True)
     rng = np.random.default_rng(2000 + n + b)
-    monkeypatch.delenv("NOA_HIP_RASTERIZE_LAYOUT", raising=False)
+    monkeypatch.setenv("NOA_HIP_RASTERIZE_LAYOUT", "tiles")      # also the calls that the default leaves to a lane per pixel
     if per_item is not None:
         monkeypatch.setenv("NOA_HIP_RASTERIZE_PAIRS", str(per_item))
     wr = n // 2 + 1
@@ -297,7 +298,7 @@ def test_boxes_match_the_oracle(monkeypatch, n, b, kind, per_item):
         monkeypatch.setenv("NOA_HIP_RASTERIZE_LAYOUT", "direct")
         call()
         want_v, want_w = vol.clone(), wv.clone()
-        monkeypatch.delenv("NOA_HIP_RASTERIZE_LAYOUT")
+        monkeypatch.setenv("NOA_HIP_RASTERIZE_LAYOUT", "tiles")
     else:
         want_v, want_w = np.zeros((1, n, n, wr), sl.dtype), np.zeros((1, n, n, wr), np.float32)
         O.rasterize_central_slices_3d("h2h", sl, w, (b, 1, n, n), want_v, want_w, (1, n, n, n), scale, rot,
