@@ -41,7 +41,7 @@ struct ExtractParams {
     C target[3];
     C slice_f[2];
     i32 slice_h, slice_wr, pixels, tiles, ppt;
-    i32 patch_wgs, patch_pc;            // extract_c32_kernel<PATCH>: workgroups of 8x8 patches per slice, patches per row
+    i32 patch_wgs, patch_pc;            // extract_c32_kernel: workgroups of 8x8 patches per slice, waves per row of them
     float inv_wr;          // 1 / slice_wr (lean kernel's pixel -> row)
     C cutoff_sqd;
     C ews[2];
@@ -248,13 +248,12 @@ __global__ __launch_bounds__(256) void brick_volume_kernel(const S* __restrict__
         if (live[e]) out[first + e * 256u] = v[e];
 }
 
-// PATCH: each wave takes an 8 x 8 patch of pixels (rows y0..y0+7, columns u0..u0+7) instead of 64 consecutive
-// pixels of a row: the patch samples a compact piece of the plane, so each tap load touches fewer cache lines of the
-// volume. Workgroups [0, patch_wgs) of a slice hold four patches each, the last ones of a row or column partly outside
-// the slice; where one column would be left over (wr = 8 k + 1, the half of a size that is a multiple of 16), the next
-// workgroups take it, 256 rows each.
-constexpr i32 NPATCH = 2;              // patches per wave, next to each other along x, their loads in flight together
-template<int SHIFT, bool BRICK, class S, bool PATCH = false>
+// NPATCH > 0: each wave takes NPATCH 8 x 8 patches of pixels (rows y0..y0+7, columns u0..u0+7), next to each other along
+// x and with their loads in flight together, instead of 64 consecutive pixels of a row: the patch samples a compact piece
+// of the plane, so each tap load touches fewer cache lines of the volume. Workgroups [0, patch_wgs) of a slice hold
+// 4 x NPATCH patches each, the last ones of a row or column partly outside the slice; where one column would be left over
+// (wr = 8 k + 1, the half of a size that is a multiple of 16), the next workgroups take it, 256 rows each.
+template<int SHIFT, bool BRICK, class S, i32 NPATCH>
 __global__ __launch_bounds__(256) void extract_c32_kernel(const ExtractParams<float> p) {
     const u32 lb = xcd_swizzle(blockIdx.x, gridDim.x);
     const i32 b = static_cast<i32>(lb / static_cast<u32>(p.tiles));
@@ -273,7 +272,7 @@ __global__ __launch_bounds__(256) void extract_c32_kernel(const ExtractParams<fl
     const S* __restrict__ vol = static_cast<const S*>(p.vol);
     float2* __restrict__ out = static_cast<float2*>(p.out) + static_cast<i64>(b) * p.os_b;
 
-    constexpr i32 MAXP = PATCH ? NPATCH : 4;
+    constexpr i32 MAXP = NPATCH > 0 ? NPATCH : 4;
     Taps3<float2, float> tv[MAXP];
     bool inside[MAXP];
     i32 ys[MAXP], us[MAXP];
@@ -282,7 +281,7 @@ __global__ __launch_bounds__(256) void extract_c32_kernel(const ExtractParams<fl
     for (i32 k = 0; k < MAXP; ++k) {
         bool live;
         i32 y, u;
-        if constexpr (PATCH) {
+        if constexpr (NPATCH > 0) {
             const i32 wave = static_cast<i32>(threadIdx.x) >> 6, lane = static_cast<i32>(threadIdx.x) & 63;
             if (tile < p.patch_wgs) {
                 const i32 q = tile * 4 + wave, pr = q / p.patch_pc, pc = q - pr * p.patch_pc;
@@ -813,34 +812,48 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err) {
             CallWorkspace copy;
             if (bricks) copy = CallWorkspace(static_cast<size_t>(brick_elems) * sizeof(S), stream);
             void* brick = copy.data();
-            // Pixel patches (extract_c32_kernel<PATCH>), four per workgroup.
+            // Pixel patches (extract_c32_kernel), or rows of pixels (0).
             const bool last_column = p.slice_wr % 8 == 1 && p.slice_wr > 1;
-            const i32 pr = (p.slice_h + 7) / 8, pc = ((last_column ? p.slice_wr / 8 : (p.slice_wr + 7) / 8) + NPATCH - 1) / NPATCH;
-            const i32 patch_wgs = (pr * pc + 3) / 4;
-            const i64 patch_tiles = patch_wgs + (last_column ? (p.slice_h + 255) / 256 : 0);
-            // Where the patches cover up to an eighth more than the slice. Patches and rows: 4,096 slices of 256^2 0.95
-            // and 1.09 ms, 1,000 of 250^2 0.27 and 0.31, 500 of 384^2 from the row-major volume 0.46 and 0.60, 500 of
-            // 180^2 (8 % more) 84 and 82 us, 3,000 of 40^2 (52 % more) 40 and 37 us.
-            const i64 covered = static_cast<i64>(pr) * pc * 64 * NPATCH + (last_column ? p.slice_h : 0);
-            bool patch = n_slices * patch_tiles * 256 <= MAX_LANES && 8 * covered <= 9 * static_cast<i64>(p.pixels);
-            if (const char* pe = std::getenv("NOA_HIP_EXTRACT_PATCH"))
-                patch = pe[0] != '0' && n_slices * patch_tiles * 256 <= MAX_LANES;
-            auto launch = [&](ExtractParams<C> q, auto from_brick) {
+            const i32 pr = (p.slice_h + 7) / 8, pc = last_column ? p.slice_wr / 8 : (p.slice_wr + 7) / 8;
+            auto patch_wgs = [&](i32 np) { return (pr * ((pc + np - 1) / np) + 3) / 4; };
+            auto patch_tiles = [&](i32 np) {
+                return static_cast<i64>(patch_wgs(np)) + (last_column ? (p.slice_h + 255) / 256 : 0);
+            };
+            auto covers = [&](i32 np) {                    // pixels of the patches, of `pixels` of the slice
+                return static_cast<i64>(pr) * ((pc + np - 1) / np) * 64 * np + (last_column ? p.slice_h : 0);
+            };
+            // In pairs where they cover up to an eighth more than the slice: 4,096 slices of 256^2 0.95 ms (rows 1.09), 1,000
+            // of 250^2 0.27 (0.31), 500 of 384^2 from the row-major volume 0.46 (0.60); 3e7 pixels of 188^2 (3 % more) 114 us
+            // (127), of 180^2 (8 %) 114 (122), of 148^2 (10 %) 113 (112), of 116^2 (12 %) 107 (104), of 132^2 (23 %) 116
+            // (110), of 100^2 (31 %) 114 (98). One by one where an odd number of them in a row tiles the slice and pairs do
+            // not (widths of 16, 48, 80 and 112): 3e7 pixels of 64 x 48 from 128^3 238 us (rows 303), of 128 x 80 from 160^3
+            // 183 (243). But not with 4, 8 or 12 workgroups to a slice: the four shader engines of an XCD take workgroups in
+            // turn, so each would always get the same part of the slices (96 x 16 from 128^3 331 us, rows 223).
+            i32 patch = 0;
+            if (8 * covers(2) <= 9 * static_cast<i64>(p.pixels)) patch = 2;
+            else if (brick && last_column && covers(1) == p.pixels && (pr * pc) % 4 == 0 &&
+                     (patch_tiles(1) % 4 != 0 || patch_tiles(1) >= 16)) patch = 1;
+            if (const char* pe = std::getenv("NOA_HIP_EXTRACT_PATCH")) patch = pe[0] != '0' ? 2 : 0;
+            if (patch > 0 && n_slices * patch_tiles(patch) * 256 > MAX_LANES) patch = 0;
+            auto launch_as = [&](ExtractParams<C> q, auto from_brick, auto patches) {
                 constexpr bool B = decltype(from_brick)::value;
-                if (patch) {
+                constexpr i32 NP = decltype(patches)::value;
+                dim3 g = grid;
+                if constexpr (NP > 0) {
                     q.ppt = 1;
-                    q.patch_wgs = patch_wgs;
-                    q.patch_pc = pc;
-                    q.tiles = static_cast<i32>(patch_tiles);
-                    const dim3 pgrid(static_cast<u32>(n_slices * patch_tiles));
-                    if (q.shift_mode == 0) hipLaunchKernelGGL((extract_c32_kernel<1, B, S, true>), pgrid, block, 0, stream, q);
-                    else if (q.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, B, S, true>), pgrid, block, 0, stream, q);
-                    else hipLaunchKernelGGL((extract_c32_kernel<0, B, S, true>), pgrid, block, 0, stream, q);
-                } else {
-                    if (q.shift_mode == 0) hipLaunchKernelGGL((extract_c32_kernel<1, B, S, false>), grid, block, 0, stream, q);
-                    else if (q.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, B, S, false>), grid, block, 0, stream, q);
-                    else hipLaunchKernelGGL((extract_c32_kernel<0, B, S, false>), grid, block, 0, stream, q);
+                    q.patch_wgs = patch_wgs(NP);
+                    q.patch_pc = (pc + NP - 1) / NP;
+                    q.tiles = static_cast<i32>(patch_tiles(NP));
+                    g = dim3(static_cast<u32>(n_slices * patch_tiles(NP)));
                 }
+                if (q.shift_mode == 0) hipLaunchKernelGGL((extract_c32_kernel<1, B, S, NP>), g, block, 0, stream, q);
+                else if (q.shift_mode == 2) hipLaunchKernelGGL((extract_c32_kernel<2, B, S, NP>), g, block, 0, stream, q);
+                else hipLaunchKernelGGL((extract_c32_kernel<0, B, S, NP>), g, block, 0, stream, q);
+            };
+            auto launch = [&](const ExtractParams<C>& q, auto from_brick) {
+                if (patch == 2) launch_as(q, from_brick, std::integral_constant<i32, 2>{});
+                else if (patch == 0) launch_as(q, from_brick, std::integral_constant<i32, 0>{});
+                else launch_as(q, std::true_type{}, std::integral_constant<i32, 1>{});
             };
             if (brick) {
                 const BrickLayout L{static_cast<i32>(bz), static_cast<i32>(by)};

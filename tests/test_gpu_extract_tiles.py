@@ -191,3 +191,29 @@ def test_pixel_patches_equal_the_rows(monkeypatch, layout, n, shifts):
         outs.append(out.cpu().numpy())
     assert np.isfinite(outs[0]).all()
     np.testing.assert_array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("n,h,w", [(64, 64, 48), (128, 128, 16), (96, 32, 80), (112, 64, 112)])
+def test_single_patches_equal_the_rows(monkeypatch, n, h, w):
+    """Slices that an odd number of patches in a row tiles exactly: one patch per wave by default, against waves of 64
+    pixels of a row, bit for bit."""
+    print(f"case extract single patches n={n} {h}x{w}", flush=True)
+    rng = np.random.default_rng(700 + n)
+    b, wr = 9, w // 2 + 1
+    volume = dev(random_spectrum((1, n, n, n // 2 + 1), rng))
+    rot = dev(random_rotations(b, rng))
+    sh = dev(rng.uniform(-5, 5, (b, 2)).astype(np.float32))
+    monkeypatch.setenv("NOA_HIP_EXTRACT_LAYOUT", "bricks")
+    outs = []
+    for rows in (False, True):
+        if rows:
+            monkeypatch.setenv("NOA_HIP_EXTRACT_PATCH", "0")
+        else:
+            monkeypatch.delenv("NOA_HIP_EXTRACT_PATCH", raising=False)
+        out = torch.full((2, b, 1, h, wr), float("nan"), dtype=torch.complex64, device=DEV)
+        nx().extract_central_slices_3d("h2hc", volume, None, (1, n, n, n), out[0], None, (b, 1, h, w), None, rot)
+        nx().extract_central_slices_3d_shifted("hc2h", volume, None, (1, n, n, n), out[1], None, (b, 1, h, w), None, rot, sh)
+        torch.cuda.synchronize()
+        outs.append(out.cpu().numpy())
+    assert np.isfinite(outs[0]).all()
+    np.testing.assert_array_equal(outs[0], outs[1])
