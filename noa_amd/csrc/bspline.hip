@@ -7,14 +7,14 @@
 //
 // The recursion is sequential along a line, so one lane owns one line, with noa's expressions in noa's order
 // (bit-identical to the CPU path). What differs from a lane-per-line loop over memory is the access pattern:
-//  - lines along x that fit in LDS (up to 2,048 samples of 4 bytes), and along y and z where there are few: a
-//    workgroup copies a tile of whole lines into LDS with all of its lanes, one lane per line runs both recursions
+//  - lines along x that fit in LDS (up to 2,048 samples of 4 bytes) unless they are short and many, and along y and z
+//    where the GPU holds all of them at once: a workgroup copies a tile of whole lines into LDS with all of its lanes, one lane per line runs both recursions
 //    there, and the workgroup stores the tile: each pass reads and writes the array once, with all loads of a tile in
 //    flight (bspline_tile_kernel);
 //  - other lines along y and z: the 64 lanes of a wave own 64 neighbouring x, so every step of the recursion is one
 //    coalesced 64-element access; steps are loaded in batches of 16, the next batch in flight while the current
 //    one's dependent arithmetic runs;
-//  - longer lines along x (the contiguous axis): a wave owns 64 rows and walks them in 32-column chunks staged through
+//  - other lines along x (the contiguous axis): a wave owns 64 rows and walks them in 32-column chunks staged through
 //    LDS, loaded and stored as whole row segments; the lanes then run their row's recursion out of LDS while the
 //    next chunk's loads are in flight. In both, the anticausal half re-reads the causal half's output.
 #include "common.hpp"
@@ -255,10 +255,6 @@ __global__ __launch_bounds__(256) void bspline_lines_kernel(const LinesParams<T>
 // were no faster.
 constexpr i32 TILE_LANES = 256;
 constexpr size_t TILE_LDS = 64 * 1024;
-// Across the contiguous axis, a lane per line in memory is as fast once there are three waves of lines per CU or more
-// (49,775 lines of 300 samples 48 against 54 us, 65,536 of 256 45 against 43; 720 of 320 and 9,600 of 24, both passes, 40
-// against 17 us).
-constexpr i64 TILE_MAX_LINES = 49152;
 
 template<class T, bool ROWS, i32 WIDTH>
 __global__ __launch_bounds__(TILE_LANES) void bspline_tile_kernel(const LinesParams<T> p, i32 tiles_c) {
@@ -409,6 +405,30 @@ __global__ __launch_bounds__(TILE_LANES) void bspline_tile_kernel(const LinesPar
 
 namespace {
 
+// Whole-line tiles or, for rows, the chunks of bspline_rows_kernel. A tile costs its lines' index arithmetic (about 0.18 us
+// per 1,000 lines once there are many), a row in chunks about 9 us for each chunk after the first, in which the next one is
+// awaited; wider values make both wait for memory sooner. Chunks and tiles: 12,000 rows of 24 f32 9.0 and 7.5 us, 40,000 of
+// 24 9.5 and 12.6, of 33 18 and 12.5, of 128 40 and 23; 100,000 of 64 22 and 29, of 128 44 and 42, of 200 81 and 60;
+// 300,000 of 96 74 and 90, of 200 273 and 170. c32: 40,000 of 64 22 and 25, of 80 42 and 33; 100,000 of 128 75 and 87, of
+// 200 198 and 165. c64: 40,000 of 32 17 and 29, of 33 41 and 29, 300,000 of 33 254 and 217.
+bool tiles_for_rows(i64 lines, i64 n, size_t bytes) {
+    const i64 waits = (n + 31) / 32 - 1;           // bspline_rows_kernel's chunks after the first
+    if (lines <= 12288) return true;
+    if (bytes == 16) return waits >= 1;
+    return waits >= 4 || lines <= (bytes == 4 ? 50000 : 25000) * waits;
+}
+
+// Whole-line tiles across the contiguous axis, or a lane per line in memory: the tiles where the GPU (256 CUs, 160 KB of
+// LDS and 2,048 lanes each) holds all of them at once, or half as many again for 4-byte values and half of them for
+// 16-byte ones. Lines in memory and tiles, with the tiles' number over the ones resident: f32 40,000 of 100 (0.8) 24 and 19 us, 16,000 of 800 (1.3) 115 and 92, 54,300 of
+// 300 (1.6) 52 and 54, 40,000 of 500 (2.5) 78 and 95, 24,000 of 2,000 (5.9) 285 and 544, 40,000 of 8 with 2 neighbours
+// (9.8) 6 and 36; c32 10,000 of 400 (0.9) 71 and 39, 40,000 of 100 (1.4) 26 and 29; c64 4,096 of 64 (0.3) 16 and 11, 16,000
+// of 40 (1.0) 13 and 18.
+bool tiles_for_columns(i64 tiles, size_t lds, size_t bytes) {
+    const i64 resident = 256 * std::min<i64>(2048 / TILE_LANES, (160 * 1024) / static_cast<i64>(lds));
+    return bytes == 4 ? 2 * tiles <= 3 * resident : bytes == 8 ? tiles <= resident : 2 * tiles <= resident;
+}
+
 // Launch of one pass over `lines` lines of `n` samples; the outer dimensions are (lines / (n1 * n2), n1, n2).
 template<class T>
 int pass(bool rows, const T* in, const i64 in_s[3], i64 in_step, T* out, const i64 out_s[3], i64 out_step,
@@ -431,7 +451,8 @@ int pass(bool rows, const T* in, const i64 in_s[3], i64 in_step, T* out, const i
     const size_t lds = static_cast<size_t>(width * pitch) * sizeof(T);
     const i64 tiles_c = (n2 + width - 1) / width;
     const i64 tiles = rows ? (p.lines + width - 1) / width : n0 * n1 * tiles_c;
-    if (lds <= TILE_LDS && tiles * TILE_LANES <= MAX_LANES && (rows || p.lines < TILE_MAX_LINES)) {
+    if (lds <= TILE_LDS && tiles * TILE_LANES <= MAX_LANES &&
+        (rows ? tiles_for_rows(p.lines, n, sizeof(T)) : tiles_for_columns(tiles, lds, sizeof(T)))) {
         auto launch = [&](auto w) {
             constexpr i32 W = decltype(w)::value;
             const dim3 grid(static_cast<u32>(tiles)), block(TILE_LANES);

@@ -127,7 +127,9 @@ def test_prefilter_256_cube_interpolates_its_samples():
 @pytest.mark.parametrize("dt,shape", [
     ("f32", (1, 3, 5, 2047)), ("f32", (1, 3, 5, 2049)),         # the longest rows in LDS, and past them
     ("f64", (1, 2, 1030, 9)), ("c64", (1, 515, 3, 9)),         # columns and pages of 16 and 8 neighbours
-    ("c32", (2, 33, 65, 31)), ("f32", (1, 17, 224, 224)),       # ends of tiles; 50,176 lines along z: a lane per line
+    ("c32", (2, 33, 65, 31)), ("f32", (1, 17, 224, 224)),       # ends of tiles
+    ("f32", (20000, 1, 8, 2)), ("c64", (3000, 1, 8, 3)),        # many short lines: rows in a chunk, a lane per column
+    ("c32", (700, 1, 9, 70)), ("c64", (5200, 1, 3, 33)),        # rows on either side of the rule, a lane per column
     ("f32", (3, 1, 1, 1)), ("c32", (1, 2, 13, 17)),
 ])
 def test_prefilter_tiles_match_the_oracle(dt, shape):
