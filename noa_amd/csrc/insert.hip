@@ -1291,17 +1291,27 @@ struct Plan {
 // calls of a few hundred or thousand slices keep every CU busy instead of a few long items.
 constexpr double PLAN_MIN_ITEMS = 4096;
 
-// Most slices per work item where the active sub-bricks leave resident waves (12 on each of 256 CUs) without one: the
-// slices are cut into as many segments as fill them, of at least 8 slices. The longest item, up to all slices where a
-// tilt series crosses its axis, bounds such a call (one segment and cut: 41 tilts at 64^3 81 and 52 us, 61 at 128^3 169
-// and 82 us, at 150^3 188 and 112 us; uniform poses 57 and 48, 74 and 65, 77 and 67 us). With more sub-bricks than half
-// the waves the partial sums cost uniform poses more (41 at 192^3 in two segments: 70 and 91 us).
-// Only for the default item size: a size from the tuning table stays as it is.
-i32 few_bricks_span(i32 most, i32 n_slices, i64 bricks) {
-    constexpr i64 WAVES = 12 * 256;
-    if (bricks < 1 || 2 * bricks > WAVES) return most;
+// The default bound of the slices per work item, `most` (default_span), where the number of active sub-bricks is far from
+// what it was measured at.
+// Where the sub-bricks leave resident waves (12 on each of 256 CUs) without one: the slices are cut into as many segments as
+// fill them. The longest item, up to all slices where a tilt series crosses its axis, bounds such a call (one segment and
+// cut: 41 tilts at 64^3 81 and 52 us, 61 at 128^3 169 and 82 us, at 150^3 188 and 112 us; uniform poses 57 and 48, 74 and
+// 65, 77 and 67 us). A sub-brick's partial sums are added one after the other in about the time that a slice takes in an
+// item, so no item is shorter than about the square root of the slices, and 8 (16^3 from 5,000 slices: items of 8 slices 803
+// us, of 16 and more 425-437; 32^3 from 1,000: 8 186, 24-32 119; 256^3 to a cutoff of 0.05 from 2,000: 12 246, 24-48 187; 100
+// slices: 8 43-48, 16 51-54). With more sub-bricks than half the waves the partial sums cost uniform poses more (41 at
+// 192^3 in two segments: 70 and 91 us). Only for the default item size: a size from the tuning table stays as it is.
+// Where the sub-bricks are so many (boxes from about 420^3 on) that a segment's partial sums take a quarter of a gigabyte or
+// more: 1,024 slices (at 512^3 the default bound and 1,024: 300 uniform slices 1.18 and 0.87 ms, 1,000 2.68 and 2.00 ms, tilts
+// 3.26 and 3.65 ms; at 640^3 1,000 uniform 4.8 and 3.0 ms, tilts 4.8 and 4.5 ms, and one call with a synchronisation behind it
+// 106 and 3.1 ms, since partial sums of more than the workspaces' bound are allocated anew).
+i32 span_for(i32 most, i32 n_slices, i64 bricks, bool cut_few) {
+    constexpr i64 WAVES = 12 * 256, MANY = 20000;
+    if (bricks > MANY) return 1024;
+    if (!cut_few || bricks < 1 || 2 * bricks > WAVES) return most;
     const i32 segments = static_cast<i32>(WAVES / bricks);
-    return std::min(most, std::max(8, (n_slices + segments - 1) / segments));
+    const i32 shortest = std::max(8, static_cast<i32>(0.8 * std::sqrt(static_cast<double>(n_slices))));
+    return std::min(most, std::max(shortest, (n_slices + segments - 1) / segments));
 }
 using PlanKey = std::tuple<int, i32, i32, i32, i64, i64, i64, double, bool, i32, double, i32, i32, i32, double, int, i32>;
 std::mutex g_plan_mutex;
@@ -1387,7 +1397,7 @@ int make_plan(int device, const i32 grid[3], const i64 target[3], double cutoff,
         for (const Active& a : active) total += a.expected;
         per_item = std::min(-list_target, std::max(16.0, total / PLAN_MIN_ITEMS));
     }
-    if (max_span < 0) max_span = few_bricks_span(-max_span, n_slices, static_cast<i64>(active.size()));
+    if (max_span < 0) max_span = span_for(-max_span, n_slices, static_cast<i64>(active.size()), list_target < 0);
     for (const Active& a : active) {
                 const i32 brick = a.brick;
                 const double expected = a.expected;
@@ -1816,7 +1826,6 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                                      scratch == nullptr, planp, err, kc.order,
                                      scratch != nullptr || kc.order == 3 ? 0
                                      : kc.max_span >= 0                  ? kc.max_span
-                                     : kc.list_target > 0                ? default_span(plan_slices)
                                                                          : -default_span(plan_slices));
             if (st != NOA_HIP_OK) return st;
             // Pose-adaptive plan (item order 3; not for the allocation-free entry point): the passing slices of each

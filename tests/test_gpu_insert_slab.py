@@ -162,10 +162,10 @@ def test_slab_adds_to_the_volume_and_leaves_voxels_beyond_the_cutoff():
     np.testing.assert_array_equal(got[outside], start[outside])
 
 
-@pytest.mark.parametrize("n,b", [(16, 9), (33, 8), (64, 17), (150, 61)])
+@pytest.mark.parametrize("n,b", [(16, 9), (33, 8), (64, 17), (150, 61), (16, 700), (33, 2000)])
 def test_segments_of_boxes_with_few_sub_bricks(monkeypatch, n, b):
-    """Small boxes cut into segments of at least 8 slices, the last one shorter, give the sums of whole items (another
-    order of the sums: 1e-6)."""
+    """Small boxes cut into segments of at least 8 slices (more for many slices), the last one shorter, give the sums of
+    whole items (another order of the sums: 1e-6)."""
     print(f"case few sub-bricks n={n} b={b}", flush=True)
     rng = np.random.default_rng(n + b)
     sl = random_spectrum((b, 1, n, n // 2 + 1), rng)
