@@ -264,10 +264,11 @@ int noa_hip_insert_central_slices_3d(const noa_hip_project_args* args, void* str
 #define NOA_HIP_NOALLOC_SCRATCH_BYTES (32u << 20)
 
 /* No counterpart in noa: noa_hip_insert_central_slices_3d for callers that cannot allocate device memory (code under
- * HIP graph capture, tight serving loops, harnesses that forbid allocation). Same arguments, rules and results
- * (bit-identical). The work plan and the partial sums of split sub-bricks are carved from a
- * static device array of NOA_HIP_NOALLOC_SCRATCH_BYTES per GPU instead of being allocated; a call whose work needs
- * more returns NOA_HIP_ERROR_UNSUPPORTED with the size in noa_hip_last_error() (at 256^3, up to about 5,000 slices
+ * HIP graph capture, tight serving loops, harnesses that forbid allocation). Same arguments and rules; the same results up
+ * to the order in which the sums of a voxel are grouped (its work items have a fixed size and no bound of their slices:
+ * bit-identical with NOA_HIP_INSERT_SPAN=0 and NOA_HIP_INSERT_LIST at the default size, about 1e-7 otherwise). The work plan
+ * and the partial sums of split sub-bricks are carved from a static device array of NOA_HIP_NOALLOC_SCRATCH_BYTES per GPU
+ * instead of being allocated; a call whose work needs more returns NOA_HIP_ERROR_UNSUPPORTED with the size in noa_hip_last_error() (at 256^3, up to about 5,000 slices
  * fit). Every call on a GPU shares that GPU's array: calls that overlap on one GPU (different streams, or
  * threads) race and must be ordered by the caller. A geometry's first call builds its plan on the host. */
 int noa_hip_insert_central_slices_3d_noalloc(const noa_hip_project_args* args, void* stream);

@@ -1651,8 +1651,8 @@ SlabWindow fit_slab_window(float fs, float fb, i32 n) {
     return sw;
 }
 
-// Device scratch of the allocation-free entry point: the work plan, the slice records and the partial sums of one
-// call are carved from it (256-byte aligned pieces) instead of being allocated.
+// Device scratch of the allocation-free entry point: the work plan and the partial sums of one call are carved from it
+// (256-byte aligned pieces) instead of being allocated.
 struct Scratch {
     char* base;
     size_t bytes;
@@ -1908,8 +1908,6 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
             if (plan.n_items == 0) return NOA_HIP_OK;
             const size_t partial_bytes = static_cast<size_t>(plan.n_partials) * p.bd[0] * p.bd[1] * p.apitch * 3 *
                                          sizeof(float);
-            // The allocation-free entry point's limit counts 64 bytes per slice beside the plan and the partial sums.
-            const size_t record_bytes = static_cast<size_t>(p.n_slices) * 64;
             CallWorkspace partial_ws;
             void* partials = nullptr;
             if (scratch) {
@@ -1917,7 +1915,7 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                 auto round = [](size_t b) { return (b + 255) & ~static_cast<size_t>(255); };
                 const size_t items_bytes = round(plan.h_items.size() * sizeof(int4));
                 const size_t reduce_bytes = round(plan.h_reduce.size() * sizeof(int4));
-                const size_t need = items_bytes + reduce_bytes + round(record_bytes) + round(partial_bytes);
+                const size_t need = items_bytes + reduce_bytes + round(partial_bytes);
                 if (need > scratch->bytes) {
                     err = "insert (no allocation): this call needs " + std::to_string(need) +
                           " bytes of scratch, more than the " + std::to_string(scratch->bytes) +

@@ -1,7 +1,7 @@
 """noa_hip_insert_central_slices_3d_noalloc: the insertion without device allocations (static scratch per GPU).
 
-It runs the same plan and kernels as noa_hip_insert_central_slices_3d, so its output must equal that entry point's bit
-for bit. Two calls in a row share the scratch; the second, smaller one must not see the first one's leftovers. A call
+It runs the kernels of noa_hip_insert_central_slices_3d, and with one item size and no bound of an item's slices for both
+its output must equal that entry point's bit for bit. Two calls in a row share the scratch; the second, smaller one must not see the first one's leftovers. A call
 whose work exceeds the scratch is refused before anything is launched.
 """
 import numpy as np
@@ -87,6 +87,18 @@ def test_noalloc_matches_the_allocating_default_plan():
     (ref_v, ref_w), (got_v, got_w) = both("h2h", sl, w, inv, b, n)
     rel = lambda a, r: float(np.linalg.norm(a - r) / np.linalg.norm(r))
     assert rel(got_v, ref_v) < 1e-6 and rel(got_w, ref_w) < 1e-6
+
+
+def test_noalloc_takes_what_fits_the_scratch(monkeypatch):
+    """64^3 with 10,240 slices in items of 141 passing slices: the plan and the partial sums take 31.8 of the scratch's 32
+    MiB, and nothing else is counted."""
+    print("case noalloc 64^3 x 10240 fits", flush=True)
+    monkeypatch.setenv("NOA_HIP_INSERT_SPAN", "0")
+    monkeypatch.setenv("NOA_HIP_INSERT_LIST", "141")
+    n, b = 64, 10240
+    sl, w, inv = inputs(np.random.default_rng(970), n, b)
+    (ref_v, ref_w), (got_v, got_w) = both("h2h", sl, w, inv, b, n)
+    assert np.array_equal(got_v, ref_v) and np.array_equal(got_w, ref_w)
 
 
 def test_noalloc_refuses_work_beyond_the_scratch():
