@@ -126,8 +126,11 @@ __device__ __forceinline__ i32 frequency2index(bool centered, i32 frequency, i32
     return frequency < 0 ? frequency + size : frequency;
 }
 
-// i / n rounded to nearest, for integers |i| <= n < 2^12 with inv_n = 1 / n rounded: one Newton step on the product
-// (the remainder is exact); the same as the division for every such pair.
+// i / n rounded to nearest, for integers |i| <= n < 2^22 with inv_n = 1 / n rounded: one Newton step on the product, the
+// same as the division for every such pair. With u the last place of the product q: two roundings leave q within 2u of
+// i / n, so the remainder is an integer below 2^24 times u, which a fused multiply-add gives exactly, and the sum before
+// its rounding is i / n moved by at most 2u * 2^-24. A quotient is no midpoint between two floats (its numerator would have
+// 25 bits) and is at least u / (2n) > u * 2^-23 away from one, so the moved sum rounds to the same float.
 __device__ __forceinline__ float divide_index(float i, float n, float inv_n) {
     const float q = i * inv_n;
     return fmaf(fmaf(-q, n, i), inv_n, q);

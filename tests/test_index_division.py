@@ -5,6 +5,20 @@ import numpy as np
 import pytest
 
 
+@pytest.mark.parametrize("sizes", [(4096, 4097, 10007, 65535, 1 << 20), ((1 << 21) - 1, (1 << 22) - 3, (1 << 22) - 1)])
+def test_newton_step_rounds_like_the_division_for_long_axes(sizes):
+    """Axes of slices with fewer than 2^21 pixels: up to 2^22. The sum before the last rounding needs up to 72 bits and is
+    formed in 64 here, which moves it by far less than its distance from a midpoint."""
+    for n in sizes:
+        i = np.arange(0, n + 1, dtype=np.float32)
+        inv = np.float32(1) / np.float32(n)
+        q = i * inv
+        r = i.astype(np.longdouble) - q.astype(np.longdouble) * n
+        assert (r.astype(np.float32) == r).all()
+        got = (q.astype(np.longdouble) + r * np.longdouble(inv)).astype(np.float32)
+        assert (got == i / np.float32(n)).all()
+
+
 @pytest.mark.parametrize("sizes", [range(1, 1025), (1536, 2047, 2048, 3000, 4095)])
 def test_newton_step_rounds_like_the_division(sizes):
     for n in sizes:
