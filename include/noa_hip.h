@@ -329,9 +329,9 @@ int noa_hip_volume_blocks(const noa_hip_view* volume, void* blocks, int64_t capa
  *   NOA_HIP_OP_INSERT_BATCH:  values = {workgroups (default 3072); -; -; -}
  * Environment variables (NOA_HIP_EXTRACT_LAYOUT, NOA_HIP_EXTRACT_PAIRS, NOA_HIP_INSERT_KERNEL, NOA_HIP_INSERT_LIST,
  * NOA_HIP_INSERT_PAIRED, NOA_HIP_INSERT_ORDER) override the table; NOA_HIP_INSERT_SPAN sets the most slices of one
- * insertion work item (default a quarter of the slices, between 256 and 1024; 1024 for boxes from about 420^3 on; fewer,
- * down to 8, for boxes of up to about 160^3 where the table does not set the slices per item; 0: no bound; not applied by
- * the allocation-free entry point or item order 3). */
+ * insertion work item (default a quarter of the slices, between 256 and 1024; 1024 for boxes from about 420^3 on, 270^3 on
+ * the one-wave kernel, and for up to 384 slices; fewer, down to 8, for boxes of up to about 160^3 where the table does not
+ * set the slices per item; 0: no bound; not applied by the allocation-free entry point or item order 3). */
 enum {
     NOA_HIP_OP_EXTRACT = 1,
     NOA_HIP_OP_INSERT = 2,

@@ -1303,19 +1303,22 @@ constexpr double PLAN_MIN_ITEMS = 4096;
 // us, of 16 and more 425-437; 32^3 from 1,000: 8 186, 24-32 119; 256^3 to a cutoff of 0.05 from 2,000: 12 246, 24-48 187; 100
 // slices: 8 43-48, 16 51-54). With more sub-bricks than half the waves the partial sums cost uniform poses more (41 at
 // 192^3 in two segments: 70 and 91 us). Only for the default item size: a size from the tuning table stays as it is.
-// Where the sub-bricks are so many (boxes from about 420^3 on) that a segment's partial sums take a quarter of a gigabyte or
-// more: 1,024 slices (at 512^3 the default bound and 1,024: 300 uniform slices 1.18 and 0.87 ms, 1,000 2.68 and 2.00 ms, tilts
-// 3.26 and 3.65 ms; at 640^3 1,000 uniform 4.8 and 3.0 ms, tilts 4.8 and 4.5 ms, and one call with a synchronisation behind it
-// 106 and 3.1 ms, since partial sums of more than the workspaces' bound are allocated anew).
-i32 span_for(i32 most, i32 n_slices, i64 bricks, bool cut_few) {
-    constexpr i64 WAVES = 12 * 256, MANY = 20000;
-    if (bricks > MANY) return 1024;
+// Where the sub-bricks are so many that partial sums of every segment cost uniform poses more than the segments save a tilt
+// series: 1,024 slices, for the slab kernel from about 420^3 on and for the one-wave kernel, whose items are smaller anyway,
+// from about 270^3 on. The default bound and 1,024, uniform poses and tilts: slab kernel at 384^3 from 1,000 slices 1.27 and
+// 1.00 ms, 1.74 and 2.56 ms; at 512^3 from 300 1.18 and 0.87 ms, 1.44 and 1.34 ms, from 1,000 2.68 and 2.00 ms, 3.26 and 3.65
+// ms; at 640^3 from 1,000 4.8 and 3.0 ms, 4.8 and 4.5 ms, and one call with a synchronisation behind it 106 and 3.1 ms, since
+// partial sums of more than the workspaces' bound are allocated anew; one-wave kernel (inverse scalings) at 384^3 from 1,000
+// uniform 2.21 and 2.00 ms.
+i32 span_for(i32 most, i32 n_slices, i64 bricks, bool slab, bool cut_few) {
+    constexpr i64 WAVES = 12 * 256;
+    if (bricks > (slab ? 20000 : 6000)) return 1024;
     if (!cut_few || bricks < 1 || 2 * bricks > WAVES) return most;
     const i32 segments = static_cast<i32>(WAVES / bricks);
     const i32 shortest = std::max(8, static_cast<i32>(0.8 * std::sqrt(static_cast<double>(n_slices))));
     return std::min(most, std::max(shortest, (n_slices + segments - 1) / segments));
 }
-using PlanKey = std::tuple<int, i32, i32, i32, i64, i64, i64, double, bool, i32, double, i32, i32, i32, double, int, i32>;
+using PlanKey = std::tuple<int, i32, i32, i32, i64, i64, i64, double, bool, i32, double, i32, i32, i32, double, int, i32, bool>;
 std::mutex g_plan_mutex;
 std::map<PlanKey, Plan> g_plans;
 
@@ -1344,9 +1347,9 @@ int upload_plan(Plan& pl, std::string& err) {
 // same time read neighbouring slices: their footprints are shared in the L2); 2 = XCD-aware spatial order (below).
 int make_plan(int device, const i32 grid[3], const i64 target[3], double cutoff, bool centered, i32 n_slices,
               double fftfreq_blackman, const i32 bd[3], double list_target, bool upload, const Plan*& plan,
-              std::string& err, int order = 0, i32 max_span = 0) {
+              std::string& err, int order = 0, i32 max_span = 0, bool slab = false) {
     const PlanKey key{device, grid[0], grid[1], grid[2], target[0], target[1], target[2], cutoff, centered, n_slices,
-                      fftfreq_blackman, bd[0], bd[1], bd[2], list_target, order, max_span};
+                      fftfreq_blackman, bd[0], bd[1], bd[2], list_target, order, max_span, slab};
     std::lock_guard<std::mutex> lock(g_plan_mutex);
     auto it = g_plans.find(key);
     if (it != g_plans.end()) {
@@ -1399,7 +1402,8 @@ int make_plan(int device, const i32 grid[3], const i64 target[3], double cutoff,
         for (const Active& a : active) total += a.expected;
         per_item = std::min(-list_target, std::max(16.0, total / PLAN_MIN_ITEMS));
     }
-    if (max_span < 0) max_span = span_for(-max_span, n_slices, static_cast<i64>(active.size()), list_target < 0);
+    if (max_span < 0)
+        max_span = span_for(-max_span, n_slices, static_cast<i64>(active.size()), slab, list_target < 0);
     for (const Active& a : active) {
                 const i32 brick = a.brick;
                 const double expected = a.expected;
@@ -1585,11 +1589,13 @@ KernelChoice kernel_choice(const ProjectDesc& d) {
 }
 
 // Most slices of the range per work item: a sub-brick crossed by many more slices than the uniform model expects (a tilt
-// series) still gets several items. A quarter of the slices, between 256 and 1,024: fewer cost uniform poses partial sums
+// series) still gets several items. A quarter of the slices, between 256 and 1,024, and none up to 384 slices, which it
+// would cut in two (300 slices of 256^2: uniform poses 229 us in two and 205 in one, with NEAREST 303 and 260, a tilt series
+// 518 and 653); fewer cost uniform poses partial sums
 // (1,000 slices of 256^2: 0.62 ms, 0.71 ms with a bound of 128, which takes a tilt series from 2.5 to 1.0 ms); 2,000
 // slices of 200^2, uniform and tilt series, with bounds of 128 0.73 and 0.97 ms, 256 0.60 and 1.09 ms, 512 0.57 and 1.75
 // ms, 1,024 0.60 and 3.05 ms; 10,000 of 256^2 4.60 ms with 1,024, 4.87 with 512.
-i32 default_span(i32 n_slices) { return std::clamp(n_slices / 4, 256, 1024); }
+i32 default_span(i32 n_slices) { return n_slices <= 384 ? 1024 : std::clamp(n_slices / 4, 256, 1024); }
 
 // Window of the slab kernel: windowed_sinc(pz / n, fs, fb) (FourierProject.hpp:99-110) as a polynomial of degree
 // SLAB_NWIN in t = 2 (pz / fbT)^2 - 1, pz in samples (fbT = fb * n): Chebyshev interpolation at the Chebyshev nodes,
@@ -1828,7 +1834,8 @@ int run(const ProjectDesc& d, hipStream_t stream, std::string& err, const Scratc
                                      scratch == nullptr, planp, err, kc.order,
                                      scratch != nullptr || kc.order == 3 ? 0
                                      : kc.max_span >= 0                  ? kc.max_span
-                                                                         : -default_span(plan_slices));
+                                                                         : -default_span(plan_slices),
+                                     slab);
             if (st != NOA_HIP_OK) return st;
             // Pose-adaptive plan (item order 3; not for the allocation-free entry point): the passing slices of each
             // active sub-brick are counted on the device, and the segments are cut from the counts.
