@@ -17,9 +17,9 @@
 // The tiles nearest to the origin are issued first: with tiles in row order the last slices' middle tiles started last
 // and ran with the chip nearly empty (61 -> 61 slices of 256^2: twice the time). And for the common calls (arrays in
 // single precision, LINEAR, no scaling, no Ewald sphere) the taps of one candidate are in flight while the next one's
-// coordinates are computed, a candidate that no pixel of the tile hits costs no load, and the window takes one sine and
-// one cosine instead of a sine and two cosines (84 -> 76 us; 178 us without any of these). Scaled, Ewald, value and FP64
-// inputs and the other interpolations keep the plain loop.
+// coordinates are computed, a candidate that no pixel of the tile hits costs no load, and the window's sine and cosines are
+// short polynomials (84 -> 68 us; 178 us without any of these). Scaled, Ewald, value and FP64 inputs and the other
+// interpolations keep the plain loop.
 //
 // The w-windowed (4D) form keeps the window sum in registers: the outputs start from 0 (or from their value when
 // adding) and the w terms are added in increasing w, the order of noa's serial CPU path; no atomics are needed
@@ -61,25 +61,42 @@ struct InsExtParams {
     // The pipelined path (arrays, single precision, LINEAR, no scaling or Ewald sphere).
     bool pipelined;
     u32 slice_bytes, wslice_bytes;         // byte extent of one slice and of one weight slice (buffer loads)
+    float inv_sinc, inv_blackman;          // 1 / in_sinc, 1 / in_blackman
     float out_inv[2];                      // 1 / out_f
 };
 
-// windowed_sinc (FourierProject.hpp:99-110) of the pipelined path: cos(2b) taken as 2 cos(b)^2 - 1, so that the Blackman
-// window is 0.34 + cos(b) (0.5 + 0.16 cos(b)) in two fused multiply-adds, and one sincos where the two widths are equal (the
-// default). Fewer roundings than noa's expression: largest error 1.8e-7 against 2.0e-7, root mean square 3.1e-8 against
-// 3.6e-8 (default width; wider ones alike), and a cosine less. (A polynomial of degree 12, as the culled insertion's, was
-// 16 us faster for 61 slices of 256^2 than noa's expression, but 2 to 3 times less exact for wide windows.)
-__device__ __forceinline__ float pipelined_window(float fz, float sinc, float blackman) {
-    const float f = fz * 3.141592653589793238462643383279502884f;
-    const float x = f / sinc;
+// windowed_sinc (FourierProject.hpp:99-110) of the pipelined path, |fz| < blackman. cos(2b) is taken as 2 cos(b)^2 - 1, so
+// that the Blackman window is 0.34 + cos(b) (0.5 + 0.16 cos(b)) in two fused multiply-adds. Where the sinc is as wide as the
+// window or wider (the default), sin(x) / x and cos(b) are polynomials in the squares of fz / sinc and fz / blackman, which
+// are at most 1: (sin(pi q) / (pi q) - 1) / q^2 and (cos(pi q) - 1) / q^2 fitted at 200 Chebyshev nodes of q^2 in [0, 1] and
+// rounded; 1 at q = 0 exactly. Fewer roundings than noa's expression: largest error 1.3e-7 to 1.5e-7 against 1.9e-7 to
+// 2.0e-7, root mean square 2.4e-8 to 3.0e-8 against 3.4e-8 to 3.6e-8 (widths of 1/16 to 1/384); a narrower sinc takes the
+// sine and the cosine (1.6e-7 against 1.7e-7). 61 -> 61 slices of 256^2: 84 us with noa's expression, 76 us with a sincos. (The
+// culled insertion's polynomial of the whole window is 2 to 3 times less exact for narrower sincs.)
+__device__ __forceinline__ float pipelined_window(float fz, float sinc, float blackman, float inv_sinc, float inv_blackman) {
     float s, c;
-    if (sinc == blackman) {        // uniform
-        sincosf(x, &s, &c);
+    if (sinc >= blackman) {        // uniform
+        const float qs = fz * inv_sinc, qb = fz * inv_blackman;
+        const float us = qs * qs, ub = qb * qb;
+        s = fmaf(0.0001288788771489635f, us, -0.0023245925549417734f);
+        s = fmaf(s, us, 0.026136834174394608f);
+        s = fmaf(s, us, -0.19074925780296326f);
+        s = fmaf(s, us, 0.8117421865463257f);
+        s = fmaf(s, us, -1.644934058189392f);
+        s = fmaf(s, us, 1.f);
+        c = fmaf(-9.057378338184208e-05f, ub, 0.0019106826512143016f);
+        c = fmaf(c, ub, -0.02579416148364544f);
+        c = fmaf(c, ub, 0.23532620072364807f);
+        c = fmaf(c, ub, -1.3352620601654053f);
+        c = fmaf(c, ub, 4.058712005615234f);
+        c = fmaf(c, ub, -4.934802055358887f);
+        c = fmaf(c, ub, 1.f);
     } else {
-        s = sinf(x);
+        const float f = fz * 3.141592653589793238462643383279502884f, x = f / sinc;
+        s = x == 0.f ? 1.f : sinf(x) / x;
         c = cosf(f / blackman);
     }
-    return (x == 0.f ? 1.f : s / x) * fmaf(c, fmaf(c, 0.16f, 0.5f), 0.34f);
+    return s * fmaf(c, fmaf(c, 0.16f, 0.5f), 0.34f);
 }
 
 // The candidate whose taps are in flight while the next one's coordinates are computed.
@@ -217,7 +234,7 @@ __global__ __launch_bounds__(IE_TILE * IE_TILE * IE_WAVES) void insert_extract_k
                                                         : static_cast<const void*>(p.in), p.wslice_bytes);
                         InsExtTaps<C, In, W> next;
                         next.hit = hit;
-                        next.window = pipelined_window(g.z, p.in_sinc, p.in_blackman);
+                        next.window = pipelined_window(g.z, p.in_sinc, p.in_blackman, p.inv_sinc, p.inv_blackman);
                         next.taps = fetch_taps<INTERP, false, In, W>(sb, p.is_y, p.is_x, wb, p.wis_y, p.wis_x,
                                                                      p.win_present, p.in_h, p.in_w, p.in_centered,
                                                                      g.y * p.in_f[0], g.x * p.in_f[1], hit);
@@ -391,6 +408,8 @@ int run(const InsertExtractDesc& d, hipStream_t stream, std::string& err) {
                       d.out_shape[2] < 4096 && d.out_shape[3] < 4096;
         p.slice_bytes = static_cast<u32>(sb);
         p.wslice_bytes = static_cast<u32>(wb);
+        p.inv_sinc = 1.f / p.in_sinc;
+        p.inv_blackman = 1.f / p.in_blackman;
         for (int i = 0; i < 2; ++i) p.out_inv[i] = 1.f / p.out_f[i];
     }
     p.cull = !(d.ews_radius[0] != 0 || d.ews_radius[1] != 0);

@@ -169,7 +169,7 @@ def test_pipelined_candidates_match_the_oracle(n, n_out, b_in, b_out, weights, c
     close(got_w, want_w)
 
 
-@pytest.mark.parametrize("sinc", [None, (0.03, 0.045), (0.06, 0.13), (0.1, 0.3)])
+@pytest.mark.parametrize("sinc", [None, (0.03, 0.03), (0.05, 0.04), (0.03, 0.045), (0.06, 0.13), (0.1, 0.3)])
 def test_the_pipelined_window_is_as_exact_as_the_plain_loops(sinc):
     """One input slice in the volume's xy plane and no weights: the output weight is the window of fz, here a product of two
     single-precision numbers. Its error against double precision, largest and root mean square, is no larger on the
