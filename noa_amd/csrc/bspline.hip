@@ -407,26 +407,29 @@ namespace {
 
 // Whole-line tiles or, for rows, the chunks of bspline_rows_kernel. A tile costs its lines' index arithmetic (about 0.18 us
 // per 1,000 lines once there are many), a row in chunks about 9 us for each chunk after the first, in which the next one is
-// awaited; wider values make both wait for memory sooner. Chunks and tiles: 12,000 rows of 24 f32 9.0 and 7.5 us, 40,000 of
-// 24 9.5 and 12.6, of 33 18 and 12.5, of 128 40 and 23; 100,000 of 64 22 and 29, of 128 44 and 42, of 200 81 and 60;
-// 300,000 of 96 74 and 90, of 200 273 and 170. c32: 40,000 of 64 22 and 25, of 80 42 and 33; 100,000 of 128 75 and 87, of
-// 200 198 and 165. c64: 40,000 of 32 17 and 29, of 33 41 and 29, 300,000 of 33 254 and 217.
+// awaited; wider values make both wait for memory sooner. Chunks and tiles: 12,000 rows of 24 f32 9.0 and 7.5 us (c64 12.2
+// and 12.3), 40,000 of 24 9.5 and 12.6 (they cross at about 20,000, for 2 samples at 15,000), of 33 18 and 12.5, of 128 40
+// and 23; 100,000 of 64 22 and 29, of 128 44 and 42, of 200 81 and 60; 300,000 of 96 74 and 90, of 200 273 and 170. c32:
+// 40,000 of 64 22 and 25, of 80 42 and 33; 100,000 of 128 75 and 87, of 200 198 and 165. c64: 40,000 of 32 17 and 29, of 33
+// 41 and 29, 300,000 of 33 254 and 217.
 bool tiles_for_rows(i64 lines, i64 n, size_t bytes) {
     const i64 waits = (n + 31) / 32 - 1;           // bspline_rows_kernel's chunks after the first
-    if (lines <= 12288) return true;
+    if (lines <= (bytes == 16 ? 12288 : 16384)) return true;
     if (bytes == 16) return waits >= 1;
     return waits >= 4 || lines <= (bytes == 4 ? 50000 : 25000) * waits;
 }
 
 // Whole-line tiles across the contiguous axis, or a lane per line in memory: the tiles where the GPU (256 CUs, 160 KB of
-// LDS and 2,048 lanes each) holds all of them at once, or half as many again for 4-byte values and half of them for
-// 16-byte ones. Lines in memory and tiles, with the tiles' number over the ones resident: f32 40,000 of 100 (0.8) 24 and 19 us, 16,000 of 800 (1.3) 115 and 92, 54,300 of
-// 300 (1.6) 52 and 54, 40,000 of 500 (2.5) 78 and 95, 24,000 of 2,000 (5.9) 285 and 544, 40,000 of 8 with 2 neighbours
-// (9.8) 6 and 36; c32 10,000 of 400 (0.9) 71 and 39, 40,000 of 100 (1.4) 26 and 29; c64 4,096 of 64 (0.3) 16 and 11, 16,000
-// of 40 (1.0) 13 and 18.
-bool tiles_for_columns(i64 tiles, size_t lds, size_t bytes) {
+// LDS and 2,048 lanes each) holds all of them at once, twice as many for long lines of 4-byte values (a lane's chain along
+// the line then bounds the other form) and half of them for 16-byte ones. Lines in memory and tiles, with the tiles' number
+// over the ones resident: f32 40,000 of 100 (0.8) 24 and 19 us, 63,000 of 37 (1.06) 3 us less than tiles, 16,000 of 800 (1.3)
+// 115 and 92, 54,300 of 300 (1.6) 52 and 54, 16,000 of 1,000 (1.97) 144 and 115, 40,000 of 500 (2.5) 78 and 95, 24,000 of
+// 2,000 (5.9) 285 and 544, 40,000 of 8 with 2 neighbours (9.8) 6 and 36; c32 10,000 of 400 (0.9) 71 and 39, 40,000 of 100
+// (1.4) 26 and 29; c64 4,096 of 64 (0.3) 16 and 11, 16,000 of 40 (1.0) 13 and 18.
+bool tiles_for_columns(i64 tiles, i64 n, size_t lds, size_t bytes) {
     const i64 resident = 256 * std::min<i64>(2048 / TILE_LANES, (160 * 1024) / static_cast<i64>(lds));
-    return bytes == 4 ? 2 * tiles <= 3 * resident : bytes == 8 ? tiles <= resident : 2 * tiles <= resident;
+    if (bytes == 16) return 2 * tiles <= resident;
+    return tiles <= (bytes == 4 && n >= 400 ? 2 : 1) * resident;
 }
 
 // Launch of one pass over `lines` lines of `n` samples; the outer dimensions are (lines / (n1 * n2), n1, n2).
@@ -452,7 +455,7 @@ int pass(bool rows, const T* in, const i64 in_s[3], i64 in_step, T* out, const i
     const i64 tiles_c = (n2 + width - 1) / width;
     const i64 tiles = rows ? (p.lines + width - 1) / width : n0 * n1 * tiles_c;
     if (lds <= TILE_LDS && tiles * TILE_LANES <= MAX_LANES &&
-        (rows ? tiles_for_rows(p.lines, n, sizeof(T)) : tiles_for_columns(tiles, lds, sizeof(T)))) {
+        (rows ? tiles_for_rows(p.lines, n, sizeof(T)) : tiles_for_columns(tiles, n, lds, sizeof(T)))) {
         auto launch = [&](auto w) {
             constexpr i32 W = decltype(w)::value;
             const dim3 grid(static_cast<u32>(tiles)), block(TILE_LANES);
