@@ -11,7 +11,7 @@
 // float reassociation, as with noa's CUDA and OpenMP paths.
 //
 // One cubic size (FP32 values and weights, single-precision rotations, cutoff <= 0.5) takes rasterize_box_kernel
-// instead: the accumulation happens in LDS and reaches the volume once per work item.
+// instead, but for the smallest calls: the accumulation happens in LDS and reaches the volume once per work item.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "workspace.hpp"
