@@ -230,17 +230,29 @@ __device__ __forceinline__ BoxOrigin box_origin(i32 box, i32 nby, i32 nbx, i32 b
     return {base + (zy / nby) * RB_Z, base + (zy % nby) * RB_Y, bx * RB_X};
 }
 
-// Does the plane of `r` (spanned by its 2nd and 3rd columns; any matrix) cross the box widened by M? The plane is
-// symmetric through the origin, so this also decides the mirrored box.
-__device__ __forceinline__ bool box_crossed(const Rot<float>& r, BoxOrigin o, float M) {
-    const float nz = r.m[4] * r.m[8] - r.m[7] * r.m[5];
-    const float ny = r.m[7] * r.m[2] - r.m[1] * r.m[8];
-    const float nx = r.m[1] * r.m[5] - r.m[4] * r.m[2];
+// The normal of the plane spanned by the 2nd and 3rd columns a and c of a matrix, which need not be orthogonal or of unit
+// length: a x c.
+__device__ __forceinline__ vec3<float> plane_normal(const Rot<float>& r) {
+    vec3<float> v;
+    v.z = r.m[4] * r.m[8] - r.m[7] * r.m[5];
+    v.y = r.m[7] * r.m[2] - r.m[1] * r.m[8];
+    v.x = r.m[1] * r.m[5] - r.m[4] * r.m[2];
+    return v;
+}
+
+// Does the plane of `r` with the normal `v` cross the box widened by M? The plane is symmetric through the origin, so this
+// also decides the mirrored box. The rounding of the normal, and of the pixels' positions, moves the distance by up to
+// 3e-7 n times the square of the columns' length and not of the normal's, which is far smaller where they are nearly
+// parallel.
+__device__ __forceinline__ bool box_crossed(const Rot<float>& r, const vec3<float>& v, BoxOrigin o, float n, float M) {
     const float cz = static_cast<float>(o.z) + 0.5f * RB_Z, cy = static_cast<float>(o.y) + 0.5f * RB_Y;
     const float cx = static_cast<float>(o.x) + 0.5f * RB_X;
-    const float d = fabsf((nz * cz + ny * cy) + nx * cx);
-    const float az = fabsf(nz), ay = fabsf(ny), ax = fabsf(nx);
-    return d <= ((0.5f * RB_Z) * az + (0.5f * RB_Y) * ay) + (0.5f * RB_X) * ax + M * ((az + ay) + ax) + 1e-6f;
+    const float d = fabsf((v.z * cz + v.y * cy) + v.x * cx);
+    const float az = fabsf(v.z), ay = fabsf(v.y), ax = fabsf(v.x);
+    const float top = fmaxf(fmaxf(fmaxf(fabsf(r.m[1]), fabsf(r.m[4])), fmaxf(fabsf(r.m[7]), fabsf(r.m[2]))),
+                            fmaxf(fabsf(r.m[5]), fabsf(r.m[8])));
+    return d <= ((0.5f * RB_Z) * az + (0.5f * RB_Y) * ay) + (0.5f * RB_X) * ax + M * ((az + ay) + ax) +
+                    (3e-6f * n) * (top * top);
 }
 
 // The first slice of each item, for more than 64 slices (otherwise, and where nothing can be allocated, the items scan
@@ -259,9 +271,10 @@ __global__ __launch_bounds__(RB_SCAN) void rasterize_items_kernel(const RasterBo
     i32 seen = 0, turn = 0;
     for (i32 c0 = 0; c0 < p.n_slices; c0 += RB_SCAN, turn ^= 1) {
         bool cross = false;
-        if (c0 + t < p.n_slices)
-            cross = box_crossed(plane_matrix(load_rotation(p.rot, c0 + t), slice_scaling(p.scale, p.scaled, c0 + t)), o,
-                                p.margin);
+        if (c0 + t < p.n_slices) {
+            const Rot<float> r = plane_matrix(load_rotation(p.rot, c0 + t), slice_scaling(p.scale, p.scaled, c0 + t));
+            cross = box_crossed(r, plane_normal(r), o, static_cast<float>(p.n), p.margin);
+        }
         const unsigned long long m = __ballot(cross);
         if ((t & 63) == 0) passed[turn][wave] = static_cast<i32>(__popcll(m));
         __syncthreads();                 // one barrier per turn: the next one writes the other half
@@ -302,7 +315,7 @@ __global__ __launch_bounds__(64) void rasterize_box_kernel(const RasterBoxParams
     const i32 lo = -n / 2, hi = (n - 1) / 2, hix = n / 2;
     const float P0[3] = {static_cast<float>(Z0), static_cast<float>(Y0), static_cast<float>(X0)};
     constexpr float EXT[3] = {RB_Z, RB_Y, RB_X};
-    const float M = p.margin;
+    const float nf = static_cast<float>(n), M = p.margin;
     // The item's first slice: its slices are the next `left` ones that cross the box.
     i32 first = 0, left = p.per_item;
     if (p.starts) {
@@ -313,9 +326,11 @@ __global__ __launch_bounds__(64) void rasterize_box_kernel(const RasterBoxParams
         unsigned long long m = 0;
         for (; first < p.n_slices; first += 64) {
             bool cross = false;
-            if (first + lane < p.n_slices)
-                cross = box_crossed(plane_matrix(load_rotation(p.rot, first + lane),
-                                                 slice_scaling(p.scale, GEN && p.scaled, first + lane)), at0, M);
+            if (first + lane < p.n_slices) {
+                const Rot<float> r = plane_matrix(load_rotation(p.rot, first + lane),
+                                                  slice_scaling(p.scale, GEN && p.scaled, first + lane));
+                cross = box_crossed(r, plane_normal(r), at0, nf, M);
+            }
             m = __ballot(cross);
             const i32 cnt = static_cast<i32>(__popcll(m));
             if (skip < cnt) break;
@@ -331,7 +346,6 @@ __global__ __launch_bounds__(64) void rasterize_box_kernel(const RasterBoxParams
     }
     lds_order();
 
-    const float nf = static_cast<float>(n);
     // The box of this lane's set, widened by the margin: direct positions in [P0, P0 + EXT), mirrored ones in
     // (-P0 - EXT, -P0].
     const bool mirrored_rows = lane >= 32;
@@ -461,14 +475,19 @@ __global__ __launch_bounds__(64) void rasterize_box_kernel(const RasterBoxParams
         bool cross = false, flat = false;
         if (c0 + lane < p.n_slices) {
             const Rot<float> r = plane_matrix(load_rotation(p.rot, c0 + lane), slice_scaling(p.scale, GEN && p.scaled, c0 + lane));
-            cross = box_crossed(r, at0, M);
+            const vec3<float> v = plane_normal(r);
+            cross = box_crossed(r, v, at0, nf, M);
             a[0] = r.m[1]; a[1] = r.m[4]; a[2] = r.m[7];
             c[0] = r.m[2]; c[1] = r.m[5]; c[2] = r.m[8];
             const float aa = (a[0] * a[0] + a[1] * a[1]) + a[2] * a[2];
             const float ac = (a[0] * c[0] + a[1] * c[1]) + a[2] * c[2];
             const float cc = (c[0] * c[0] + c[1] * c[1]) + c[2] * c[2];
-            const float det = aa * cc - ac * ac;
-            flat = !(det > 1e-6f * aa * cc);
+            // The determinant, far more exact than aa cc - ac^2 where the columns are nearly parallel. All pixels are
+            // tried where the columns are parallel to 1e-3, and where they are long enough for the products that cancel
+            // inside the volume to round by as much as the margin of 1e-5 n: up to 1e-7 n per unit of length and, below
+            // that, n / 1e7 over the sine of the columns' angle, hence a length of 10 and a sine of 0.03.
+            const float det = dot3(v);
+            flat = !(det > 1e-6f * aa * cc) || (det < 1e-3f * aa * cc && fmaxf(aa, cc) > 100.f);
             const float idet = 1.f / det;
 #pragma unroll
             for (int i = 0; i < 3; ++i) {

@@ -350,3 +350,28 @@ def test_first_call_of_a_size_can_be_captured(b, monkeypatch):
         graph.replay()
         torch.cuda.synchronize()
         assert rel_l2(vol.cpu().numpy(), want_v) < 1e-6 and rel_l2(wv.cpu().numpy(), want_w) < 1e-6
+
+
+@pytest.mark.parametrize("n,length,ratio", [(512, 100.0, 1e3), (512, 100.0, 1.5e3), (700, 20.0, 1.5e3), (512, 9.0, 900.0),
+                                            (512, 1.0, 900.0), (512, 0.5, 5e3)])
+def test_boxes_find_the_pixels_of_sheared_scalings(monkeypatch, n, length, ratio):
+    """Inverse scalings that make a slice's axes nearly parallel and long: the plane's normal and the coordinates round in
+    proportion, and no pixel may fall between the boxes. Against the lane-per-pixel kernel; the voxels around the origin
+    sum some 10,000 terms in another order, which 1e-5 rel-L2 holds (2^-24 times the square root of their number)."""
+    print(f"case rasterize sheared scalings n={n} {length} {ratio}", flush=True)
+    rng = np.random.default_rng(int(ratio))
+    b = 20
+    turn = lambda t: np.stack([np.stack([np.cos(t), -np.sin(t)], -1), np.stack([np.sin(t), np.cos(t)], -1)], -2)
+    scale = turn(rng.uniform(0, np.pi, b)) @ np.diag([length, length / ratio]) @ turn(rng.uniform(0, np.pi, b))
+    scale = dev(scale.astype(np.float32))
+    sl, rot = dev(random_spectrum((b, 1, n, n // 2 + 1), rng)), nx().Mat33Array(dev(random_rotations(b, rng)), DEV)
+    got = {}
+    for layout in ("direct", "tiles"):
+        monkeypatch.setenv("NOA_HIP_RASTERIZE_LAYOUT", layout)
+        vol = torch.zeros((1, n, n, n // 2 + 1), dtype=torch.complex64, device=DEV)
+        wv = torch.zeros((1, n, n, n // 2 + 1), dtype=torch.float32, device=DEV)
+        nx().rasterize_central_slices_3d("h2h", sl, None, (b, 1, n, n), vol, wv, (1, n, n, n), scale, rot)
+        torch.cuda.synchronize()
+        got[layout] = vol, wv
+    for a, want in zip(got["tiles"], got["direct"]):
+        assert float(torch.linalg.vector_norm(a - want) / torch.linalg.vector_norm(want)) < 1e-5
