@@ -243,7 +243,7 @@ __device__ __forceinline__ vec3<float> plane_normal(const Rot<float>& r) {
 // Does the plane of `r` with the normal `v` cross the box widened by M? The plane is symmetric through the origin, so this
 // also decides the mirrored box. The rounding of the normal, and of the pixels' positions, moves the distance by up to
 // 3e-7 n times the square of the columns' length and not of the normal's, which is far smaller where they are nearly
-// parallel.
+// parallel. A matrix that is not finite crosses every box.
 __device__ __forceinline__ bool box_crossed(const Rot<float>& r, const vec3<float>& v, BoxOrigin o, float n, float M) {
     const float cz = static_cast<float>(o.z) + 0.5f * RB_Z, cy = static_cast<float>(o.y) + 0.5f * RB_Y;
     const float cx = static_cast<float>(o.x) + 0.5f * RB_X;
@@ -251,8 +251,8 @@ __device__ __forceinline__ bool box_crossed(const Rot<float>& r, const vec3<floa
     const float az = fabsf(v.z), ay = fabsf(v.y), ax = fabsf(v.x);
     const float top = fmaxf(fmaxf(fmaxf(fabsf(r.m[1]), fabsf(r.m[4])), fmaxf(fabsf(r.m[7]), fabsf(r.m[2]))),
                             fmaxf(fabsf(r.m[5]), fabsf(r.m[8])));
-    return d <= ((0.5f * RB_Z) * az + (0.5f * RB_Y) * ay) + (0.5f * RB_X) * ax + M * ((az + ay) + ax) +
-                    (3e-6f * n) * (top * top);
+    return !(d > ((0.5f * RB_Z) * az + (0.5f * RB_Y) * ay) + (0.5f * RB_X) * ax + M * ((az + ay) + ax) +
+                     (3e-6f * n) * (top * top));
 }
 
 // The first slice of each item, for more than 64 slices (otherwise, and where nothing can be allocated, the items scan

@@ -375,3 +375,26 @@ def test_boxes_find_the_pixels_of_sheared_scalings(monkeypatch, n, length, ratio
         got[layout] = vol, wv
     for a, want in zip(got["tiles"], got["direct"]):
         assert float(torch.linalg.vector_norm(a - want) / torch.linalg.vector_norm(want)) < 1e-5
+
+
+def test_boxes_keep_what_is_not_a_number(monkeypatch):
+    """A matrix of no numbers gives voxels that are not numbers, the same ones with both kernels, and no others."""
+    print("case rasterize non-finite matrix", flush=True)
+    n, b = 64, 20
+    rng = np.random.default_rng(3)
+    sl, m = dev(random_spectrum((b, 1, n, n // 2 + 1), rng)), random_rotations(b, rng)
+    m[7] = np.nan
+    rot, got = nx().Mat33Array(dev(m), DEV), {}
+    for layout in ("direct", "tiles"):
+        monkeypatch.setenv("NOA_HIP_RASTERIZE_LAYOUT", layout)
+        vol = torch.zeros((1, n, n, n // 2 + 1), dtype=torch.complex64, device=DEV)
+        wv = torch.zeros((1, n, n, n // 2 + 1), dtype=torch.float32, device=DEV)
+        nx().rasterize_central_slices_3d("h2h", sl, None, (b, 1, n, n), vol, wv, (1, n, n, n), None, rot)
+        torch.cuda.synchronize()
+        got[layout] = vol, wv
+    assert bool(torch.isnan(got["direct"][1]).any())
+    for a, want in zip(got["tiles"], got["direct"]):
+        a, want = (torch.view_as_real(t) if t.is_complex() else t for t in (a, want))
+        assert torch.equal(torch.isnan(a), torch.isnan(want))
+        a, want = torch.nan_to_num(a), torch.nan_to_num(want)
+        assert float(torch.linalg.vector_norm(a - want) / torch.linalg.vector_norm(want)) < 1e-6
